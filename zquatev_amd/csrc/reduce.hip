@@ -40,7 +40,7 @@ __host__ __device__ constexpr int matvec_spg(int m, int tsm) { return m <= tsm ?
 // matvec tiles of a trailing size with G row groups: group g holds spg (g + 1) strips
 __host__ __device__ constexpr int ntiles(int G, int spg) { return spg * G * (G + 1) / 2; }
 constexpr int NBMAX = 128;   // largest supported panel width
-constexpr int TAILN = 64;    // trailing size from which one workgroup finishes in LDS (k_tail)
+constexpr int TAILN = 64;    // trailing size from which one workgroup finishes (k_tail)
 
 // ceil(a / b) for b > 0, and 0 for a <= 0
 __device__ __forceinline__ int cdiv_d(int a, int b) { return a > 0 ? (a + b - 1) / b : 0; }
@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
   // and stores nothing -- so the body is one scheduling region: the
   // wave-uniform loads of x at the tile's columns issue alongside the tile
   // loads instead of after their wait, and the kernel needs 64 VGPRs instead
-  // of 84 (four 512-thread blocks per CU instead of two).  2n = 8192 solve
+  // of 84 (three 512-thread blocks per CU instead of two).  2n = 8192 solve
   // -1.5 ms.  The narrow tiles keep the branches: branch-free they made the
   // 512-problem batch 1.3% slower (also when held to five blocks per CU, their
   // residency with branches), for 0.7% on single solves of 2n <= 1024.
@@ -553,20 +553,34 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
 }
 
 // ---------------------------------------------------------------------------
-// LDS-resident tail.  Once the trailing matrix has at most TAILN rows, one
-// workgroup per problem finishes the reduction with the whole Hermitian
-// trailing block in LDS (TAILN x TAILN quaternions, 128 KB, both triangles so
-// that every access is a row-contiguous, conflict-free read): per column the
-// reflector, y = A u, K = u^* y / 2, w = y - K u and the rank-2 update
-// A -= u w^* + w u^* at once (unblocked: no panel, no W), separated by
-// barriers instead of kernel launches.  Lane = row, the 4 waves split the
-// columns.  It starts at a panel boundary p, after the trailing update of the
+// Register-resident tail.  Once the trailing matrix has at most TAILN rows,
+// one workgroup per problem finishes the reduction: per column the reflector,
+// y = A u, K = u^* y / 2, w = y - K u and the rank-2 update A -= u w^* + w u^*
+// at once (unblocked: no panel, no W), separated by barriers instead of kernel
+// launches.  It starts at a panel boundary p, after the trailing update of the
 // panel before it, and writes d and e of columns p .. n-2, d[n-1], and the
 // reflectors u into M below the subdiagonal (the blocked columns'
 // conventions).
+//
+// The whole Hermitian block (both triangles) is held in registers: lane = row,
+// and wave v owns columns v, v + 16, v + 32, v + 48 (cyclic, so that the waves
+// stay evenly loaded as columns retire).  The matrix is never re-read: per
+// column only u, w (broadcast reads) and the waves' partials of y pass
+// through LDS, with three barriers.  Wave cl % 16 owns column cl, so after the
+// update of column cl - 1 it forms the next reflector from its own registers
+// while the other waves are still updating.  Retired and absent rows and
+// columns have u = w = 0, so no lane masks are needed.  A version with the
+// block in LDS and four waves was bound by its re-reads of the block, one wave
+// per SIMD having nothing to hide them behind: 64 columns took 242 us, now
+// 150 us (a 2n = 128 solve 679 -> 580 us, 2n = 1024 5.94 -> 5.82 ms).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_tail(quat* __restrict__ M, int ld, int n, int p, const int* __restrict__ pstart,
-                                              double* __restrict__ d, quat* __restrict__ e, ZB zb) {
+constexpr int TT = 1024;            // threads: 16 waves
+constexpr int TWV = TT / 64;
+constexpr int TKC = TAILN / TWV;    // columns per wave
+static_assert(TAILN == 64 && TKC * TWV == TAILN, "k_tail: lane = row, TKC columns per wave");
+
+__global__ void __launch_bounds__(TT) k_tail(quat* __restrict__ M, int ld, int n, int p, const int* __restrict__ pstart,
+                                             double* __restrict__ d, quat* __restrict__ e, ZB zb) {
   if (zb.nvec) {
     n = zb.nvec[blockIdx.z];
     p = pstart[blockIdx.z];
@@ -574,84 +588,79 @@ __global__ void __launch_bounds__(256) k_tail(quat* __restrict__ M, int ld, int 
   }
   const int ms = n - p;
   if (ms < 1 || ms > TAILN) return;   // uniform: a problem without a tail
-  __shared__ quat A[TAILN * TAILN];     // A[j * TAILN + i] = element (i, j)
-  __shared__ quat us[TAILN], ys[TAILN];
-  __shared__ quat part[RB / 64][TAILN];
-  const int tid = threadIdx.x;
-  const int tx = tid & 63, ty = tid >> 6;   // row, column group
-  for (int j = ty; j < ms; j += RB / 64) {
-    if (tx < ms) {
-      quat a = tx >= j ? qload(M + (p + tx) + (size_t)(p + j) * ld) : qconj(qload(M + (p + j) + (size_t)(p + tx) * ld));
-      if (tx == j) a = quat{a.ar, 0.0, 0.0, 0.0};
-      A[j * TAILN + tx] = a;
+  __shared__ quat us[2][TAILN], ys[2][TAILN];   // u and w, by column parity
+  __shared__ quat part[TWV][TAILN];             // the waves' partials of A u
+  const int tx = threadIdx.x & 63;              // row
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  quat a[TKC];   // elements (tx, wv + TWV k)
+#pragma unroll
+  for (int k = 0; k < TKC; ++k) {
+    const int j = wv + TWV * k;
+    a[k] = qzero();
+    if (tx < ms && j < ms) {
+      a[k] = tx >= j ? qload(M + (p + tx) + (size_t)(p + j) * ld) : qconj(qload(M + (p + j) + (size_t)(p + tx) * ld));
+      if (tx == j) a[k] = quat{a[k].ar, 0.0, 0.0, 0.0};
     }
   }
-  __syncthreads();
-  // Every row of the block lives in wave 0 (lane = row), so the two sums over
-  // rows per column (the tail norm, u^* y) are wave sums there, and the tail
-  // norm of the next column is formed by wave 0 right after it updates that
-  // column: four barriers per column.
-  __shared__ double tnorm;
-  if (ty == 0) {
-    const double v = (tx > 1 && tx < ms) ? qnorm2(A[tx]) : 0.0;
-    const double t = wave_sum_d(v);
-    if (tx == 0) tnorm = t;
-  }
-  __syncthreads();
-  for (int cl = 0; cl + 1 < ms; ++cl) {
-    const int r0 = cl + 1;                  // first row of the trailing block
-    const bool row = tx >= r0 && tx < ms;   // this lane's row is in the trailing block
-    const double tail = tnorm;
+  // the reflector of column cl from its owner's registers (column x)
+  auto reflect = [&](int cl, const quat& x) {
+    const int r0 = cl + 1;
+    const bool row = tx >= r0 && tx < ms;
+    const double tail = wave_sum_d(tx > r0 && tx < ms ? qnorm2(x) : 0.0);
+    const quat x1 = quat{lane_d(x.ar, r0), lane_d(x.ai, r0), lane_d(x.br, r0), lane_d(x.bi, r0)};
     quat alpha;
-    const Refl R = reflector(A[cl * TAILN + r0], tail, &alpha);
-    if (tid == 0) {
-      d[p + cl] = A[cl * TAILN + cl].ar;
+    const Refl R = reflector(x1, tail, &alpha);
+    if (tx == cl) {
+      d[p + cl] = x.ar;
       qstore(e + p + cl, alpha);
     }
-    if (ty == 0 && row) {
-      const quat ui = tx == r0 ? R.u1 : qscale(A[cl * TAILN + tx], R.g);
-      us[tx] = ui;
-      qstore(M + (p + tx) + (size_t)(p + cl) * ld, ui);
-    }
-    __syncthreads();
-    quat acc = qzero();   // this lane's row of A22 u over this wave's columns
-    if (row)
-      for (int jj = r0 + ty; jj < ms; jj += RB / 64) qfma(acc, A[jj * TAILN + tx], us[jj]);
-    part[ty][tx] = acc;
-    __syncthreads();
-    if (ty == 0) {
-      quat y = qzero();
-      double kv = 0.0;
-      if (row) {
-        y = part[0][tx];
+    const quat ui = row ? (tx == r0 ? R.u1 : qscale(x, R.g)) : qzero();
+    us[cl & 1][tx] = ui;
+    if (row) qstore(M + (p + tx) + (size_t)(p + cl) * ld, ui);
+  };
+  if (wv == 0 && ms > 1) reflect(0, a[0]);
 #pragma unroll
-        for (int k = 1; k < RB / 64; ++k) y = qadd(y, part[k][tx]);
-        const quat u = us[tx];
-        kv = u.ar * y.ar + u.ai * y.ai + u.br * y.br + u.bi * y.bi;   // Re(conj(u_i) y_i)
+  for (int kk = 0; kk < TKC; ++kk) {
+    for (int c = 0; c < TWV; ++c) {
+      const int cl = TWV * kk + c;
+      if (cl + 1 >= ms) break;   // uniform
+      const int r0 = cl + 1, par = cl & 1;
+      __syncthreads();   // us of column cl is complete
+      const quat ui = us[par][tx];
+      quat acc = qzero();   // this lane's row of A u over this wave's columns
+#pragma unroll
+      for (int k = kk; k < TKC; ++k)
+        if (wv + TWV * k >= r0) qfma(acc, a[k], us[par][wv + TWV * k]);   // uniform
+      part[wv][tx] = acc;
+      __syncthreads();
+      if (wv == 0) {
+        quat y = part[0][tx];
+#pragma unroll
+        for (int k = 1; k < TWV; ++k) y = qadd(y, part[k][tx]);
+        // K = u^* y / 2; u = 0 outside the trailing rows
+        const double K = 0.5 * wave_sum_d(ui.ar * y.ar + ui.ai * y.ai + ui.br * y.br + ui.bi * y.bi);
+        ys[par][tx] = (tx >= r0 && tx < ms) ? qsub(y, qscale(ui, K)) : qzero();   // w
       }
-      const double K = 0.5 * wave_sum_d(kv);
-      if (row) ys[tx] = qsub(y, qscale(us[tx], K));   // w
-    }
-    __syncthreads();
-    if (row) {
-      const quat ui = us[tx], wi = ys[tx];
-      for (int jj = r0 + ty; jj < ms; jj += RB / 64) {
-        quat a = A[jj * TAILN + tx];
-        a = qsub(a, qmul(ui, qconj(ys[jj])));
-        a = qsub(a, qmul(wi, qconj(us[jj])));
-        if (jj == tx) a = quat{a.ar, 0.0, 0.0, 0.0};   // Hermitian diagonal: real
-        A[jj * TAILN + tx] = a;
+      __syncthreads();
+      const quat wi = ys[par][tx];
+      // the rank-2 update; the wave owning the next column forms its
+      // reflector right after updating that column, before its others
+#pragma unroll
+      for (int k = kk; k < TKC; ++k) {
+        const int j = wv + TWV * k;
+        if (j < r0) continue;   // uniform
+        const quat uj = us[par][j], wj = ys[par][j];
+        const quat nu = quat{-ui.ar, -ui.ai, -ui.br, -ui.bi}, nw = quat{-wi.ar, -wi.ai, -wi.br, -wi.bi};
+        qfma_cr(a[k], nu, wj);
+        qfma_cr(a[k], nw, uj);
+        if (tx == j) a[k] = quat{a[k].ar, 0.0, 0.0, 0.0};   // Hermitian diagonal: real
+        if (j == r0 && r0 + 1 < ms) reflect(r0, a[k]);
       }
     }
-    // tail norm of the next column, r0, whose rows this wave (jj = r0) just updated
-    if (ty == 0) {
-      const double v = (tx > r0 + 1 && tx < ms) ? qnorm2(A[r0 * TAILN + tx]) : 0.0;
-      const double t = wave_sum_d(v);
-      if (tx == 0) tnorm = t;
-    }
-    __syncthreads();
   }
-  if (tid == 0) d[n - 1] = A[(ms - 1) * TAILN + (ms - 1)].ar;
+#pragma unroll
+  for (int k = 0; k < TKC; ++k)
+    if (wv + TWV * k == ms - 1 && tx == ms - 1) d[n - 1] = a[k].ar;
 }
 
 int tail_start(int n, int nb) {
@@ -750,7 +759,7 @@ int reduce(quat* M, int n, int ld, int nb, double* d, quat* e, const ReduceWork&
       if (rc) return rc;
     }
   }
-  if (ts < n) hipLaunchKernelGGL(k_tail, dim3(1), dim3(RB), 0, s, M, ld, n, ts, nullptr, d, e, ZB{nullptr, 0});
+  if (ts < n) hipLaunchKernelGGL(k_tail, dim3(1), dim3(TT), 0, s, M, ld, n, ts, nullptr, d, e, ZB{nullptr, 0});
   else hipLaunchKernelGGL(k_last_diag, dim3(1), dim3(64), 0, s, M, ld, n, d, ZB{nullptr, 0});
   return hipGetLastError() == hipSuccess ? ZQI_OK : ZQI_ERR_HIP;
 }
@@ -856,7 +865,7 @@ int reduce_batched(int nprob, const int* nh, ZB zb, quat* M, int ld, int nb, dou
   }
   // problems without a tail take d[n-1] here; the tails overwrite theirs
   hipLaunchKernelGGL(k_last_diag, dim3(1, 1, nprob), dim3(64), 0, s, M, ld, L, d, zb);
-  hipLaunchKernelGGL(k_tail, dim3(1, 1, nprob), dim3(RB), 0, s, M, ld, L, 0, tstart, d, e, zb);
+  hipLaunchKernelGGL(k_tail, dim3(1, 1, nprob), dim3(TT), 0, s, M, ld, L, 0, tstart, d, e, zb);
   return hipGetLastError() == hipSuccess ? ZQI_OK : ZQI_ERR_HIP;
 }
 
