@@ -60,12 +60,13 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
 // Reflector for column c: x = M[c+1:, c].  H x = alpha e_1 with
 // alpha = -q |x|, q = x_1/|x_1|; u = gamma (x - alpha e_1), gamma = 1/sqrt(|x| (|x| + |x_1|)),
 // so u^* u = 2.  A zero tail gives u = 0 and alpha = x_1.  Computed identically
-// by every block of the matvec from the tail-norm partials.
+// by every block that needs it.
 struct Refl {
   double g;
   quat u1;
 };
 __device__ __forceinline__ Refl reflector(const quat& x1, double tail, quat* alpha) {
+#pragma clang fp contract(off)
   const double ax1 = sqrt(qnorm2(x1));
   Refl R;
   if (!(tail > 0.0)) {
@@ -123,7 +124,7 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
   const int NF = NT > 0 ? NT : 1;
   if (zb.nvec) {
     n = zb.nvec[blockIdx.z];
-    nparts = (n - c + RQ - 1) / RQ;
+    nparts = (n - c - 1 + RQ - 1) / RQ;
     const int Gz = (n - c - 1 + SG - 1) / SG;
     if ((int)blockIdx.x >= ntiles(Gz, SPG) + NF) return;
     M = zoff(M, zb); W = zoff(W, zb); part = zoff(part, zb); scal = zoff(scal, zb); d = zoff(d, zb);
@@ -155,7 +156,7 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
     double mss = 0.0, mcc = 0.0;
     if (bt == 0 && tid == 0) {
       mss = M[s0 + (size_t)s0 * ld].ar;
-      mcc = M[c + (size_t)c * ld].ar;
+      if (j == 0) mcc = M[c + (size_t)c * ld].ar;
     }
     double tsacc = 0.0;
     if (has_ts) {
@@ -186,9 +187,8 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
       scal[0] = R.g;
       scal[1] = R.u1.ar; scal[2] = R.u1.ai; scal[3] = R.u1.br; scal[4] = R.u1.bi;
       scal[5] = x1.ar; scal[6] = x1.ai; scal[7] = x1.br; scal[8] = x1.bi;
-      // the trailing diagonal M[s0, s0] before k_wcol's update of column s0 overwrites it
-      scal[9] = mss;
-      d[c] = mcc;
+      scal[9] = mss;   // M[s0, s0]
+      if (j == 0) d[c] = mcc;   // inside a panel the column kernel has left d[c]
       qstore(e + c, alpha);
     }
     if (has_ts) {
@@ -261,7 +261,7 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
       if constexpr (BF) {
         a = quat{in ? qa[cc].ar : 0.0, (in && !dg) ? qa[cc].ai : 0.0, (in && !dg) ? qa[cc].br : 0.0,
                  (in && !dg) ? qa[cc].bi : 0.0};
-        qfl -= dg ? a.ar * nua : 0.0;
+        qfl = dg ? fma(-a.ar, nua, qfl) : qfl;
         qfma(acc, a, xc[cc]);   // a = 0 where cg >= n
         qfma_cl(cp, a, ua);
         const bool below = ra > cg;
@@ -270,7 +270,7 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
         a = (cg < n && ra < n && ra >= cg) ? qa[cc] : qzero();
         if (ra == cg) {
           a = quat{a.ar, 0.0, 0.0, 0.0};
-          qfl -= a.ar * qnorm2(ua);
+          qfl = fma(-a.ar, qnorm2(ua), qfl);
         }
         qfma(acc, a, cg < n ? xc[cc] : qzero());
         if (ra > cg) qfma_cl(cp, a, ua);
@@ -282,7 +282,7 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
     red[w][2][lane] = acc.br;
     red[w][3][lane] = acc.bi;
     // x^* M x over the tile's lower part, doubled off the diagonal: 2 Re(conj(x_i) acc_i)
-    qfl += 2.0 * (ua.ar * acc.ar + ua.ai * acc.ai + ua.br * acc.br + ua.bi * acc.bi);
+    qfl = fma(2.0, qdot(ua, acc), qfl);
     // lane l ends with value vi = l / LPV (component vi & 3 of column vi >> 2), summed over the wave
     constexpr int LPV = 64 / (4 * SCW);
     const double cs = butterfly_sum<4 * SCW>(col);
@@ -312,21 +312,174 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
   }
 }
 
-// Column c's w_j and, inside a panel, column c+1's pending update, in one
-// pass over rows s0 = c+1 .. n-1 (16 threads per row, KPT panel columns each).
-//   p   = y - V (W^* u) - W (V^* u),  y = M u = gamma (M x) + M[:, s0] (u1 - gamma x1)
+// The arithmetic that finishes a column (k_wcol).  Every rounding is written
+// out (explicit FMAs, no contraction of the rest), so that the variants of the
+// kernel -- a solve and the batch it is a member of may run different ones --
+// give the same bits.
+//
+// With x the raw column c, u = gamma x + delta e_1 (delta = u1 - gamma x1, row
+// s0 = c + 1) and the panel's earlier columns V, W:
+//   p   = y - V (W^* u) - W (V^* u),  y = M u = gamma (M x) + M[:, s0] delta
 //         with (M x) from the matvec partials;
-//   K   = u^* p / 2 = (u^* y - 2 Re(a^* b)) / 2,  a = W^* u, b = V^* u (TS), and
+//   K   = u^* p / 2 = (u^* y - 2 Re(a^* b)) / 2,  a = W^* u, b = V^* u, and
 //         u^* y = gamma^2 x^* M x + 2 gamma Re(conj(delta) (M x)_{s0}) + M_{s0 s0} |delta|^2,
-//         delta = u1 - gamma x1, x^* M x from the matvec's per-tile partials (QF) --
-//         so every block has K without a grid-wide reduction of p;
-//   w_j = p - K u (final), stored in W[:, j]; u stored into M[s0:, c].
-// Unless column c closes its panel (j = nb - 1) or the reduction (c = n - 2),
-// the block then applies column c+1's pending update: subtract the
-// [V W] [W V]^*-terms of the panel's columns 0..j (row c+1's coefficients,
-// including the new w_j(c+1) = p(s0) - K u1, are formed redundantly in every
-// block), store the column, and leave its tail-norm partials in part and the
-// per-16-row partials of W^* x, V^* x in TSP.
+//         x^* M x from the matvec's per-tile partials (QF) -- so every block
+//         has K without a grid-wide reduction of p;
+//   w_j = p - K u.
+// Inside a panel, column c+1's pending update follows: subtract the
+// [V W] [W V]^*-terms of the panel's columns 0..j, whose row-s0 coefficients
+// (including the new w_j(s0) = p(s0) - K u1) every block forms redundantly.
+// Row s0 itself is formed from these sums: u1, w_j(s0), and the diagonal
+// entry d[c+1] of the updated column; the other rows start at s0 + 1, so that
+// the 16-row groups of the tall-skinny partials are the rows of the next
+// matvec's tiles.
+//
+// NCS block sums per column: 0 x^* M x, 1 Re(a^* b), 2-5 (M x)_{s0},
+// 6-9 V(s0,:) a + W(s0,:) b, 10 Re(V(s0,:) conj(W(s0,:))).
+constexpr int NCS = 11;
+struct ColScalars {
+  double gam, K;
+  quat u1, delta, wc1;   // wc1 = w_j(s0)
+  double dnext;          // the updated diagonal entry at s0
+};
+__device__ __forceinline__ ColScalars col_scalars(const double* S, double gam, const quat& u1, const quat& x1,
+                                                  double m00) {
+#pragma clang fp contract(off)
+  ColScalars C;
+  C.gam = gam;
+  C.u1 = u1;
+  C.delta = qaxpy(u1, -gam, x1);
+  const quat wrow = quat{S[2], S[3], S[4], S[5]};   // (M x)_{s0}
+  const double uy = fma(gam * gam, S[0], fma(2.0 * gam, qdot(C.delta, wrow), m00 * qnorm2(C.delta)));
+  C.K = 0.5 * fma(-2.0, S[1], uy);
+  const quat ps0 = qsub(qaxpy(qscale(wrow, gam), m00, C.delta), quat{S[6], S[7], S[8], S[9]});
+  C.wc1 = qaxpy(ps0, -C.K, u1);
+  C.dnext = fma(-2.0, qdot(u1, C.wc1), fma(-2.0, S[10], m00));
+  return C;
+}
+// This thread's terms of the block sums (thread l < j holds panel column l's
+// coefficients), summed over the wave: lane t < 16 of sh holds sum t.
+__device__ __forceinline__ void col_wave_sums(double qf, const quat& w0, const quat& al, const quat& bl,
+                                              const quat& cvl, const quat& cwl, double* sh) {
+#pragma clang fp contract(off)
+  quat rd = qzero();
+  qfma(rd, cvl, al);
+  qfma(rd, cwl, bl);
+  double v[16] = {qf, qdot(al, bl), w0.ar, w0.ai, w0.br, w0.bi, rd.ar, rd.ai, rd.br, rd.bi, qdot(cvl, cwl),
+                  0.0, 0.0, 0.0, 0.0, 0.0};
+  const double t = butterfly_sum<16>(v);
+  const int lane = threadIdx.x & 63;
+  if ((lane & 3) == 0) sh[lane >> 2] = t;
+}
+// One thread's share of a row, over the panel columns l = q + 16 k (its
+// coefficients vv, ww): ps = gamma y - (V a + W b), us = V conj(W(s0)) + W
+// conj(V(s0)); then summed over the wave's four q: lane 16 q' + r is left
+// with components 2 q', 2 q' + 1 of row r's (ps, us), stored in red[r].
+template <int KPT>
+__device__ __forceinline__ void row_share(const quat* vv, const quat* ww, const quat& yi, double gam, int q, int j,
+                                          const quat* a, const quat* b, const quat* cw, const quat* cv,
+                                          double (*red)[8]) {
+#pragma clang fp contract(off)
+  quat accp = qscale(yi, gam), accu = qzero();
+  // the coefficients beyond j are zero in LDS (and vv, ww finite), so no lane
+  // masks are needed; a panel's first column has no terms
+  if (j > 0)
+#pragma unroll
+    for (int k = 0; k < KPT; ++k) {
+      const int l = q + 16 * k;
+      const quat ak = a[l], bk = b[l], cwk = cw[l], cvk = cv[l];
+      qfma(accp, qneg(vv[k]), ak);
+      qfma(accp, qneg(ww[k]), bk);
+      qfma(accu, vv[k], cwk);
+      qfma(accu, ww[k], cvk);
+    }
+  double v[8] = {accp.ar, accp.ai, accp.br, accp.bi, accu.ar, accu.ai, accu.br, accu.bi};
+  const int lane = threadIdx.x & 63;
+  bstep<32, 4>(v, lane);
+  bstep<16, 2>(v, lane);
+  *reinterpret_cast<double2*>(&red[lane & 15][2 * (lane >> 4)]) = make_double2(v[0], v[1]);
+}
+// The row's results from the four waves' partials (red: wave, row, component):
+// u, w_j and the updated entry of column c+1 (xi: x, ms: stale column s0).
+struct RowOut {
+  quat u, w, x;
+};
+__device__ __forceinline__ RowOut row_finish(const double (*red)[RQ][8], int r, const ColScalars& C, const quat& xi,
+                                             const quat& ms) {
+#pragma clang fp contract(off)
+  double t[8];
+#pragma unroll
+  for (int h = 0; h < 8; h += 2) {
+    double2 s = *reinterpret_cast<const double2*>(&red[0][r][h]);
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+      const double2 z = *reinterpret_cast<const double2*>(&red[k][r][h]);
+      s.x += z.x;
+      s.y += z.y;
+    }
+    t[h] = s.x;
+    t[h + 1] = s.y;
+  }
+  RowOut o;
+  quat p = quat{t[0], t[1], t[2], t[3]};
+  qfma(p, ms, C.delta);
+  o.u = qscale(xi, C.gam);
+  o.w = qaxpy(p, -C.K, o.u);
+  o.x = qsub(ms, quat{t[4], t[5], t[6], t[7]});
+  qfma_cr(o.x, qneg(o.u), C.wc1);
+  qfma_cr(o.x, qneg(o.w), C.u1);
+  return o;
+}
+// Tall-skinny partials of the updated column over the panel columns 0..j:
+// this thread's columns l = q + 16 k (l = j: the new u, w) against x, summed
+// over the 16 rows, to tsp[8 l + component] (W^* x, then V^* x).
+template <int KPT>
+__device__ __forceinline__ void row_tsp(const quat* vv, const quat* ww, const quat& u, const quat& w, const quat& x,
+                                        int q, int j, double* tsp) {
+#pragma clang fp contract(off)
+  constexpr int NV = 8 * KPT;
+  double v[NV];
+#pragma unroll
+  for (int k = 0; k < KPT; ++k) {
+    const int l = q + 16 * k;
+    quat ta = qzero(), tb = qzero();
+    if (l <= j) {
+      qfma_cl(ta, l == j ? w : ww[k], x);
+      qfma_cl(tb, l == j ? u : vv[k], x);
+    }
+    v[8 * k + 0] = ta.ar; v[8 * k + 1] = ta.ai; v[8 * k + 2] = ta.br; v[8 * k + 3] = ta.bi;
+    v[8 * k + 4] = tb.ar; v[8 * k + 5] = tb.ai; v[8 * k + 6] = tb.br; v[8 * k + 7] = tb.bi;
+  }
+  row16_halving<NV>(v);
+  const int r = threadIdx.x & (RQ - 1);
+  if constexpr (KPT == 1) {   // lane r holds value r / 2
+    if ((r & 1) == 0 && q <= j) tsp[8 * q + (r >> 1)] = v[0];
+  } else {
+#pragma unroll
+    for (int t = 0; t < NV / 16; ++t) {
+      const int idx = r * (NV / 16) + t;
+      const int l = q + 16 * (idx >> 3);
+      if (l <= j) tsp[8 * l + (idx & 7)] = v[t];
+    }
+  }
+}
+
+// Column c's w_j and, inside a panel, column c+1's pending update, in one
+// pass over rows s0 + 1 .. n - 1 (s0 = c + 1; 16 threads per row, KPT panel
+// columns each): w_j stored in W[:, j], u in M[s0:, c], and unless column c
+// closes its panel (j = nb - 1) or the reduction (c = n - 2) the updated
+// column c+1 in M, its tail-norm partials in part, and the per-16-row partials
+// of W^* x, V^* x in TSP.  Two barriers: the block sums, and the four waves'
+// shares of each row; every thread then forms its row's results itself.
+// At trailing sizes below ~1500 a block's time is one round trip to memory
+// plus the instructions of one wave per SIMD, so both the barriers and the
+// instruction count are its cost: two barriers instead of four, the eleven
+// block sums by one halving butterfly instead of a full sum each, the sums in
+// scalar registers (1300 -> 1000 instructions, 9.8 -> 9.0 us per column with
+// its matvec at panel width 16; 2n = 1024 reduction 4.74 -> 4.37 ms, 2n = 8192
+// 111.0 -> 107.8 ms).  Fusing it into the next column's matvec (one launch per
+// column, every tile block repeating the row work of its 96 rows) took 11-12 us
+// per column: twice the instructions on every wave.
 // PY, PQ: partial loads per thread per gather batch (quaternion row partials,
 // x^* M x partials); WPE: the waves per SIMD the register budget aims at.
 template <int KPT, int PY, int PQ, int WPE>
@@ -334,25 +487,23 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
                                              quat* __restrict__ W, int ldw, const quat* __restrict__ Prow,
                                              const quat* __restrict__ Pcol, int ldp, const quat* __restrict__ TS,
                                              int nb, const double* __restrict__ scal, const double* __restrict__ QF,
-                                             double* __restrict__ part, double* __restrict__ TSP, int ldtsp, int tsm,
-                                             ZB zb) {
+                                             double* __restrict__ part, double* __restrict__ TSP, int ldtsp,
+                                             double* __restrict__ d, int tsm, ZB zb) {
   if (zb.nvec) {
     n = zb.nvec[blockIdx.z];
-    if (c + 1 + (int)blockIdx.x * RQ >= n) return;
+    if (blockIdx.x > 0 && c + 2 + (int)blockIdx.x * RQ >= n) return;
     M = zoff(M, zb); W = zoff(W, zb); Prow = zoff(Prow, zb); Pcol = zoff(Pcol, zb); TS = zoff(TS, zb);
-    scal = zoff(scal, zb); QF = zoff(QF, zb); part = zoff(part, zb); TSP = zoff(TSP, zb);
+    scal = zoff(scal, zb); QF = zoff(QF, zb); part = zoff(part, zb); TSP = zoff(TSP, zb); d = zoff(d, zb);
   }
   __shared__ quat a[NBMAX], b[NBMAX], cw[NBMAX], cv[NBMAX];
-  __shared__ double red[16][8][RQ];   // k-group, (p | column update) component, row
-  __shared__ double red2[8][RQ];      // the same summed over the k-groups
-  __shared__ double shr[RB / 64][10];
-  __shared__ quat xs[RQ], us[RQ], ws[RQ];
+  __shared__ double red[RB / 64][RQ][8];   // wave, row, (p | column update) component
+  __shared__ double shr[RB / 64][16];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
   const int s0 = c + 1;
   const bool more = (j + 1 < nb) && (c + 1 <= n - 2);   // uniform
   const int r = tid & (RQ - 1), q = tid >> 4;
-  const int i = s0 + blockIdx.x * RQ + r;
+  const int i = s0 + 1 + blockIdx.x * RQ + r;
   const int ic = min(i, n - 1);
   const int jl = j > 0 ? j - 1 : 0;
   // ---- loads, all issued up front
@@ -364,7 +515,7 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
     ww[k] = qload(W + ic + (size_t)l * ldw);
   }
   const quat xi = qload(M + ic + (size_t)c * ld);
-  const quat ms0raw = qload(M + ic + (size_t)s0 * ld);   // stale column s0 = c+1 (row i)
+  const quat ms = qload(M + ic + (size_t)s0 * ld);   // stale column s0 = c+1 (row i)
   // The column scalars (gamma, u1, x1, M[s0, s0]) in one vector load over
   // lanes 0..9, taken apart after the partial gathers.  As scalar loads they
   // would share the scalar-load counter with the kernel arguments the gather
@@ -418,138 +569,44 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
     for (int u = 0; u < PQ; ++u) qf += pq[u];
     w0 = qadd(w0, pw);
   }
-  const double gam = lane_d(sv, 0);
-  const quat u1 = quat{lane_d(sv, 1), lane_d(sv, 2), lane_d(sv, 3), lane_d(sv, 4)};
-  const quat x1 = quat{lane_d(sv, 5), lane_d(sv, 6), lane_d(sv, 7), lane_d(sv, 8)};
-  const double m00 = lane_d(sv, 9);   // M[s0, s0] itself is rewritten by this grid (row s0 of column s0)
-  // ---- block sums: x^* M x, Re(a^* b), (M x)_{s0}, V(s0,:) a + W(s0,:) b
-  {
-    quat rd = qmul(cvl, al);
-    qfma(rd, cwl, bl);
-    double v[10] = {qf, al.ar * bl.ar + al.ai * bl.ai + al.br * bl.br + al.bi * bl.bi,
-                    w0.ar, w0.ai, w0.br, w0.bi, rd.ar, rd.ai, rd.br, rd.bi};
-#pragma unroll
-    for (int t = 0; t < 10; ++t) v[t] = wave_sum_d(v[t]);
-    if (lane == 0)
-#pragma unroll
-      for (int t = 0; t < 10; ++t) shr[wv][t] = v[t];
-  }
-  if (tid < j) {
+  col_wave_sums(qf, w0, al, bl, cvl, cwl, shr[wv]);
+  if (tid < 16 * KPT) {   // zero beyond j
     a[tid] = al;
     b[tid] = bl;
     cw[tid] = qconj(cwl);
     cv[tid] = qconj(cvl);
   }
   __syncthreads();
-  double S[10];
+  // lane t sums the four waves' partials of sum t; then all in scalar registers
+  const int tl = lane & 15;
+  const double st = ((shr[0][tl] + shr[1][tl]) + shr[2][tl]) + shr[3][tl];
+  double S[NCS];
 #pragma unroll
-  for (int t = 0; t < 10; ++t) {
-    double x = 0.0;
-#pragma unroll
-    for (int k = 0; k < RB / 64; ++k) x += shr[k][t];
-    S[t] = x;
+  for (int t = 0; t < NCS; ++t) S[t] = lane_d(st, t);
+  const double m00 = lane_d(sv, 9);
+  const ColScalars C = col_scalars(S, lane_d(sv, 0), quat{lane_d(sv, 1), lane_d(sv, 2), lane_d(sv, 3), lane_d(sv, 4)},
+                                   quat{lane_d(sv, 5), lane_d(sv, 6), lane_d(sv, 7), lane_d(sv, 8)}, m00);
+  if (blockIdx.x == 0 && tid == 0) {   // row s0
+    qstore(M + s0 + (size_t)c * ld, C.u1);
+    qstore(W + s0 + (size_t)j * ldw, C.wc1);
+    if (more) d[s0] = C.dnext;
   }
-  const quat delta = qsub(u1, qscale(x1, gam));
-  const quat wrow = quat{S[2], S[3], S[4], S[5]};   // (M x)_{s0}
-  const double uy = gam * gam * S[0] +
-                    2.0 * gam * (delta.ar * wrow.ar + delta.ai * wrow.ai + delta.br * wrow.br + delta.bi * wrow.bi) +
-                    m00 * qnorm2(delta);
-  const double K = 0.5 * (uy - 2.0 * S[1]);
-  // p and w_j at row s0 (= c+1), needed by every block for column c+1's update
-  const quat ps0 = qsub(qadd(qscale(wrow, gam), qscale(delta, m00)), quat{S[6], S[7], S[8], S[9]});
-  const quat wc1 = qsub(ps0, qscale(u1, K));
-  // ---- this thread's shares: y(i) minus corrections, and column c+1's update over l < j
-  // branch-free (reads at a clamped index, results selected) so that every
-  // LDS read is issued before the first is used
-  quat accp = qscale(yi, gam), accu = qzero();
-#pragma unroll
-  for (int k = 0; k < KPT; ++k) {
-    const int l = q + 16 * k;
-    const bool on = l < j;
-    const int lc = on ? l : 0;
-    const quat ak = a[lc], bk = b[lc], cwk = cw[lc], cvk = cv[lc];
-    quat tp = qmul(vv[k], ak);
-    qfma(tp, ww[k], bk);
-    quat tu = qmul(vv[k], cwk);
-    qfma(tu, ww[k], cvk);
-    if (on) {
-      accp = qsub(accp, tp);
-      accu = qadd(accu, tu);
-    }
-  }
-  red[q][0][r] = accp.ar; red[q][1][r] = accp.ai; red[q][2][r] = accp.br; red[q][3][r] = accp.bi;
-  red[q][4][r] = accu.ar; red[q][5][r] = accu.ai; red[q][6][r] = accu.br; red[q][7][r] = accu.bi;
+  row_share<KPT>(vv, ww, yi, C.gam, q, j, a, b, cw, cv, red[wv]);
   __syncthreads();
-  // sums over the 16 k-groups, one (component, row) per thread
-  if (tid < 8 * RQ) {
-    const int rr = tid & (RQ - 1), comp = tid >> 4;
-    double t = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) t += red[k][comp][rr];
-    red2[comp][rr] = t;
-  }
-  __syncthreads();
-  double ss = 0.0;
-  if (q == 0) {
-    quat xn = qzero(), ui = qzero(), wi = qzero();
-    if (i < n) {
-      const quat ms0 = (i == s0) ? quat{ms0raw.ar, 0.0, 0.0, 0.0} : ms0raw;   // Hermitian diagonal: real
-      const quat pv = qadd(qmul(ms0, delta), quat{red2[0][r], red2[1][r], red2[2][r], red2[3][r]});
-      const quat su = quat{red2[4][r], red2[5][r], red2[6][r], red2[7][r]};
-      ui = (i == s0) ? u1 : qscale(xi, gam);
-      wi = qsub(pv, qscale(ui, K));
-      qstore(W + i + (size_t)j * ldw, wi);
-      qstore(M + i + (size_t)c * ld, ui);
-      if (more) {
-        // column c+1, row i: stale value minus the panel's columns 0..j
-        xn = qsub(ms0raw, su);
-        xn = qsub(xn, qmul(ui, qconj(wc1)));
-        xn = qsub(xn, qmul(wi, qconj(u1)));
-        qstore(M + i + (size_t)s0 * ld, xn);
-        if (i >= s0 + 2) ss = qnorm2(xn);
-        else xn = qzero();
-      }
-    }
-    xs[r] = xn;
-    us[r] = ui;
-    ws[r] = wi;
+  RowOut o = row_finish(red, r, C, xi, ms);
+  if (q == 0 && i < n) {
+    qstore(W + i + (size_t)j * ldw, o.w);
+    qstore(M + i + (size_t)c * ld, o.u);
+    if (more) qstore(M + i + (size_t)s0 * ld, o.x);
   }
   if (!more) return;   // uniform
-  __syncthreads();   // publishes xs, us, ws
-  // the tail-norm terms live in lanes 0..15 of wave 0 (q == 0), zero elsewhere
+  // row s0 + 1 is the updated column's x_1: not in its tail
+  if (i <= s0 + 1 || i >= n) o.x = qzero();
   if (wv == 0) {
-    ss = wave_sum_d(ss);
+    const double ss = wave_sum_d(q == 0 ? qnorm2(o.x) : 0.0);
     if (lane == 0) part[blockIdx.x] = ss;
   }
-  // tall-skinny partials of column c+1 over the panel columns 0..j (j + 1 of them):
-  // this thread's columns l = q + 16 k against x(row r), summed over the 16 rows
-  {
-    constexpr int NV = (8 * KPT < 16) ? 16 : 8 * KPT;
-    double v[NV];
-#pragma unroll
-    for (int t = 0; t < NV; ++t) v[t] = 0.0;
-    const quat x = xs[r];
-#pragma unroll
-    for (int k = 0; k < KPT; ++k) {
-      const int l = q + 16 * k;
-      if (l <= j) {
-        const quat wl = (l == j) ? ws[r] : ww[k];
-        const quat vl = (l == j) ? us[r] : vv[k];
-        quat ta = qzero(), tb = qzero();
-        qfma_cl(ta, wl, x);
-        qfma_cl(tb, vl, x);
-        v[8 * k + 0] = ta.ar; v[8 * k + 1] = ta.ai; v[8 * k + 2] = ta.br; v[8 * k + 3] = ta.bi;
-        v[8 * k + 4] = tb.ar; v[8 * k + 5] = tb.ai; v[8 * k + 6] = tb.br; v[8 * k + 7] = tb.bi;
-      }
-    }
-    row16_halving<NV>(v);
-#pragma unroll
-    for (int t = 0; t < NV / 16; ++t) {
-      const int idx = r * (NV / 16) + t;
-      const int k = idx >> 3, l = q + 16 * k;
-      if (k < KPT && l <= j) TSP[(size_t)blockIdx.x * ldtsp + 8 * l + (idx & 7)] = v[t];
-    }
-  }
+  row_tsp<KPT>(vv, ww, o.u, o.w, o.x, q, j, TSP + (size_t)blockIdx.x * ldtsp);
 }
 
 // ---------------------------------------------------------------------------
@@ -729,8 +786,8 @@ int reduce(quat* M, int n, int ld, int nb, double* d, quat* e, const ReduceWork&
     const int wdt = (nb < n - 1 - p) ? nb : (n - 1 - p);
     for (int j = 0; j < wdt; ++j) {
       const int c = p + j;
-      const int nblk = cdiv(n - c, RQ);            // row blocks from c
       const int sz = n - c - 1;                    // trailing size
+      const int nparts = cdiv(sz, RQ);             // partials the column kernel left for this column
       const int G = cdiv(sz, SG);
       const int spg = matvec_spg(sz, w.tsm);
       const int nmain = ntiles(G, spg) + (j > 0 ? (8 * j + 63) / 64 : 1);
@@ -738,14 +795,14 @@ int reduce(quat* M, int n, int ld, int nb, double* d, quat* e, const ReduceWork&
         // algorithmic bytes: one read of the trailing lower triangle
         ProfScope ps(PROF_SYMV, s, 32.0 * 0.5 * (double)sz * (sz + 1));
         if (spg == 4)
-          launch_k(k_symv<256, 16>, dim3(nmain), dim3(256), 0, s, M, ld, n, p, c, j, w.W, ldw, w.part, nblk,
+          launch_k(k_symv<256, 16>, dim3(nmain), dim3(256), 0, s, M, ld, n, p, c, j, w.W, ldw, w.part, nparts,
                    w.scal, d, e, w.Prow, w.Pcol, n, w.TS, nb, w.TSP, w.ldtsp, w.QF, ZB{nullptr, 0});
         else
-          launch_k(k_symv<512, 32>, dim3(nmain), dim3(512), 0, s, M, ld, n, p, c, j, w.W, ldw, w.part, nblk,
+          launch_k(k_symv<512, 32>, dim3(nmain), dim3(512), 0, s, M, ld, n, p, c, j, w.W, ldw, w.part, nparts,
                    w.scal, d, e, w.Prow, w.Pcol, n, w.TS, nb, w.TSP, w.ldtsp, w.QF, ZB{nullptr, 0});
       }
-      launch_wcol(kpt, sz, dim3(cdiv(sz, RQ)), s, M, ld, n, p, c, j, w.W, ldw, w.Prow, w.Pcol, n, w.TS, nb, w.scal,
-                  w.QF, w.part, w.TSP, w.ldtsp, w.tsm, ZB{nullptr, 0});
+      launch_wcol(kpt, sz, dim3(std::max(1, cdiv(sz - 1, RQ))), s, M, ld, n, p, c, j, w.W, ldw, w.Prow, w.Pcol, n, w.TS,
+                  nb, w.scal, w.QF, w.part, w.TSP, w.ldtsp, d, w.tsm, ZB{nullptr, 0});
     }
     // trailing update of rows/cols [p+wdt, n): M -= [V W] [W V]^*  (lower triangle)
     const int r0 = p + wdt;
@@ -826,9 +883,8 @@ int reduce_batched(int nprob, const int* nh, ZB zb, quat* M, int ld, int nb, dou
   for (int c = 0; c < cend; ++c) {
     while (act > 0 && lim[act - 1] <= c) --act;
     const int p = (c / nb) * nb, j = c - p;
-    const int nrow = L - c;
-    const int nblk = cdiv(nrow, RQ);
     const int sz = L - c - 1;
+    const int nparts = cdiv(sz, RQ);
     const int NF = j > 0 ? (8 * j + 63) / 64 : 1;
     // each problem's matvec takes the tile shape of its own trailing size:
     // problems [0, k1) wide strips, [k1, act) narrow ones (sizes descending)
@@ -843,19 +899,19 @@ int reduce_batched(int nprob, const int* nh, ZB zb, quat* M, int ld, int nb, dou
     if (k1 > 0) {
       ProfScope ps(PROF_SYMV, s, tri_bytes(0, k1));
       launch_k(k_symv<512, 32>, dim3(ntiles(cdiv(sz, SG), 2) + NF, 1, k1), dim3(512), 0, s, M, ld, L, p, c, j, w.W,
-               ldw, w.part, nblk, w.scal, d, e, w.Prow, w.Pcol, ld, w.TS, nb, w.TSP, w.ldtsp, w.QF, zb);
+               ldw, w.part, nparts, w.scal, d, e, w.Prow, w.Pcol, ld, w.TS, nb, w.TSP, w.ldtsp, w.QF, zb);
     }
     if (k1 < act) {
       const size_t sh = (size_t)k1 * zb.zs;
       const int szn = nh[k1] - c - 1;
       ProfScope ps(PROF_SYMV, s, tri_bytes(k1, act));
       launch_k(k_symv<256, 16>, dim3(ntiles(cdiv(szn, SG), 4) + NF, 1, act - k1), dim3(256), 0, s, zshift(M, sh), ld,
-               L, p, c, j, zshift(w.W, sh), ldw, zshift(w.part, sh), nblk, zshift(w.scal, sh), zshift(d, sh),
+               L, p, c, j, zshift(w.W, sh), ldw, zshift(w.part, sh), nparts, zshift(w.scal, sh), zshift(d, sh),
                zshift(e, sh), zshift(w.Prow, sh), zshift(w.Pcol, sh), ld, zshift(w.TS, sh), nb, zshift(w.TSP, sh),
                w.ldtsp, zshift(w.QF, sh), ZB{zb.nvec + k1, zb.zs});
     }
-    launch_wcol(kpt, sz, dim3(cdiv(sz, RQ), 1, act), s, M, ld, L, p, c, j, w.W, ldw, w.Prow, w.Pcol, ld, w.TS, nb,
-                w.scal, w.QF, w.part, w.TSP, w.ldtsp, w.tsm, zb);
+    launch_wcol(kpt, sz, dim3(std::max(1, cdiv(sz - 1, RQ)), 1, act), s, M, ld, L, p, c, j, w.W, ldw, w.Prow, w.Pcol,
+                ld, w.TS, nb, w.scal, w.QF, w.part, w.TSP, w.ldtsp, d, w.tsm, zb);
     if (j == nb - 1 || c == cend - 1) {
       const int P = c / nb;
       const int cnt = toff[P + 1] - toff[P];

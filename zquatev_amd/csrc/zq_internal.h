@@ -75,9 +75,16 @@ __device__ __forceinline__ quat qscale(const quat& x, double s) {
   return quat{x.ar * s, x.ai * s, x.br * s, x.bi * s};
 }
 __device__ __forceinline__ quat qconj(const quat& x) { return quat{x.ar, -x.ai, -x.br, -x.bi}; }
-__device__ __forceinline__ double qnorm2(const quat& x) {
-  return x.ar * x.ar + x.ai * x.ai + x.br * x.br + x.bi * x.bi;
+// Re(conj(x) y), the dot product of the components
+__device__ __forceinline__ double qdot(const quat& x, const quat& y) {
+  return fma(x.bi, y.bi, fma(x.br, y.br, fma(x.ai, y.ai, x.ar * y.ar)));
 }
+__device__ __forceinline__ double qnorm2(const quat& x) { return qdot(x, x); }
+// x + s y
+__device__ __forceinline__ quat qaxpy(const quat& x, double s, const quat& y) {
+  return quat{fma(s, y.ar, x.ar), fma(s, y.ai, x.ai), fma(s, y.br, x.br), fma(s, y.bi, x.bi)};
+}
+__device__ __forceinline__ quat qneg(const quat& x) { return quat{-x.ar, -x.ai, -x.br, -x.bi}; }
 
 // x * y
 __device__ __forceinline__ quat qmul(const quat& x, const quat& y) {
@@ -112,7 +119,7 @@ __device__ __forceinline__ double shfl_xor_d(double v, int m) {
 }
 
 // ---- cross-lane exchanges without the LDS crossbar (gfx950) ----------------
-// xor 1, 2, 4, 8 inside a 16-lane row through DPP; the row-crossing steps of a
+// lane bits 0 .. 3 inside a 16-lane row through DPP; the row-crossing steps of a
 // butterfly through v_permlane16_swap / v_permlane32_swap.
 __device__ __forceinline__ unsigned lo32(double v) { return (unsigned)(unsigned long long)__double_as_longlong(v); }
 __device__ __forceinline__ unsigned hi32(double v) {
@@ -125,24 +132,23 @@ __device__ __forceinline__ double mkd(unsigned lo, unsigned hi) {
 __device__ __forceinline__ double lane_d(double v, int k) {
   return mkd((unsigned)__builtin_amdgcn_readlane((int)lo32(v), k), (unsigned)__builtin_amdgcn_readlane((int)hi32(v), k));
 }
+// Every lane of these patterns reads a lane of its own row, so the bound
+// control never acts; with it set the destination's old value is dead and
+// needs no v_mov.
 template <int CTRL>
 __device__ __forceinline__ double dppd(double v) {
-  return mkd(__builtin_amdgcn_update_dpp(0u, lo32(v), CTRL, 0xF, 0xF, false),
-             __builtin_amdgcn_update_dpp(0u, hi32(v), CTRL, 0xF, 0xF, false));
+  return mkd(__builtin_amdgcn_update_dpp(0u, lo32(v), CTRL, 0xF, 0xF, true),
+             __builtin_amdgcn_update_dpp(0u, hi32(v), CTRL, 0xF, 0xF, true));
 }
-// xor 4: row_shl:4 on banks 0 and 2, row_shr:4 on banks 1 and 3
-__device__ __forceinline__ double dpp_xor4(double v) {
-  unsigned l = __builtin_amdgcn_update_dpp(0u, lo32(v), 0x104, 0xF, 0x5, false);
-  l = __builtin_amdgcn_update_dpp(l, lo32(v), 0x114, 0xF, 0xA, false);
-  unsigned h = __builtin_amdgcn_update_dpp(0u, hi32(v), 0x104, 0xF, 0x5, false);
-  h = __builtin_amdgcn_update_dpp(h, hi32(v), 0x114, 0xF, 0xA, false);
-  return mkd(l, h);
-}
-// value of v in lane (lane ^ M), M in {1, 2, 4, 8}
+// Partner's value for the butterfly step over lane bit M in {1, 2, 4, 8}.
+// The partner differs in bit M; for M = 4 it is lane 7 - i of the eight
+// (row_half_mirror, one move where xor 4 takes two masked ones), which differs
+// in the lower bits too: a sum over all lanes of the lower bits, as every
+// user here goes on to take, is the same set of terms.
 template <int M>
 __device__ __forceinline__ double xlane(double v) {
   if (M == 8) return dppd<0x128>(v);   // row_ror:8
-  if (M == 4) return dpp_xor4(v);
+  if (M == 4) return dppd<0x141>(v);   // row_half_mirror
   if (M == 2) return dppd<0x4E>(v);    // quad_perm [2,3,0,1]
   return dppd<0xB1>(v);                // quad_perm [1,0,3,2]
 }
@@ -198,16 +204,17 @@ __device__ __forceinline__ double butterfly_sum(double* v) {
   if (N == 1) r = bf32(r, r);
   return r;
 }
-// Halving butterfly inside each 16-lane row for N (power of two, >= 16)
-// values per lane: afterwards v[t], t < N/16, of lane l holds the row sum of
-// value (l & 15) * (N/16) + t.
+// Halving butterfly inside each 16-lane row for N (power of two, >= 8) values
+// per lane: afterwards v[t], t < max(1, N / 16), of lane l holds the row sum
+// of value (l & 15) * N / 16 + t.
 template <int N>
 __device__ __forceinline__ void row16_halving(double* v) {
   const int lane = threadIdx.x & 63;
   bstep<8, N / 2>(v, lane);
   bstep<4, N / 4>(v, lane);
   bstep<2, N / 8>(v, lane);
-  bstep<1, N / 16>(v, lane);
+  if (N >= 16) bstep<1, (N >= 16 ? N / 16 : 1)>(v, lane);
+  else v[0] += xlane<1>(v[0]);
 }
 // sum over all 64 lanes, result in every lane
 __device__ __forceinline__ double wave_sum_d(double v) {
