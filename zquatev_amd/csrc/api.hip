@@ -263,8 +263,9 @@ void slab_layout(Bump& b, int n, int nb, bool vectors, Plan* p) {
   p->e = b.take<quat>(nmax);
   p->ea = b.take<double>(nmax);
   p->rw.W = b.take<quat>((size_t)n * nb);
-  p->rw.Prow = b.take<quat>((size_t)zq::matvec_row_slots(nmax) * n);
-  p->rw.Pcol = b.take<quat>((size_t)zq::matvec_col_slots(nmax) * n);
+  p->rw.pcs = zq::matvec_row_slots(nmax);
+  p->rw.Prow = b.take<quat>((size_t)(p->rw.pcs + zq::matvec_col_slots(nmax)) * n);
+  p->rw.Pcol = p->rw.Prow ? p->rw.Prow + (size_t)p->rw.pcs * n : nullptr;
   p->rw.TS = b.take<quat>((size_t)2 * nb);
   p->rw.ldtsp = 8 * nb;
   p->rw.TSP = b.take<double>((size_t)(cdiv(nmax, 16) + 1) * 8 * nb);

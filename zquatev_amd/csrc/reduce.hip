@@ -109,20 +109,19 @@ __device__ __forceinline__ Refl reflector(const quat& x1, double tail, quat* alp
 // TS = [W^* u | V^* u]: they add the per-block partials of W^* x and V^* x
 // that k_wcol left in TSP (the waves over the partial index, then the
 // wave sums, in a fixed order), scale by gamma and add the row s0 term.
-template <int SYT, int SW>
-__global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld, int n, int p, int c, int j,
-                                              const quat* __restrict__ W, int ldw, const double* __restrict__ part,
-                                              int nparts, double* __restrict__ scal, double* __restrict__ d,
-                                              quat* __restrict__ e, quat* __restrict__ Prow, quat* __restrict__ Pcol,
-                                              int ldp, quat* __restrict__ TS, int nb, const double* __restrict__ TSP,
-                                              int ldtsp, double* __restrict__ QF, ZB zb) {
+template <int SYT, int SW, bool BT>
+__global__ void __launch_bounds__(SYT) k_symv(
+    const quat* __restrict__ M, const quat* __restrict__ W, const double* __restrict__ TSP,
+    const double* __restrict__ part, int ld, int n, int p, int c, int j, int ldw, int nparts, int ldtsp,
+    double* __restrict__ scal, double* __restrict__ d, quat* __restrict__ e, quat* __restrict__ Prow,
+    quat* __restrict__ Pcol, int ldp, int nb, quat* __restrict__ TS, double* __restrict__ QF, ZB zb) {
   constexpr int NWV = SYT / 64;    // waves per block
   constexpr int SCW = SW / NWV;     // strip columns per wave
   constexpr int SPG = SG / SW;      // strips per row group and group index
   static_assert(SW <= SG && SG % SW == 0 && SW % NWV == 0, "matvec tile shape");
   const int NT = j > 0 ? (8 * j + 63) / 64 : 0;
   const int NF = NT > 0 ? NT : 1;
-  if (zb.nvec) {
+  if constexpr (BT) {
     n = zb.nvec[blockIdx.z];
     nparts = (n - c - 1 + RQ - 1) / RQ;
     const int Gz = (n - c - 1 + SG - 1) / SG;
@@ -213,7 +212,7 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
     return;
   }
   // ---- tile block: block -> (g, J) with ntiles(g) <= b < ntiles(g + 1)
-  int g = (int)((sqrt(8.0 * b / SPG + 1.0) - 1.0) * 0.5);
+  int g = (int)((sqrtf(8.0f / SPG * (float)b + 1.0f) - 1.0f) * 0.5f);   // corrected below
   while (ntiles(g + 1, SPG) <= b) ++g;
   while (ntiles(g, SPG) > b) --g;
   const int J = b - ntiles(g, SPG);
@@ -295,19 +294,20 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
   qfl = wave_sum_d(qfl);
   if (lane == 0) sqf[w] = qfl;
   __syncthreads();
-  if (tid == 0) {
+  // wave v < 4 sums component v of the rows; the last wave x^* M x too
+  if (tid == SYT - 64) {
     double t = 0.0;
 #pragma unroll
     for (int k = 0; k < SYT / 64; ++k) t += sqf[k];
     QF[b] = t;
   }
-  if (active && tid < SG) {
-    const int i = R0 + tid;
+  if (active && w < 4) {
+    const int i = R0 + lane;
     if (i < n && i >= C0) {
-      quat sum = qzero();
+      double t = red[0][w][lane];
 #pragma unroll
-      for (int k = 0; k < NWV; ++k) sum = qadd(sum, quat{red[k][0][tid], red[k][1][tid], red[k][2][tid], red[k][3][tid]});
-      qstore(Prow + (size_t)J * ldp + i, sum);
+      for (int k = 1; k < NWV; ++k) t += red[k][w][lane];
+      reinterpret_cast<double*>(Prow + (size_t)J * ldp + i)[w] = t;
     }
   }
 }
@@ -334,51 +334,59 @@ __global__ void __launch_bounds__(SYT) k_symv(const quat* __restrict__ M, int ld
 // the 16-row groups of the tall-skinny partials are the rows of the next
 // matvec's tiles.
 //
-// NCS block sums per column: 0 x^* M x, 1 Re(a^* b), 2-5 (M x)_{s0},
-// 6-9 V(s0,:) a + W(s0,:) b, 10 Re(V(s0,:) conj(W(s0,:))).
-constexpr int NCS = 11;
+// Block sums per column: qf = x^* M x, ab = Re(a^* b), wrow = (M x)_{s0},
+// rd = V(s0,:) a + W(s0,:) b, cc = Re(V(s0,:) conj(W(s0,:))).
 struct ColScalars {
   double gam, K;
   quat u1, delta, wc1;   // wc1 = w_j(s0)
   double dnext;          // the updated diagonal entry at s0
 };
-__device__ __forceinline__ ColScalars col_scalars(const double* S, double gam, const quat& u1, const quat& x1,
-                                                  double m00) {
+__device__ __forceinline__ ColScalars col_scalars(double qf, double ab, double cc, const quat& rd, const quat& wrow,
+                                                  double gam, const quat& u1, const quat& x1, double m00) {
 #pragma clang fp contract(off)
   ColScalars C;
   C.gam = gam;
   C.u1 = u1;
   C.delta = qaxpy(u1, -gam, x1);
-  const quat wrow = quat{S[2], S[3], S[4], S[5]};   // (M x)_{s0}
-  const double uy = fma(gam * gam, S[0], fma(2.0 * gam, qdot(C.delta, wrow), m00 * qnorm2(C.delta)));
-  C.K = 0.5 * fma(-2.0, S[1], uy);
-  const quat ps0 = qsub(qaxpy(qscale(wrow, gam), m00, C.delta), quat{S[6], S[7], S[8], S[9]});
+  const double uy = fma(gam * gam, qf, fma(2.0 * gam, qdot(C.delta, wrow), m00 * qnorm2(C.delta)));
+  C.K = 0.5 * fma(-2.0, ab, uy);
+  const quat ps0 = qsub(qaxpy(qscale(wrow, gam), m00, C.delta), rd);
   C.wc1 = qaxpy(ps0, -C.K, u1);
-  C.dnext = fma(-2.0, qdot(u1, C.wc1), fma(-2.0, S[10], m00));
+  C.dnext = fma(-2.0, qdot(u1, C.wc1), fma(-2.0, cc, m00));
   return C;
 }
-// This thread's terms of the block sums (thread l < j holds panel column l's
-// coefficients), summed over the wave: lane t < 16 of sh holds sum t.
-__device__ __forceinline__ void col_wave_sums(double qf, const quat& w0, const quat& al, const quat& bl,
-                                              const quat& cvl, const quat& cwl, double* sh) {
+// The block sums, from the first two waves' lanes (wave 0: lane l < j holds
+// panel column l's coefficients, or with two columns per lane l and l + 64;
+// wave 1: the terms of (M x)_{s0}); x^* M x terms are in every lane.  Each wave
+// sums only what it holds: sh[wave][t] = its sum t.
+__device__ __forceinline__ void col_wave_sums(int wv, double qf, const quat& w0, double ab, const quat& rd, double cc,
+                                              double (*sh)[8]) {
 #pragma clang fp contract(off)
-  quat rd = qzero();
-  qfma(rd, cvl, al);
-  qfma(rd, cwl, bl);
-  double v[16] = {qf, qdot(al, bl), w0.ar, w0.ai, w0.br, w0.bi, rd.ar, rd.ai, rd.br, rd.bi, qdot(cvl, cwl),
-                  0.0, 0.0, 0.0, 0.0, 0.0};
-  const double t = butterfly_sum<16>(v);
   const int lane = threadIdx.x & 63;
-  if ((lane & 3) == 0) sh[lane >> 2] = t;
+  if (wv == 0) {
+    double v[8] = {qf, ab, cc, rd.ar, rd.ai, rd.br, rd.bi, 0.0};
+    const double t = butterfly_sum<8>(v);
+    if ((lane & 7) == 0) sh[0][lane >> 3] = t;
+  } else if (wv == 1) {
+    double v[8] = {qf, w0.ar, w0.ai, w0.br, w0.bi, 0.0, 0.0, 0.0};
+    const double t = butterfly_sum<8>(v);
+    if ((lane & 7) == 0) sh[1][lane >> 3] = t;
+  } else {
+    const double t = wave_sum_d(qf);
+    if (lane == 0) sh[wv][0] = t;
+  }
 }
 // One thread's share of a row, over the panel columns l = q + 16 k (its
 // coefficients vv, ww): ps = gamma y - (V a + W b), us = V conj(W(s0)) + W
 // conj(V(s0)); then summed over the wave's four q: lane 16 q' + r is left
 // with components 2 q', 2 q' + 1 of row r's (ps, us), stored in red[r].
+// RPAD: a row's 8 components and a gap of 2, which puts the 16 rows' 16-byte
+// accesses in distinct banks.
+constexpr int RPAD = 10;
 template <int KPT>
 __device__ __forceinline__ void row_share(const quat* vv, const quat* ww, const quat& yi, double gam, int q, int j,
                                           const quat* a, const quat* b, const quat* cw, const quat* cv,
-                                          double (*red)[8]) {
+                                          double (*red)[RPAD]) {
 #pragma clang fp contract(off)
   quat accp = qscale(yi, gam), accu = qzero();
   // the coefficients beyond j are zero in LDS (and vv, ww finite), so no lane
@@ -404,7 +412,7 @@ __device__ __forceinline__ void row_share(const quat* vv, const quat* ww, const 
 struct RowOut {
   quat u, w, x;
 };
-__device__ __forceinline__ RowOut row_finish(const double (*red)[RQ][8], int r, const ColScalars& C, const quat& xi,
+__device__ __forceinline__ RowOut row_finish(const double (*red)[RQ][RPAD], int r, const ColScalars& C, const quat& xi,
                                              const quat& ms) {
 #pragma clang fp contract(off)
   double t[8];
@@ -482,24 +490,23 @@ __device__ __forceinline__ void row_tsp(const quat* vv, const quat* ww, const qu
 // per column: twice the instructions on every wave.
 // PY, PQ: partial loads per thread per gather batch (quaternion row partials,
 // x^* M x partials); WPE: the waves per SIMD the register budget aims at.
-template <int KPT, int PY, int PQ, int WPE>
-__global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) k_wcol(quat* __restrict__ M, int ld, int n, int p, int c, int j,
-                                             quat* __restrict__ W, int ldw, const quat* __restrict__ Prow,
-                                             const quat* __restrict__ Pcol, int ldp, const quat* __restrict__ TS,
-                                             int nb, const double* __restrict__ scal, const double* __restrict__ QF,
-                                             double* __restrict__ part, double* __restrict__ TSP, int ldtsp,
-                                             double* __restrict__ d, int tsm, ZB zb) {
-  if (zb.nvec) {
+template <int KPT, int PY, int PQ, int WPE, bool BT>
+__global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) k_wcol(
+    quat* __restrict__ M, quat* __restrict__ W, const quat* __restrict__ Prow, int pcs, int ld,
+    int n, int p, int c, int j, int ldw, int ldp, int nb, const quat* __restrict__ TS, const double* __restrict__ scal,
+    const double* __restrict__ QF, double* __restrict__ part, double* __restrict__ TSP, double* __restrict__ d,
+    int ldtsp, int tsm, ZB zb) {
+  if constexpr (BT) {
     n = zb.nvec[blockIdx.z];
     if (blockIdx.x > 0 && c + 2 + (int)blockIdx.x * RQ >= n) return;
-    M = zoff(M, zb); W = zoff(W, zb); Prow = zoff(Prow, zb); Pcol = zoff(Pcol, zb); TS = zoff(TS, zb);
+    M = zoff(M, zb); W = zoff(W, zb); Prow = zoff(Prow, zb); TS = zoff(TS, zb);
     scal = zoff(scal, zb); QF = zoff(QF, zb); part = zoff(part, zb); TSP = zoff(TSP, zb); d = zoff(d, zb);
   }
   __shared__ quat a[NBMAX], b[NBMAX], cw[NBMAX], cv[NBMAX];
-  __shared__ double red[RB / 64][RQ][8];   // wave, row, (p | column update) component
-  __shared__ double shr[RB / 64][16];
+  __shared__ __align__(16) double red[RB / 64][RQ][RPAD];   // wave, row, (p | column update) component
+  __shared__ double shr[RB / 64][8];
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wv = tid >> 6;
+  const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int s0 = c + 1;
   const bool more = (j + 1 < nb) && (c + 1 <= n - 2);   // uniform
   const int r = tid & (RQ - 1), q = tid >> 4;
@@ -521,71 +528,100 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
   // would share the scalar-load counter with the kernel arguments the gather
   // loop needs, and the loop's loads could not issue before they arrived.
   const double sv = scal[min(lane, 9)];
-  quat al = qzero(), bl = qzero(), cwl = qzero(), cvl = qzero();
-  if (tid < j) {
-    al = qload(TS + tid);
-    bl = qload(TS + nb + tid);
-    cwl = qload(W + s0 + (size_t)tid * ldw);
-    cvl = qload(M + s0 + (size_t)(p + tid) * ld);
-  }
+  // wave 0: the panel's coefficients, lane l those of columns l + 64 h
+  constexpr int NH = (16 * KPT + 63) / 64;
+  quat al[NH], bl[NH], cwl[NH], cvl[NH];
+  if (wv == 0)
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      al[h] = bl[h] = cwl[h] = cvl[h] = qzero();
+      const int l = lane + 64 * h;
+      if (l < j) {
+        al[h] = qload(TS + l);
+        bl[h] = qload(TS + nb + l);
+        cwl[h] = qload(W + s0 + (size_t)l * ldw);
+        cvl[h] = qload(M + s0 + (size_t)(p + l) * ld);
+      }
+    }
   const int G = (n - s0 + SG - 1) / SG;
-  // The matvec partials this thread sums, gathered in fixed-size batches of
-  // predicated loads so that one wait covers them all (one batch up to
-  // trailing sizes of ~4k rows with the wide variant, ~1k with the light one):
+  // The matvec partials this thread sums, gathered in fixed-size batches at
+  // clamped addresses (surplus values are dropped), so that one wait covers
+  // them all (one batch up to trailing sizes of ~4k rows with the wide variant,
+  // ~1k with the light one) and no load sits in a branch of its own:
   //   y(i):  slots k = q + 16 t of row i's list, Prow[J][i] for J <= li / SW
   //          (SW the strip width of this trailing size)
-  //          (k < nJ), then Pcol[g][i] for g >= li / SG;
+  //          (k < nJ), then Pcol[g][i] for g >= li / SG (slot pcs + g of Prow);
   //   x^* M x: QF[tid + RB t], t over the G (G + 1) tile partials;
-  //   (M x)_{s0}: Prow[0][s0] and Pcol[g][s0] as slots tid + RB t of G + 1.
+  //   (M x)_{s0}: Prow[0][s0] and Pcol[g][s0] as slots lane + 64 t of G + 1, in wave 1.
   const int li = ic - s0;
   const int spg = matvec_spg(n - s0, tsm);
   const int nJ = (spg == 4 ? li >> 4 : li >> 5) + 1, g0 = li / SG;
-  const int cy = cdiv_d(nJ + G - g0 - q, 16);
+  const int ns = nJ + G - g0;   // slots of row i
+  const int shift = pcs + g0 - nJ;
+  const int cy = cdiv_d(ns - q, 16);
   const int nq = ntiles(G, spg);
   const int cq = cdiv_d(nq - tid, RB);
-  const int cw0 = cdiv_d(G + 1 - tid, RB);
+  const int cw0 = wv == 1 ? cdiv_d(G + 1 - lane, 64) : 0;
   quat yi = qzero(), w0 = qzero();
   double qf = 0.0;
-  for (int bt = 0; bt * PY < cy || bt * PQ < cq || bt < cw0; ++bt) {
+  // surplus values are dropped by a factor 0: one select where zeroing the
+  // value takes eight (they repeat the row's last slot, so a NaN or infinity
+  // there is in the row's sum anyway)
+  auto gather = [&](int bt) {
     quat py[PY];
     double pq[PQ];
 #pragma unroll
     for (int u = 0; u < PY; ++u) {
-      const int t = bt * PY + u;
-      const int k = q + 16 * t;
-      const quat* src = k < nJ ? Prow + (size_t)k * ldp + ic : Pcol + (size_t)(g0 + k - nJ) * ldp + ic;
-      py[u] = t < cy ? qload(src) : qzero();
+      const int k = min(q + 16 * (bt * PY + u), ns - 1);
+      py[u] = qload(Prow + (unsigned)((k < nJ ? k : k + shift) * ldp + ic));
     }
 #pragma unroll
-    for (int u = 0; u < PQ; ++u) {
-      const int t = bt * PQ + u;
-      pq[u] = t < cq ? QF[tid + RB * t] : 0.0;
+    for (int u = 0; u < PQ; ++u) pq[u] = QF[(unsigned)min(tid + RB * (bt * PQ + u), nq - 1)];
+    quat pw;
+    if (wv == 1) {
+      const int k = min(lane + 64 * bt, G);
+      pw = qload(Prow + (unsigned)((k == 0 ? 0 : pcs + k - 1) * ldp + s0));
     }
-    const int kw = tid + RB * bt;
-    const quat pw = bt < cw0 ? qload(kw == 0 ? Prow + s0 : Pcol + (size_t)(kw - 1) * ldp + s0) : qzero();
 #pragma unroll
-    for (int u = 0; u < PY; ++u) yi = qadd(yi, py[u]);
+    for (int u = 0; u < PY; ++u) yi = qaxpy(yi, bt * PY + u < cy ? 1.0 : 0.0, py[u]);
 #pragma unroll
-    for (int u = 0; u < PQ; ++u) qf += pq[u];
-    w0 = qadd(w0, pw);
-  }
-  col_wave_sums(qf, w0, al, bl, cvl, cwl, shr[wv]);
-  if (tid < 16 * KPT) {   // zero beyond j
-    a[tid] = al;
-    b[tid] = bl;
-    cw[tid] = qconj(cwl);
-    cv[tid] = qconj(cvl);
+    for (int u = 0; u < PQ; ++u) qf = fma(bt * PQ + u < cq ? 1.0 : 0.0, pq[u], qf);
+    if (wv == 1) w0 = qaxpy(w0, bt < cw0 ? 1.0 : 0.0, pw);
+  };
+  gather(0);
+  const int nbt = max(max(cdiv_d(ns, 16 * PY), cdiv_d(nq, RB * PQ)), cdiv_d(G + 1, 64));
+  for (int bt = 1; bt < nbt; ++bt) gather(bt);
+  {
+#pragma clang fp contract(off)
+    quat rd = qzero();
+    double ab = 0.0, cc = 0.0;
+    if (wv == 0) {
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        qfma(rd, cvl[h], al[h]);
+        qfma(rd, cwl[h], bl[h]);
+        ab = h ? ab + qdot(al[h], bl[h]) : qdot(al[h], bl[h]);
+        cc = h ? cc + qdot(cvl[h], cwl[h]) : qdot(cvl[h], cwl[h]);
+        const int l = lane + 64 * h;
+        if (l < 16 * KPT) {   // zero beyond j
+          a[l] = al[h];
+          b[l] = bl[h];
+          cw[l] = qconj(cwl[h]);
+          cv[l] = qconj(cvl[h]);
+        }
+      }
+    }
+    col_wave_sums(wv, qf, w0, ab, rd, cc, shr);
   }
   __syncthreads();
-  // lane t sums the four waves' partials of sum t; then all in scalar registers
-  const int tl = lane & 15;
-  const double st = ((shr[0][tl] + shr[1][tl]) + shr[2][tl]) + shr[3][tl];
-  double S[NCS];
-#pragma unroll
-  for (int t = 0; t < NCS; ++t) S[t] = lane_d(st, t);
-  const double m00 = lane_d(sv, 9);
-  const ColScalars C = col_scalars(S, lane_d(sv, 0), quat{lane_d(sv, 1), lane_d(sv, 2), lane_d(sv, 3), lane_d(sv, 4)},
-                                   quat{lane_d(sv, 5), lane_d(sv, 6), lane_d(sv, 7), lane_d(sv, 8)}, m00);
+  // lane t holds sum t of wave 0 (t < 8), wave 1 (t < 16); to scalar registers
+  const double st = shr[(lane >> 3) & 1][lane & 7];
+  const double qs = ((lane_d(st, 0) + lane_d(st, 8)) + shr[2][0]) + shr[3][0];
+  const ColScalars C = col_scalars(qs, lane_d(st, 1), lane_d(st, 2),
+                                   quat{lane_d(st, 3), lane_d(st, 4), lane_d(st, 5), lane_d(st, 6)},
+                                   quat{lane_d(st, 9), lane_d(st, 10), lane_d(st, 11), lane_d(st, 12)}, lane_d(sv, 0),
+                                   quat{lane_d(sv, 1), lane_d(sv, 2), lane_d(sv, 3), lane_d(sv, 4)},
+                                   quat{lane_d(sv, 5), lane_d(sv, 6), lane_d(sv, 7), lane_d(sv, 8)}, lane_d(sv, 9));
   if (blockIdx.x == 0 && tid == 0) {   // row s0
     qstore(M + s0 + (size_t)c * ld, C.u1);
     qstore(W + s0 + (size_t)j * ldw, C.wc1);
@@ -603,7 +639,11 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
   // row s0 + 1 is the updated column's x_1: not in its tail
   if (i <= s0 + 1 || i >= n) o.x = qzero();
   if (wv == 0) {
-    const double ss = wave_sum_d(q == 0 ? qnorm2(o.x) : 0.0);
+    double ss = qnorm2(o.x);   // lanes 0..15: the 16 rows
+    ss += xlane<1>(ss);
+    ss += xlane<2>(ss);
+    ss += xlane<4>(ss);
+    ss += xlane<8>(ss);
     if (lane == 0) part[blockIdx.x] = ss;
   }
   row_tsp<KPT>(vv, ww, o.u, o.w, o.x, q, j, TSP + (size_t)blockIdx.x * ldtsp);
@@ -636,7 +676,8 @@ constexpr int TWV = TT / 64;
 constexpr int TKC = TAILN / TWV;    // columns per wave
 static_assert(TAILN == 64 && TKC * TWV == TAILN, "k_tail: lane = row, TKC columns per wave");
 
-__global__ void __launch_bounds__(TT) k_tail(quat* __restrict__ M, int ld, int n, int p, const int* __restrict__ pstart,
+__global__ void __launch_bounds__(TT) k_tail(quat* __restrict__ M, int ld, int n, int p,
+                                  const int* __restrict__ pstart,
                                              double* __restrict__ d, quat* __restrict__ e, ZB zb) {
   if (zb.nvec) {
     n = zb.nvec[blockIdx.z];
@@ -751,21 +792,21 @@ static int kpt_for(int nb) {
 
 // k_wcol variants: light gathers (more blocks per CU: batches of small
 // problems) up to trailing size 1536, wide ones (one gather batch) above.
-template <int KPT, class... Args>
+template <int KPT, bool BT, class... Args>
 static void launch_wcol_k(int sz, dim3 grid, hipStream_t s, Args... args) {
   // register budgets that compile without spills: 3 waves per SIMD at KPT 1,
   // 2 at KPT 2 and 4, 1 at KPT 8
   constexpr int WPE = KPT == 1 ? 3 : (KPT == 8 ? 1 : 2);
-  if (sz <= 1536) hipLaunchKernelGGL((k_wcol<KPT, 4, 2, WPE>), grid, dim3(RB), 0, s, args...);
-  else hipLaunchKernelGGL((k_wcol<KPT, 10, 18, 1>), grid, dim3(RB), 0, s, args...);
+  if (sz <= 1536) hipLaunchKernelGGL((k_wcol<KPT, 4, 2, WPE, BT>), grid, dim3(RB), 0, s, args...);
+  else hipLaunchKernelGGL((k_wcol<KPT, 10, 18, 1, BT>), grid, dim3(RB), 0, s, args...);
 }
-template <class... Args>
+template <bool BT, class... Args>
 static void launch_wcol(int kpt, int sz, dim3 grid, hipStream_t s, Args... args) {
   switch (kpt) {
-    case 1: launch_wcol_k<1>(sz, grid, s, args...); break;
-    case 2: launch_wcol_k<2>(sz, grid, s, args...); break;
-    case 4: launch_wcol_k<4>(sz, grid, s, args...); break;
-    default: launch_wcol_k<8>(sz, grid, s, args...); break;
+    case 1: launch_wcol_k<1, BT>(sz, grid, s, args...); break;
+    case 2: launch_wcol_k<2, BT>(sz, grid, s, args...); break;
+    case 4: launch_wcol_k<4, BT>(sz, grid, s, args...); break;
+    default: launch_wcol_k<8, BT>(sz, grid, s, args...); break;
   }
 }
 
@@ -795,14 +836,14 @@ int reduce(quat* M, int n, int ld, int nb, double* d, quat* e, const ReduceWork&
         // algorithmic bytes: one read of the trailing lower triangle
         ProfScope ps(PROF_SYMV, s, 32.0 * 0.5 * (double)sz * (sz + 1));
         if (spg == 4)
-          launch_k(k_symv<256, 16>, dim3(nmain), dim3(256), 0, s, M, ld, n, p, c, j, w.W, ldw, w.part, nparts,
-                   w.scal, d, e, w.Prow, w.Pcol, n, w.TS, nb, w.TSP, w.ldtsp, w.QF, ZB{nullptr, 0});
+          launch_k(k_symv<256, 16, false>, dim3(nmain), dim3(256), 0, s, M, w.W, w.TSP, w.part, ld, n, p, c, j, ldw,
+                   nparts, w.ldtsp, w.scal, d, e, w.Prow, w.Pcol, n, nb, w.TS, w.QF, ZB{nullptr, 0});
         else
-          launch_k(k_symv<512, 32>, dim3(nmain), dim3(512), 0, s, M, ld, n, p, c, j, w.W, ldw, w.part, nparts,
-                   w.scal, d, e, w.Prow, w.Pcol, n, w.TS, nb, w.TSP, w.ldtsp, w.QF, ZB{nullptr, 0});
+          launch_k(k_symv<512, 32, false>, dim3(nmain), dim3(512), 0, s, M, w.W, w.TSP, w.part, ld, n, p, c, j, ldw,
+                   nparts, w.ldtsp, w.scal, d, e, w.Prow, w.Pcol, n, nb, w.TS, w.QF, ZB{nullptr, 0});
       }
-      launch_wcol(kpt, sz, dim3(std::max(1, cdiv(sz - 1, RQ))), s, M, ld, n, p, c, j, w.W, ldw, w.Prow, w.Pcol, n, w.TS,
-                  nb, w.scal, w.QF, w.part, w.TSP, w.ldtsp, d, w.tsm, ZB{nullptr, 0});
+      launch_wcol<false>(kpt, sz, dim3(std::max(1, cdiv(sz - 1, RQ))), s, M, w.W, w.Prow, w.pcs, ld, n, p, c, j, ldw,
+                         n, nb, w.TS, w.scal, w.QF, w.part, w.TSP, d, w.ldtsp, w.tsm, ZB{nullptr, 0});
     }
     // trailing update of rows/cols [p+wdt, n): M -= [V W] [W V]^*  (lower triangle)
     const int r0 = p + wdt;
@@ -898,20 +939,20 @@ int reduce_batched(int nprob, const int* nh, ZB zb, quat* M, int ld, int nb, dou
     };
     if (k1 > 0) {
       ProfScope ps(PROF_SYMV, s, tri_bytes(0, k1));
-      launch_k(k_symv<512, 32>, dim3(ntiles(cdiv(sz, SG), 2) + NF, 1, k1), dim3(512), 0, s, M, ld, L, p, c, j, w.W,
-               ldw, w.part, nparts, w.scal, d, e, w.Prow, w.Pcol, ld, w.TS, nb, w.TSP, w.ldtsp, w.QF, zb);
+      launch_k(k_symv<512, 32, true>, dim3(ntiles(cdiv(sz, SG), 2) + NF, 1, k1), dim3(512), 0, s, M, w.W, w.TSP,
+               w.part, ld, L, p, c, j, ldw, nparts, w.ldtsp, w.scal, d, e, w.Prow, w.Pcol, ld, nb, w.TS, w.QF, zb);
     }
     if (k1 < act) {
       const size_t sh = (size_t)k1 * zb.zs;
       const int szn = nh[k1] - c - 1;
       ProfScope ps(PROF_SYMV, s, tri_bytes(k1, act));
-      launch_k(k_symv<256, 16>, dim3(ntiles(cdiv(szn, SG), 4) + NF, 1, act - k1), dim3(256), 0, s, zshift(M, sh), ld,
-               L, p, c, j, zshift(w.W, sh), ldw, zshift(w.part, sh), nparts, zshift(w.scal, sh), zshift(d, sh),
-               zshift(e, sh), zshift(w.Prow, sh), zshift(w.Pcol, sh), ld, zshift(w.TS, sh), nb, zshift(w.TSP, sh),
-               w.ldtsp, zshift(w.QF, sh), ZB{zb.nvec + k1, zb.zs});
+      launch_k(k_symv<256, 16, true>, dim3(ntiles(cdiv(szn, SG), 4) + NF, 1, act - k1), dim3(256), 0, s, zshift(M,
+               sh), zshift(w.W, sh), zshift(w.TSP, sh), zshift(w.part, sh), ld, L, p, c, j, ldw, nparts, w.ldtsp,
+               zshift(w.scal, sh), zshift(d, sh), zshift(e, sh), zshift(w.Prow, sh), zshift(w.Pcol, sh), ld, nb,
+               zshift(w.TS, sh), zshift(w.QF, sh), ZB{zb.nvec + k1, zb.zs});
     }
-    launch_wcol(kpt, sz, dim3(std::max(1, cdiv(sz - 1, RQ)), 1, act), s, M, ld, L, p, c, j, w.W, ldw, w.Prow, w.Pcol,
-                ld, w.TS, nb, w.scal, w.QF, w.part, w.TSP, w.ldtsp, d, w.tsm, zb);
+    launch_wcol<true>(kpt, sz, dim3(std::max(1, cdiv(sz - 1, RQ)), 1, act), s, M, w.W, w.Prow, w.pcs, ld, L, p, c, j,
+                      ldw, ld, nb, w.TS, w.scal, w.QF, w.part, w.TSP, d, w.ldtsp, w.tsm, zb);
     if (j == nb - 1 || c == cend - 1) {
       const int P = c / nb;
       const int cnt = toff[P + 1] - toff[P];

@@ -313,7 +313,8 @@ __device__ __forceinline__ T* zoff(T* p, const ZB& zb) {
 struct ReduceWork {
   quat* W;        // n x nb (global row index)
   quat* Prow;     // matvec row partials: ceil(n/32) x n
-  quat* Pcol;     // matvec column partials: ceil(n/64) x n
+  quat* Pcol;     // matvec column partials: ceil(n/64) x n, right after Prow's
+  int pcs;        // Pcol = Prow + pcs n
   quat* TS;       // tall-skinny products [W^* u | V^* u]: 2 x nb
   double* TSP;    // their per-block partials: ceil(n/16) x ldtsp
   int ldtsp;      // 8 nb
