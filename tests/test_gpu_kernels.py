@@ -134,6 +134,46 @@ def test_qgemm_tile_rows_change_no_result(gpu_ctx, m, n, k, ta, tb, lower):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 33, 16), (15, 31, 15), (16, 32, 16), (17, 33, 17), (33, 65, 31), (48, 64, 33),
+                                   (160, 320, 1), (1000, 31, 48), (511, 511, 32)])
+@pytest.mark.parametrize("ta,tb,lower", [("N", "N", False), ("C", "N", False), ("N", "C", True)])
+def test_qgemm_small_tiles(gpu_ctx, m, n, k, ta, tb, lower):
+    """Products of fewer than two 32 x 64 tiles per CU (16 x 32 tiles, K in
+    stages of 16), at the edges of tiles and stages.  Each real component of
+    C sums 4 k products of magnitude <= 1 in FMAs, then C itself: rounding at
+    most (4 k + 2) eps (4 k + 1) with inputs in (-1, 1); 4x less is asserted
+    (errors of random sign)."""
+    import torch
+    if lower:
+        n = m
+    _say(f"case: qgemm small tiles m={m} n={n} k={k} {ta}{tb} lower={lower}")
+    rng = np.random.default_rng(m + 31 * n + 7 * k)
+
+    def rand(r, c):
+        return tuple(rng.uniform(-1, 1, (r, c)) + 1j * rng.uniform(-1, 1, (r, c)) for _ in range(2))
+
+    A = rand(*((k, m) if ta == "C" else (m, k)))
+    B = rand(*((n, k) if tb == "C" else (k, n)))
+    C = rand(m, n)
+    lda, ldb, ldc = A[0].shape[0] + 1, B[0].shape[0], m + 3
+    dA = torch.from_numpy(_pack(*A, lda)).cuda()
+    dB = torch.from_numpy(_pack(*B, ldb)).cuda()
+    dC = torch.from_numpy(_pack(*C, ldc)).cuda()
+    before = dC.clone()
+    torch.cuda.synchronize()
+    assert gpu_ctx.qgemm_device(ta, tb, m, n, k, -1.0, dA.data_ptr(), lda, dB.data_ptr(), ldb, 1.0, dC.data_ptr(), ldc,
+                                lower) == 0
+    gpu_ctx.synchronize()
+    ref = _unembed(_embed(*C) - _embed(*(_ct(*A) if ta == "C" else A)) @ _embed(*(_ct(*B) if tb == "C" else B)), m, n)
+    mask = np.tril(np.ones((m, n), dtype=bool)) if lower else np.ones((m, n), dtype=bool)
+    bound = (4 * k + 2) * (4 * k + 1) * np.finfo(float).eps / 4
+    for g, r in zip(_unpack(dC.cpu().numpy(), m, n), ref):
+        assert np.abs(g - r)[mask].max() <= max(bound, 1e-14)
+    for g, o in zip(_unpack(dC.cpu().numpy(), m, n), _unpack(before.cpu().numpy(), m, n)):
+        assert np.array_equal(g[~mask], o[~mask])
+    assert torch.equal(dC[:, m:, :], before[:, m:, :])
+
+
 def test_qgemm_argument_errors(gpu_ctx):
     assert gpu_ctx.qgemm_device("X", "N", 2, 2, 2, 1.0, 0, 2, 0, 2, 0.0, 0, 2) == -2
     assert gpu_ctx.qgemm_device("N", "N", -1, 2, 2, 1.0, 0, 2, 0, 2, 0.0, 0, 2) == -4

@@ -24,29 +24,43 @@
 // (zquatev.cc:86-90).
 #include "zq_internal.h"
 #include <climits>
-#include <cstdlib>
 
 namespace zq {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------
-// Tiles of TBM x 64 quaternions per workgroup, TBM = 64 or 32 (2 x 2 waves,
-// TBM/2 x 32 quaternions = TBM/4 MFMA accumulators per wave; the smaller tile
-// doubles the workgroups of products too small to fill the device), K staged 8 quaternions at a
-// time through double-buffered LDS.  The next stage's operands are fetched
-// into registers before the current stage's MFMAs, so global latency hides
-// behind the wave's own work, and one barrier per stage suffices (a buffer is
-// rewritten only after the barrier that follows its last read).  The
-// conjugate-transpose flags are template parameters (branch-free address
+// Tiles of TBM x TBN quaternions per workgroup (2 x 2 waves), K staged GBK
+// quaternions at a time through double-buffered LDS.  The next stage's operands
+// are fetched into registers before the current stage's MFMAs, so global
+// latency hides behind the wave's own work, and one barrier per stage suffices
+// (a buffer is rewritten only after the barrier that follows its last read).
+// The conjugate-transpose flags are template parameters (branch-free address
 // math); the sign of the L(A) expansion is applied by flipping the sign bit.
+// The tile shape changes no result: an element's K-sum is one wave's
+// accumulator in the same order in every shape.
+//   64 x 64, GBK 8    the most reuse per fetch, for launches of very many tiles;
+//   32 x 64, GBK 8    twice the workgroups (balance, registers);
+//   16 x 32, GBK 16   for launches that leave CUs idle otherwise: a wave's time
+//                     is K x (its 16 x 16 x 4 products) x 64 cycles whatever
+//                     the other CUs do -- 14 us for 32 x 64 at K = 64, a
+//                     quarter of that here -- and its shorter stages (1024
+//                     cycles at GBK 8) would wait for the next fetch, hence 16.
+//                     C is fetched before the K loop.
 // ---------------------------------------------------------------------------
-constexpr int GBN = 64, GBK = 8;
-// LDS layouts (doubles).  A: [k][row][component], B: [k][component][column],
-// each k slice padded by 2 doubles, so that fragment reads (16 consecutive
-// doubles per component group) and the stage writes of either operand
-// orientation (8 consecutive k per 8 threads) fall in distinct banks.
-constexpr int BSK = GBN * 4 + 2;   // B k-slice stride
+template <int TBM_, int TBN_, int GBK_>
+struct QTile {
+  static constexpr int TBM = TBM_, TBN = TBN_, GBK = GBK_;
+  // LDS layouts (doubles).  A: [k][row][component], B: [k][component][column],
+  // each k slice padded by 2 doubles, so that fragment reads (16 consecutive
+  // doubles per component group) and the stage writes of either operand
+  // orientation fall in distinct banks.
+  static constexpr int ASK = TBM * 4 + 2, BSK = TBN * 4 + 2;
+  static constexpr bool PREC = TBM == 16;   // C fetched before the K loop
+};
+using Tile64 = QTile<64, 64, 8>;
+using Tile32 = QTile<32, 64, 8>;
+using Tile16 = QTile<16, 32, 16>;
 
 // Operand elements as stored.  The conjugation of a CT operand is applied
 // when the stage is stashed in LDS, after the current stage's MFMAs: sign
@@ -78,36 +92,39 @@ __device__ __forceinline__ double flip_sign(double v, unsigned mask) {
   return mkd(lo32(v), hi32(v) ^ mask);
 }
 
-template <int TBM, bool ACT, bool BCT>
+template <class T, bool ACT, bool BCT>
 __device__ __forceinline__ void qgemm2_tile(const QGemmTask& t, int row0, int col0, int kbeg, int kend, quat* C) {
-  constexpr int AH = TBM / 32;          // A stage elements per thread
-  constexpr int AK = TBM * 4 + 2;       // A k-slice stride (doubles)
-  constexpr int WR = TBM / 2;           // quaternion rows per wave
-  constexpr int NA = WR / 4;            // 4-row MFMA tiles per wave
+  constexpr int TBM = T::TBM, TBN = T::TBN, GBK = T::GBK;
+  constexpr int AH = TBM * GBK / 256;   // A stage elements per thread
+  constexpr int BH = TBN * GBK / 256;   // B stage elements per thread
+  constexpr int WR = TBM / 2, WC = TBN / 2;   // quaternion rows and columns per wave
+  constexpr int NA = WR / 4, NBC = WC / 16;   // MFMA accumulators per wave: NA x NBC
+  static_assert(AH * 256 == TBM * GBK && BH * 256 == TBN * GBK && NA * 4 == WR && NBC * 16 == WC, "tile shape");
   const int m = t.m, nn = t.nn, K = t.K;
-  __shared__ double As[2][GBK * AK];
-  __shared__ double Bs[2][GBK * BSK];
+  __shared__ double As[2][GBK * T::ASK];
+  __shared__ double Bs[2][GBK * T::BSK];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
-  const int wr = wv >> 1, wc = wv & 1;   // wave tile: rows wr*WR..+WR, cols wc*32..+32 (quaternions)
+  const int wr = wv >> 1, wc = wv & 1;   // wave tile: rows wr*WR..+WR, cols wc*WC..+WC (quaternions)
   const int cr = (lane & 15) >> 2, ck = lane >> 4;
   const int acomp = cr ^ ck;
   const unsigned smask = ((0x428E >> (cr * 4 + ck)) & 1) ? 0x80000000u : 0u;
   const int aq = lane & 3;
   const int bkc = lane >> 4, bj = lane & 15;
-  // this thread's A and B stage elements
-  int ai[AH], ak[AH], bk[2], bjj[2];
+  // this thread's A and B stage elements: consecutive threads along the
+  // storage's contiguous direction
+  int ai[AH], ak[AH], bk[BH], bjj[BH];
 #pragma unroll
   for (int h = 0; h < AH; ++h) {
     if (!ACT) { ai[h] = tid % TBM; ak[h] = tid / TBM + (256 / TBM) * h; }
-    else { ak[h] = tid & 7; ai[h] = (tid >> 3) + 32 * h; }
+    else { ak[h] = tid % GBK; ai[h] = tid / GBK + (256 / GBK) * h; }
   }
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    if (!BCT) { bk[h] = tid & 7; bjj[h] = (tid >> 3) + 32 * h; }
-    else { bjj[h] = tid & 63; bk[h] = (tid >> 6) + 4 * h; }
+  for (int h = 0; h < BH; ++h) {
+    if (!BCT) { bk[h] = tid % GBK; bjj[h] = tid / GBK + (256 / GBK) * h; }
+    else { bjj[h] = tid % TBN; bk[h] = tid / TBN + (256 / TBN) * h; }
   }
-  quat ra[AH], rb[2];
+  quat ra[AH], rb[BH];
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int h = 0; h < AH; ++h) {
@@ -115,7 +132,7 @@ __device__ __forceinline__ void qgemm2_tile(const QGemmTask& t, int row0, int co
       ra[h] = (ka < kend) ? ld_opA<ACT>(t.A, row0 + ai[h], ka, m, K) : qzero();
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < BH; ++h) {
       const int kb = k0 + bk[h];
       rb[h] = (kb < kend) ? ld_opB<BCT>(t.B, kb, col0 + bjj[h], K, nn) : qzero();
     }
@@ -124,25 +141,42 @@ __device__ __forceinline__ void qgemm2_tile(const QGemmTask& t, int row0, int co
 #pragma unroll
     for (int h = 0; h < AH; ++h) {
       const quat a = ACT ? qconj(ra[h]) : ra[h];
-      double2* pa = reinterpret_cast<double2*>(&As[buf][ak[h] * AK + ai[h] * 4]);
+      double2* pa = reinterpret_cast<double2*>(&As[buf][ak[h] * T::ASK + ai[h] * 4]);
       pa[0] = make_double2(a.ar, a.ai);
       pa[1] = make_double2(a.br, a.bi);
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < BH; ++h) {
       const quat bv = BCT ? qconj(rb[h]) : rb[h];
-      double* pb = &Bs[buf][bk[h] * BSK + bjj[h]];
+      double* pb = &Bs[buf][bk[h] * T::BSK + bjj[h]];
       pb[0] = bv.ar;
-      pb[GBN] = bv.ai;
-      pb[2 * GBN] = bv.br;
-      pb[3 * GBN] = bv.bi;
+      pb[TBN] = bv.ai;
+      pb[2 * TBN] = bv.br;
+      pb[3 * TBN] = bv.bi;
     }
   };
-  d4 acc[NA][2];
+  // lane holds quaternion (row wr*WR + 4a + lane/16, col wc*WC + 16b + lane%16) of C
+  const double alpha = t.alpha, beta = t.beta;
+  const int ci = row0 + wr * WR + (lane >> 4), cj = col0 + wc * WC + (lane & 15);
+  auto written = [&](int a, int b) {
+    const int i = ci + 4 * a, jj = cj + 16 * b;
+    return i < m && jj < nn && (!t.lower_only || i >= jj);
+  };
+  quat cold[T::PREC ? NA : 1][T::PREC ? NBC : 1];
+  if constexpr (T::PREC) {
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+      for (int b = 0; b < NBC; ++b) {
+        cold[a][b] = qzero();
+        if (beta != 0.0 && written(a, b)) cold[a][b] = qload_g(C + (ci + 4 * a) + (size_t)(cj + 16 * b) * t.ldc);
+      }
+  }
+  d4 acc[NA][NBC];
 #pragma unroll
   for (int a = 0; a < NA; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int b = 0; b < NBC; ++b) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
   int cur = 0;
   if (kbeg < kend) {
     fetch(kbeg);
@@ -154,32 +188,29 @@ __device__ __forceinline__ void qgemm2_tile(const QGemmTask& t, int row0, int co
     if (more) fetch(k0 + GBK);
 #pragma unroll
     for (int kk = 0; kk < GBK; ++kk) {
-      double af[NA], bf[2];
+      double af[NA], bf[NBC];
 #pragma unroll
-      for (int a = 0; a < NA; ++a) af[a] = flip_sign(As[cur][kk * AK + (wr * WR + 4 * a + aq) * 4 + acomp], smask);
+      for (int a = 0; a < NA; ++a) af[a] = flip_sign(As[cur][kk * T::ASK + (wr * WR + 4 * a + aq) * 4 + acomp], smask);
 #pragma unroll
-      for (int b = 0; b < 2; ++b) bf[b] = Bs[cur][kk * BSK + bkc * GBN + wc * 32 + 16 * b + bj];
+      for (int b = 0; b < NBC; ++b) bf[b] = Bs[cur][kk * T::BSK + bkc * TBN + wc * WC + 16 * b + bj];
 #pragma unroll
       for (int a = 0; a < NA; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[a], bf[b], acc[a][b], 0, 0, 0);
+        for (int b = 0; b < NBC; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[a], bf[b], acc[a][b], 0, 0, 0);
     }
     if (more) stash(cur ^ 1);
     __syncthreads();
     cur ^= 1;
   }
-  // epilogue: lane holds quaternion (row wr*WR + 4a + lane/16, col wc*32 + 16b + lane%16)
-  const double alpha = t.alpha, beta = t.beta;
 #pragma unroll
   for (int a = 0; a < NA; ++a) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int i = row0 + wr * WR + 4 * a + (lane >> 4);
-      const int jj = col0 + wc * 32 + 16 * b + (lane & 15);
-      if (i < m && jj < nn && (!t.lower_only || i >= jj)) {
-        quat* cp = C + i + (size_t)jj * t.ldc;
+    for (int b = 0; b < NBC; ++b) {
+      if (written(a, b)) {
+        quat* cp = C + (ci + 4 * a) + (size_t)(cj + 16 * b) * t.ldc;
         quat r = quat{alpha * acc[a][b][0], alpha * acc[a][b][1], alpha * acc[a][b][2], alpha * acc[a][b][3]};
-        if (beta != 0.0) r = qadd(r, qscale(qload_g(cp), beta));
+        if (beta != 0.0) r = qaxpy(r, beta, T::PREC ? cold[T::PREC ? a : 0][T::PREC ? b : 0] : qload_g(cp));
         qstore_g(cp, r);
       }
     }
@@ -196,43 +227,44 @@ __device__ __forceinline__ int xcd_remap(int t, int T) {
 }
 
 // Lower-triangle products enumerate only the tiles that meet the lower
-// triangle: column block y (64 wide) has row tiles x >= (64 y) / TBM.
-__host__ __device__ inline int lower_tiles(int m, int tbm) {
-  const int gx = (m + tbm - 1) / tbm, gy = (m + 63) / 64;
-  int cnt = 0;
-  for (int y = 0; y < gy; ++y) cnt += gx - (64 * y) / tbm;
-  return cnt;
+// triangle: column block y (TBN wide) has row tiles x >= y TBN / TBM, so the
+// blocks before it hold y gx - (TBN / TBM) y (y - 1) / 2 tiles.
+template <class T>
+__host__ __device__ inline int tiles_before(int y, int gx) {
+  static_assert(T::TBN % T::TBM == 0, "lower-triangle tile enumeration");
+  return y * gx - T::TBN / T::TBM * (y * (y - 1) / 2);
+}
+template <class T>
+__host__ __device__ inline int tile_count(int m, int nn, bool lower) {
+  const int gx = (m + T::TBM - 1) / T::TBM, gy = (nn + T::TBN - 1) / T::TBN;
+  return lower ? tiles_before<T>((m + T::TBN - 1) / T::TBN, gx) : gx * gy;
 }
 
-template <int TBM>
-__device__ __forceinline__ bool tile_of(const QGemmTask& t, int u, int gx_rect, int& tx, int& ty) {
+template <class T>
+__device__ __forceinline__ void tile_of(const QGemmTask& t, int u, int& tx, int& ty) {
+  const int gx = (t.m + T::TBM - 1) / T::TBM;
   if (!t.lower_only) {
-    tx = u % gx_rect;
-    ty = u / gx_rect;
-    return true;
+    ty = u / gx;
+    tx = u - ty * gx;
+    return;
   }
-  const int gx = (t.m + TBM - 1) / TBM, gy = (t.nn + 63) / 64;
-  int acc = 0;
-  for (int y = 0; y < gy; ++y) {
-    const int x0 = (64 * y) / TBM;
-    const int cnt = gx - x0;
-    if (u < acc + cnt) {
-      tx = x0 + (u - acc);
-      ty = y;
-      return true;
-    }
-    acc += cnt;
-  }
-  return false;
+  // the largest y with tiles_before(y) <= u: the root of the quadratic, then exact
+  constexpr int rho = T::TBN / T::TBM;
+  const float bq = 2.0f * (float)gx / rho + 1.0f;
+  int y = (int)(0.5f * (bq - sqrtf(fmaxf(bq * bq - 8.0f / rho * (float)u, 0.0f))));
+  const int gy = (t.m + T::TBN - 1) / T::TBN;
+  y = max(0, min(y, gy - 1));
+  while (y + 1 < gy && tiles_before<T>(y + 1, gx) <= u) ++y;
+  while (y > 0 && tiles_before<T>(y, gx) > u) --y;
+  ty = y;
+  tx = rho * y + (u - tiles_before<T>(y, gx));
 }
 
-// grid: x = tiles (rectangular: gx * gy of them, gx given; lower: lower_tiles), z = K chunks
-template <int TBM, bool ACT, bool BCT>
-__global__ void __launch_bounds__(256, 2) k_qgemm2(QGemmTask t, int kchunk, size_t cstride, int gx) {
+// grid: x = tiles, z = K chunks
+template <class T, bool ACT, bool BCT>
+__global__ void __launch_bounds__(256, 2) k_qgemm2(QGemmTask t, int kchunk, size_t cstride) {
   int tx, ty;
-  if (!tile_of<TBM>(t, xcd_remap(blockIdx.x, gridDim.x), gx, tx, ty)) return;
-  const int row0 = tx * TBM;
-  const int col0 = ty * GBN;
+  tile_of<T>(t, xcd_remap(blockIdx.x, gridDim.x), tx, ty);
   int kbeg = t.kbeg, kend = t.kend;
   quat* C = t.C;
   if (gridDim.z > 1) {
@@ -240,23 +272,18 @@ __global__ void __launch_bounds__(256, 2) k_qgemm2(QGemmTask t, int kchunk, size
     kend = min(t.kend, kbeg + kchunk);
     C += (size_t)blockIdx.z * cstride;
   }
-  qgemm2_tile<TBM, ACT, BCT>(t, row0, col0, kbeg, kend, C);
+  qgemm2_tile<T, ACT, BCT>(t, tx * T::TBM, ty * T::TBN, kbeg, kend, C);
 }
 
 // grid: x = tiles of the largest task, z = tasks
-template <int TBM, bool ACT, bool BCT>
+template <class T, bool ACT, bool BCT>
 __global__ void __launch_bounds__(256, 2) k_qgemm2_batch(const QGemmTask* __restrict__ tasks) {
   const QGemmTask t = tasks[blockIdx.z];
-  // tiles of this task: the launch covers the largest task's; gx from the task
-  const int gx = (t.m + TBM - 1) / TBM;
-  const int ntile = t.lower_only ? lower_tiles(t.m, TBM) : gx * ((t.nn + GBN - 1) / GBN);
   const int u = xcd_remap(blockIdx.x, gridDim.x);
-  if (u >= ntile) return;
+  if (u >= tile_count<T>(t.m, t.nn, t.lower_only)) return;
   int tx, ty;
-  if (!tile_of<TBM>(t, u, gx, tx, ty)) return;
-  const int row0 = tx * TBM;
-  const int col0 = ty * GBN;
-  qgemm2_tile<TBM, ACT, BCT>(t, row0, col0, t.kbeg, t.kend, t.C);
+  tile_of<T>(t, u, tx, ty);
+  qgemm2_tile<T, ACT, BCT>(t, tx * T::TBM, ty * T::TBN, t.kbeg, t.kend, t.C);
 }
 
 // Tile rows: 64 only for launches with at least 16 64 x 64 tiles per compute
@@ -279,32 +306,43 @@ static int device_cus() {
 
 thread_local int g_tile64_per_cu = 16;
 
-static int tile_rows(long tiles64) { return tiles64 >= (long)g_tile64_per_cu * device_cus() ? 64 : 32; }
+// 16 x 32 tiles for launches of fewer than SMALL_PER_CU 32 x 64 tiles per
+// compute unit.  Against 32 x 64 tiles throughout (2n = 510, 1024, 2048, 4096
+// solves 2.55, 5.13, 11.25, 33.8 ms): below 1 tile per unit 2.31, 4.66, 10.83,
+// 33.4 ms, below 2 2.30, 4.65, 10.78, 33.2 ms, below 4 2.30, 4.65, 10.82, 33.8
+// ms, below 8 the 2n = 8192 solve too is slower (149.0 -> 151.9 ms): more
+// operand traffic per product once every CU is busy.
+constexpr int SMALL_PER_CU = 2;
+static int tile_rows(long tiles64, long tiles32) {
+  if (tiles32 < (long)SMALL_PER_CU * device_cus()) return 16;
+  return tiles64 >= (long)g_tile64_per_cu * device_cus() ? 64 : 32;
+}
 
-template <int TBM>
+template <class T>
 static void launch_gemm2_t(bool act, bool bct, hipStream_t s, const QGemmTask& t, int nz, int kchunk,
                            size_t cstride) {
-  const int gx = (t.m + TBM - 1) / TBM;
-  const int nt = t.lower_only ? lower_tiles(t.m, TBM) : gx * ((t.nn + GBN - 1) / GBN);
-  const dim3 grid(nt, 1, nz);
-  if (!act && !bct) launch_k(k_qgemm2<TBM, false, false>, grid, dim3(256), 0, s, t, kchunk, cstride, gx);
-  else if (act && !bct) launch_k(k_qgemm2<TBM, true, false>, grid, dim3(256), 0, s, t, kchunk, cstride, gx);
-  else if (!act && bct) launch_k(k_qgemm2<TBM, false, true>, grid, dim3(256), 0, s, t, kchunk, cstride, gx);
-  else launch_k(k_qgemm2<TBM, true, true>, grid, dim3(256), 0, s, t, kchunk, cstride, gx);
+  const dim3 grid(tile_count<T>(t.m, t.nn, t.lower_only), 1, nz);
+  if (!act && !bct) launch_k(k_qgemm2<T, false, false>, grid, dim3(256), 0, s, t, kchunk, cstride);
+  else if (act && !bct) launch_k(k_qgemm2<T, true, false>, grid, dim3(256), 0, s, t, kchunk, cstride);
+  else if (!act && bct) launch_k(k_qgemm2<T, false, true>, grid, dim3(256), 0, s, t, kchunk, cstride);
+  else launch_k(k_qgemm2<T, true, true>, grid, dim3(256), 0, s, t, kchunk, cstride);
 }
 
 static void launch_gemm2(bool act, bool bct, hipStream_t s, const QGemmTask& t, int nz, int kchunk, size_t cstride) {
-  const long t64 = (long)(t.lower_only ? lower_tiles(t.m, 64) : ((t.m + 63) / 64) * ((t.nn + GBN - 1) / GBN)) * nz;
-  if (tile_rows(t64) == 64) launch_gemm2_t<64>(act, bct, s, t, nz, kchunk, cstride);
-  else launch_gemm2_t<32>(act, bct, s, t, nz, kchunk, cstride);
+  const bool low = t.lower_only;
+  switch (tile_rows((long)tile_count<Tile64>(t.m, t.nn, low) * nz, (long)tile_count<Tile32>(t.m, t.nn, low) * nz)) {
+    case 64: launch_gemm2_t<Tile64>(act, bct, s, t, nz, kchunk, cstride); break;
+    case 32: launch_gemm2_t<Tile32>(act, bct, s, t, nz, kchunk, cstride); break;
+    default: launch_gemm2_t<Tile16>(act, bct, s, t, nz, kchunk, cstride); break;
+  }
 }
 
-template <int TBM>
+template <class T>
 static void launch_gemm2_batch_t(bool act, bool bct, dim3 grid, hipStream_t s, const QGemmTask* tasks) {
-  if (!act && !bct) launch_k(k_qgemm2_batch<TBM, false, false>, grid, dim3(256), 0, s, tasks);
-  else if (act && !bct) launch_k(k_qgemm2_batch<TBM, true, false>, grid, dim3(256), 0, s, tasks);
-  else if (!act && bct) launch_k(k_qgemm2_batch<TBM, false, true>, grid, dim3(256), 0, s, tasks);
-  else launch_k(k_qgemm2_batch<TBM, true, true>, grid, dim3(256), 0, s, tasks);
+  if (!act && !bct) launch_k(k_qgemm2_batch<T, false, false>, grid, dim3(256), 0, s, tasks);
+  else if (act && !bct) launch_k(k_qgemm2_batch<T, true, false>, grid, dim3(256), 0, s, tasks);
+  else if (!act && bct) launch_k(k_qgemm2_batch<T, false, true>, grid, dim3(256), 0, s, tasks);
+  else launch_k(k_qgemm2_batch<T, true, true>, grid, dim3(256), 0, s, tasks);
 }
 
 int qgemm(int m, int nn, int k, double alpha, const QOperand& A, const QOperand& B, double beta, quat* C, int ldc,
@@ -318,21 +356,22 @@ int qgemm(int m, int nn, int k, double alpha, const QOperand& A, const QOperand&
 int qgemm_tasks(const QGemmTask* tasks_dev, int ntasks, int maxm, int maxnn, bool act, bool bct, bool lower,
                 hipStream_t s) {
   if (ntasks <= 0 || maxm <= 0 || maxnn <= 0) return ZQI_OK;
-  auto ntiles = [&](int tbm) {
-    return lower ? lower_tiles(maxm, tbm) : ((maxm + tbm - 1) / tbm) * ((maxnn + GBN - 1) / GBN);
-  };
-  if (tile_rows((long)ntiles(64) * ntasks) == 64)
-    launch_gemm2_batch_t<64>(act, bct, dim3(ntiles(64), 1, ntasks), s, tasks_dev);
-  else
-    launch_gemm2_batch_t<32>(act, bct, dim3(ntiles(32), 1, ntasks), s, tasks_dev);
+  const int n64 = tile_count<Tile64>(maxm, maxnn, lower), n32 = tile_count<Tile32>(maxm, maxnn, lower);
+  switch (tile_rows((long)n64 * ntasks, (long)n32 * ntasks)) {
+    case 64: launch_gemm2_batch_t<Tile64>(act, bct, dim3(n64, 1, ntasks), s, tasks_dev); break;
+    case 32: launch_gemm2_batch_t<Tile32>(act, bct, dim3(n32, 1, ntasks), s, tasks_dev); break;
+    default:
+      launch_gemm2_batch_t<Tile16>(act, bct, dim3(tile_count<Tile16>(maxm, maxnn, lower), 1, ntasks), s, tasks_dev);
+  }
   return hipGetLastError() == hipSuccess ? ZQI_OK : ZQI_ERR_HIP;
 }
 
+constexpr int KCHUNK = 8;   // split-K chunks are multiples of this
 int splitk_count(int K, int nsplit, int* kchunk_out) {
   if (nsplit < 1) nsplit = 1;
   int kchunk = (K + nsplit - 1) / nsplit;
-  kchunk = ((kchunk + GBK - 1) / GBK) * GBK;
-  if (kchunk < GBK) kchunk = GBK;
+  kchunk = ((kchunk + KCHUNK - 1) / KCHUNK) * KCHUNK;
+  if (kchunk < KCHUNK) kchunk = KCHUNK;
   if (kchunk_out) *kchunk_out = kchunk;
   const int nz = (K + kchunk - 1) / kchunk;
   return nz > 0 ? nz : 1;

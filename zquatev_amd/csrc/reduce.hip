@@ -482,11 +482,13 @@ __device__ __forceinline__ void row_tsp(const quat* vv, const quat* ww, const qu
 // At trailing sizes below ~1500 a block's time is one round trip to memory
 // plus the instructions of one wave per SIMD, so both the barriers and the
 // instruction count are its cost: two barriers instead of four, the eleven
-// block sums by one halving butterfly instead of a full sum each, the sums in
-// scalar registers (1300 -> 1000 instructions, 9.8 -> 9.0 us per column with
-// its matvec at panel width 16; 2n = 1024 reduction 4.74 -> 4.37 ms, 2n = 8192
-// 111.0 -> 107.8 ms).  Fusing it into the next column's matvec (one launch per
-// column, every tile block repeating the row work of its 96 rows) took 11-12 us
+// block sums by halving butterflies, each wave only those whose terms it holds,
+// the sums in scalar registers, the row partials padded to distinct LDS banks,
+// unconditional loads at clamped addresses, the batch addressing compiled out
+// of single solves.  Per column with its matvec at panel width 16: 9.8 us ->
+// 8.2 us; 2n = 1024 reduction 4.74 -> 4.07 ms, 2n = 8192 111.0 -> 104.3 ms.
+// Fusing it into the next column's matvec (one launch per column, every tile
+// block repeating the row work of its 96 rows) took 11-12 us
 // per column: twice the instructions on every wave.
 // PY, PQ: partial loads per thread per gather batch (quaternion row partials,
 // x^* M x partials); WPE: the waves per SIMD the register budget aims at.
