@@ -17,7 +17,7 @@
  *
  * Return codes: 0 success; -i argument i is invalid (LAPACK style); > 0 the
  * tridiagonal eigensolver did not converge (as zhbev's info at zquatev.cc:84,
- * :99: a leaf QL iteration, a secular-equation root or an eigenvalue bracket
+ * :99: a leaf's Jacobi iteration, a secular-equation root or an eigenvalue bracket
  * that did not converge; the value is 1 + a local row or root index);
  * ZQ_ERR_* below for runtime errors and for a non-finite input.
  */
@@ -303,8 +303,8 @@ int zq_synchronize(zq_context* ctx);
  * batch, the aggregate its batched call returns. */
 int zq_last_info(zq_context* ctx);
 
-/* Iteration caps of the tridiagonal eigensolver on ctx (0 = default): QL
- * sweeps per eigenvalue of a divide & conquer leaf (60), safeguarded Newton
+/* Iteration caps of the tridiagonal eigensolver on ctx (0 = default):
+ * Jacobi sweeps per divide & conquer leaf (60), safeguarded Newton
  * steps per secular-equation root (200), multisection steps per eigenvalue
  * of the eigenvalues-only path (64).  A cap reached is reported as
  * non-convergence (info > 0), as zhbev reports a QL failure (zquatev.cc:84).

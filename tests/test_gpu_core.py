@@ -119,6 +119,43 @@ def test_tridiag_eig(gpu_ctx, n, kind):
     assert np.abs(dw2.cpu().numpy() - ref).max() <= 1e-13 * tn * max(1, np.sqrt(n))
 
 
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 6, 8, 9, 13, 16, 17, 31, 32, 33, 47, 63, 64])
+@pytest.mark.parametrize("kind", ["rand", "clust", "split", "mirror", "glued", "graded"])
+def test_tridiag_eig_one_block(gpu_ctx, n, kind):
+    """Orders solved by one workgroup, at every depth of its tree.  Each of its
+    up to 4 merge levels deflates at 8 unit roundoffs and multiplies
+    orthogonal matrices of order <= n, and a leaf's Jacobi adds its own few
+    roundoffs: within 8 eps (4 + n) of the norm, with eps twice the roundoff."""
+    import torch
+    _say(f"case: tridiag_eig one block n={n} kind={kind}")
+    rng = np.random.default_rng(100 * n + len(kind))
+    d, e = rng.normal(size=n), np.abs(rng.normal(size=n - 1))
+    if kind == "clust":
+        d, e = 1.0 + 1e-13 * d, 1e-11 * e
+    elif kind == "split":
+        e[:: 3] = 0.0
+    elif kind == "mirror":
+        d, e = np.r_[d[: (n + 1) // 2], d[: n // 2][::-1]], np.r_[e[: n // 2], e[: (n - 1) // 2][::-1]]
+    elif kind == "glued":
+        d, e = np.abs(np.arange(n) % 5 - 2.0), np.where(np.arange(n - 1) % 5 == 4, 1e-9, 1.0)
+    elif kind == "graded":
+        d, e = d * 10.0 ** -np.arange(n, dtype=float), e * 10.0 ** -np.arange(n - 1, dtype=float)
+    dd, de = torch.from_numpy(d.copy()).cuda(), torch.from_numpy(np.r_[e, 0.0]).cuda()
+    dw = torch.zeros(n, dtype=torch.float64, device="cuda")
+    dz = torch.zeros(n * n, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    assert gpu_ctx.tridiag_eig_device(n, dd.data_ptr(), de.data_ptr(), dw.data_ptr(), dz.data_ptr()) == 0
+    assert gpu_ctx.last_info() == 0
+    w, Z = dw.cpu().numpy(), dz.cpu().numpy().reshape(n, n).T
+    T = np.diag(d) + np.diag(e, 1) + np.diag(e, -1)
+    tol = 8 * np.finfo(float).eps * (4 + n)
+    tn = np.linalg.norm(T, 2)
+    assert np.all(np.diff(w) >= 0)
+    assert np.abs(w - np.linalg.eigvalsh(T)).max() <= tol * tn
+    assert np.abs(T @ Z - Z * w[None, :]).max() <= tol * tn
+    assert np.abs(Z.T @ Z - np.eye(n)).max() <= tol
+
+
 @pytest.mark.parametrize("n2", [2, 4, 6, 8, 16, 22, 42, 44, 64, 128, 130, 400, 510, 512])
 def test_zquatev_host(gpu_ctx, n2):
     _say(f"case: zquatev host 2n={n2}")

@@ -8,10 +8,11 @@
 // the real tridiagonal (d, |e|) and returns the eigenvalues ascending, as
 // zhbev does, with an orthonormal real eigenvector matrix.
 //
-// Tree: halve until a block has at most LEAF rows; each split point s couples
+// Tree: halve until a block has at most BASE rows; each split point s couples
 // rows s-1 and s with beta = e[s-1] >= 0, and T = diag(T1', T2') + beta v v^T,
 // v = e_{s-1} + e_s, where T1', T2' have beta subtracted from the touching
-// diagonal entries.  Leaves run implicit QL in one wavefront each; merges run
+// diagonal entries.  A base block runs its whole divide & conquer (leaves of <=
+// 4 rows, then merges) in one workgroup (k_dc_base); the merges above run
 // level by level (all merges of a level in one launch):
 //   prep   : stable merge of the two sorted spectra, z = [last row of Q1;
 //            first row of Q2]/sqrt(2), rho = 2 beta, deflation scan (small
@@ -32,7 +33,7 @@
 
 namespace zq {
 
-constexpr int LEAF = 16;
+constexpr int BASE = 64;   // rows a workgroup solves by itself
 constexpr double DEPS = DBL_EPSILON * 0.5;   // unit roundoff
 
 static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -86,118 +87,6 @@ __global__ void k_dc_tear(int nsplit, const int* __restrict__ splits, const doub
   const double b = es[s - 1];
   lam[s - 1] -= b;
   lam[s] -= b;
-}
-
-// --------------------------------------------------------------------------
-// leaf: implicit QL with Wilkinson-type shift on a <= LEAF tridiagonal.  The
-// scalar recurrence runs identically in every lane; lane k owns row k of the
-// leaf's eigenvector block and applies each rotation to it.  A leaf is
-// (lo, hi, problem base, problem index).
-// --------------------------------------------------------------------------
-// Element i (wave-uniform) of a value held one per lane.
-__device__ __forceinline__ double lane_get(double v, int i) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), i);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), i);
-  return __hiloint2double(hi, lo);
-}
-
-// One leaf per wavefront.  The tridiagonal lives in registers, d[k] and e[k]
-// in lane k; every lane runs the (wave-uniform) QL recurrence redundantly,
-// reading element i with readlane, and the owning lane keeps an update, so
-// the sequential chain has no barrier and no LDS access.  Lane k owns row k
-// of the leaf's eigenvectors (in LDS), to which it applies each rotation.
-__global__ void __launch_bounds__(64) k_dc_leaf(const int* __restrict__ leaves, double* __restrict__ lam,
-                                                const double* __restrict__ es, double* __restrict__ Z, int ldz,
-                                                int* __restrict__ info, int cap) {
-  __shared__ double zz[LEAF][LEAF + 1];
-  const int lo = leaves[4 * blockIdx.x], hi = leaves[4 * blockIdx.x + 1];
-  const int ob = leaves[4 * blockIdx.x + 2], pr = leaves[4 * blockIdx.x + 3];
-  const int m = hi - lo;
-  const int k = threadIdx.x;
-  double dk = 0.0, ek = 0.0;
-  if (k < m) {
-    dk = lam[lo + k];
-    ek = (k < m - 1) ? es[lo + k] : 0.0;
-    for (int i = 0; i < m; ++i) zz[k][i] = (i == k) ? 1.0 : 0.0;
-  }
-  int fail = 0;
-  for (int l = 0; l < m; ++l) {
-    int iter = 0;
-    int mm;
-    while (true) {
-      for (mm = l; mm < m - 1; ++mm) {
-        const double s = fabs(lane_get(dk, mm)) + fabs(lane_get(dk, mm + 1));
-        if (fabs(lane_get(ek, mm)) <= DEPS * s) break;
-      }
-      if (mm == l) break;
-      if (++iter > cap) { fail = 1; break; }
-      const double el = lane_get(ek, l);
-      double g = (lane_get(dk, l + 1) - lane_get(dk, l)) / (2.0 * el);
-      double r = hypot(g, 1.0);
-      g = lane_get(dk, mm) - lane_get(dk, l) + el / (g + copysign(r, g));
-      double s = 1.0, c = 1.0, p = 0.0;
-      int i;
-      bool early = false;
-      for (i = mm - 1; i >= l; --i) {
-        const double ei = lane_get(ek, i);
-        const double f = s * ei;
-        const double b = c * ei;
-        // |(f, g)|: the plain square root unless the squares could over- or
-        // underflow (the chain of rotations is the leaf's critical path)
-        const double rr = f * f + g * g;
-        r = (rr > 1e-280 && rr < 1e280) ? sqrt(rr) : hypot(f, g);
-        if (k == i + 1) ek = r;
-        if (r == 0.0) {
-          if (k == i + 1) dk -= p;
-          if (k == mm) ek = 0.0;
-          early = true;
-          break;
-        }
-        const double ir = 1.0 / r;
-        s = f * ir;
-        c = g * ir;
-        g = lane_get(dk, i + 1) - p;
-        r = (lane_get(dk, i) - g) * s + 2.0 * c * b;
-        p = s * r;
-        if (k == i + 1) dk = g + p;
-        g = c * r - b;
-        if (k < m) {
-          const double zf = zz[k][i + 1];
-          const double zi = zz[k][i];
-          zz[k][i + 1] = s * zi + c * zf;
-          zz[k][i] = c * zi - s * zf;
-        }
-      }
-      if (early) continue;
-      if (k == l) { dk -= p; ek = g; }
-      if (k == mm) ek = 0.0;
-    }
-    if (fail) break;
-  }
-  // selection sort ascending, columns follow
-  for (int i = 0; i < m - 1; ++i) {
-    int kmin = i;
-    double vmin = lane_get(dk, i);
-    for (int j = i + 1; j < m; ++j) {
-      const double dj = lane_get(dk, j);
-      if (dj < vmin) { vmin = dj; kmin = j; }
-    }
-    if (kmin != i) {
-      const double di = lane_get(dk, i);
-      if (k == kmin) dk = di;
-      if (k == i) dk = vmin;
-      if (k < m) {
-        const double t = zz[k][i];
-        zz[k][i] = zz[k][kmin];
-        zz[k][kmin] = t;
-      }
-    }
-  }
-  if (k < m) {
-    lam[lo + k] = dk;
-    for (int i = 0; i < m; ++i) Z[(lo + k) + (size_t)(lo - ob + i) * ldz] = zz[k][i];
-  }
-  if (fail && k == 0) atomicMax(info + pr, lo - ob + 1);
 }
 
 // --------------------------------------------------------------------------
@@ -514,8 +403,8 @@ __global__ void __launch_bounds__(256) k_merge_gather(const MergeDesc* __restric
     if (k0 + u < ns) Q[r + (size_t)(k0 + u) * ns] = v[u];
 }
 
-// One root of f(t) = 1 + rho sum_j z_j^2 / (delta_j - t) per wavefront, the 64
-// lanes splitting the sum.  Origin: the nearer pole (chosen by the sign of f
+// One root of f(t) = 1 + rho sum_j z_j^2 / (delta_j - t) per group of
+// LANES lanes (64, or a row of 16), which split the sum.  Origin: the nearer pole (chosen by the sign of f
 // at the midpoint of the interval), so t is small and the differences
 // delta_j - t are formed without cancellation.  Iteration: Newton on the
 // pole-free G(t) = (t - p_lo)(p_hi - t) f(t), safeguarded by a bisection
@@ -525,11 +414,22 @@ struct SecSums {
   double r, rp;   // rest = rho sum over the non-pole terms, and its derivative
 };
 
+template <int LANES>
+__device__ __forceinline__ double lanes_sum(double v) {
+  if constexpr (LANES == 64) return wave_sum_d(v);
+  v += xlane<1>(v);
+  v += xlane<2>(v);
+  v += xlane<4>(v);
+  v += xlane<8>(v);
+  return v;
+}
+
+template <int LANES>
 __device__ __forceinline__ SecSums sec_rest(const double* d, const double* z, int K, double dorg, double rho, double t,
                                             int plo, int phi) {
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & (LANES - 1);
   double r = 0.0, rp = 0.0;
-  for (int jj = lane; jj < K; jj += 64) {
+  for (int jj = lane; jj < K; jj += LANES) {
     if (jj == plo || jj == phi) continue;
     const double zj = z[jj];
     const double inv = 1.0 / ((d[jj] - dorg) - t);
@@ -537,25 +437,21 @@ __device__ __forceinline__ SecSums sec_rest(const double* d, const double* z, in
     r += q;
     rp += q * inv;
   }
-  r = wave_sum_d(r);
-  rp = wave_sum_d(rp);
+  r = lanes_sum<LANES>(r);
+  rp = lanes_sum<LANES>(rp);
   return SecSums{rho * r, rho * rp};
 }
 
-// A block serves ROOTS roots of one merge.  Every Newton step re-reads the
-// merge's poles d and weights z, so merges of up to SEC_LDS kept values
-// first stage both in LDS (one read from L2 per block instead of one per
-// root and step; the arithmetic and its order are unchanged).  The LDS is
-// sized for the level's largest merge, and levels of small merges (the many
-// deep merges of a batch) use blocks of 4 roots, so that they keep their
-// occupancy.
-constexpr int SEC_LDS = 4096;
-
-__device__ __forceinline__ void secular_root(const MergeDesc& md, const MergeBufs& B, int K, int i, const double* d,
-                                             const double* z) {
-  const int lo = md.lo;
-  const double rho = B.rho[blockIdx.y];
-  const int lane = threadIdx.x & 63;
+// Root i of a merge with K kept values (poles d, weights z): its origin (a pole
+// index) and offset; *conv false if the step cap was reached.
+struct SecRoot {
+  int org;
+  double t;
+  bool conv;
+};
+template <int LANES>
+__device__ __forceinline__ SecRoot secular_root(double rho, int cap, int K, int i, const double* d, const double* z) {
+  const int lane = threadIdx.x & (LANES - 1);
   int org, plo, phi;
   double a, b, pl, ph;   // bracket (a, b) and pole positions relative to the origin
   double t0;             // first iterate, relative to the origin
@@ -564,14 +460,14 @@ __device__ __forceinline__ void secular_root(const MergeDesc& md, const MergeBuf
     const double half = 0.5 * gap;
     // f at the midpoint with origin d_i, and the part of it from the other poles
     double s = 0.0, sr = 0.0;
-    for (int jj = lane; jj < K; jj += 64) {
+    for (int jj = lane; jj < K; jj += LANES) {
       const double zj = z[jj];
       const double q = zj * zj / ((d[jj] - d[i]) - half);
       s += q;
       if (jj != i && jj != i + 1) sr += q;
     }
-    s = wave_sum_d(s);
-    sr = wave_sum_d(sr);
+    s = lanes_sum<LANES>(s);
+    sr = lanes_sum<LANES>(sr);
     plo = i;
     phi = i + 1;
     if (1.0 + rho * s >= 0.0) { org = i; a = 0.0; b = half; pl = 0.0; ph = gap; }
@@ -593,19 +489,19 @@ __device__ __forceinline__ void secular_root(const MergeDesc& md, const MergeBuf
     t0 = (r1 > a && r1 < b) ? r1 : r2;
   } else {
     double zz = 0.0;
-    for (int jj = lane; jj < K; jj += 64) zz += z[jj] * z[jj];
-    zz = wave_sum_d(zz);
+    for (int jj = lane; jj < K; jj += LANES) zz += z[jj] * z[jj];
+    zz = lanes_sum<LANES>(zz);
     org = i; plo = i; phi = -1;
     a = 0.0; b = rho * zz; pl = 0.0; ph = 0.0;
     // First iterate: the root zl / c of the one-pole model c + rho z_i^2 / (0 - t),
     // c = 1 + rho (the other poles at the midpoint of the bracket)
     const double tm = 0.5 * (a + b);
     double sr = 0.0;
-    for (int jj = lane; jj < K - 1; jj += 64) {
+    for (int jj = lane; jj < K - 1; jj += LANES) {
       const double zj = z[jj];
       sr += zj * zj / ((d[jj] - d[i]) - tm);
     }
-    sr = wave_sum_d(sr);
+    sr = lanes_sum<LANES>(sr);
     const double c = 1.0 + rho * sr;
     const double r = rho * z[i] * z[i] / c;
     t0 = (c > 0.0 && r > a && r < b) ? r : tm;
@@ -615,8 +511,8 @@ __device__ __forceinline__ void secular_root(const MergeDesc& md, const MergeBuf
   const double zh2 = (phi >= 0) ? rho * z[phi] * z[phi] : 0.0;
   double t = (t0 > a && t0 < b) ? t0 : 0.5 * (a + b);
   bool conv = false;
-  for (int it = 0; it < B.cap; ++it) {
-    const SecSums S = sec_rest(d, z, K, dorg, rho, t, plo, phi);
+  for (int it = 0; it < cap; ++it) {
+    const SecSums S = sec_rest<LANES>(d, z, K, dorg, rho, t, plo, phi);
     const double one = 1.0 + S.r;
     double G, Gp;
     if (phi >= 0) {
@@ -652,11 +548,26 @@ __device__ __forceinline__ void secular_root(const MergeDesc& md, const MergeBuf
   // never return the pole itself
   if (org == i && !(t > 0.0)) t = b > 0.0 ? b : DBL_MIN;
   if (org != i && !(t < 0.0)) t = a < 0.0 ? a : -DBL_MIN;
-  if (lane == 0) {
-    B.org[lo + i] = org;
-    B.tau[lo + i] = t;
+  return SecRoot{org, t, conv};
+}
+
+// A block serves ROOTS roots of one merge.  Every Newton step re-reads the
+// merge's poles d and weights z, so merges of up to SEC_LDS kept values
+// first stage both in LDS (one read from L2 per block instead of one per
+// root and step; the arithmetic and its order are unchanged).  The LDS is
+// sized for the level's largest merge, and levels of small merges (the many
+// deep merges of a batch) use blocks of 4 roots, so that they keep their
+// occupancy.
+constexpr int SEC_LDS = 4096;
+
+__device__ __forceinline__ void merge_root(const MergeDesc& md, const MergeBufs& B, int K, int i, const double* d,
+                                           const double* z) {
+  const SecRoot R = secular_root<64>(B.rho[blockIdx.y], B.cap, K, i, d, z);
+  if ((threadIdx.x & 63) == 0) {
+    B.org[md.lo + i] = R.org;
+    B.tau[md.lo + i] = R.t;
     // no convergence within the step cap: reported as zhbev reports a QL failure (info > 0)
-    if (!conv) atomicMax(B.info + md.pr, lo - md.ob + i + 1);
+    if (!R.conv) atomicMax(B.info + md.pr, md.lo - md.ob + i + 1);
   }
 }
 
@@ -680,9 +591,9 @@ __global__ void __launch_bounds__(64 * ROOTS) k_merge_secular(const MergeDesc* _
       sz[q] = z[q];
     }
     __syncthreads();
-    if (i < K) secular_root(md, B, K, i, sd, sz);   // wave-uniform
+    if (i < K) merge_root(md, B, K, i, sd, sz);   // wave-uniform
   } else if (i < K) {
-    secular_root(md, B, K, i, d, z);
+    merge_root(md, B, K, i, d, z);
   }
 }
 
@@ -784,6 +695,359 @@ __global__ void __launch_bounds__(256) k_merge_copydefl(const MergeDesc* __restr
   if (r >= ns) return;
   const double* Q = B.Qtmp + (size_t)lo * B.lq;
   Z[(lo + r) + (size_t)(lo - md.ob + B.posD[lo + t]) * ldz] = Q[r + (size_t)(K + t) * ns];
+}
+
+// --------------------------------------------------------------------------
+// base block: the divide & conquer of up to BASE rows in one workgroup, with
+// the eigenvectors Q in LDS.  The block is halved D = 0 .. 4 times into 2^D
+// leaves of at most 4 rows (all at the same depth, since sizes at a depth
+// differ by at most one), each solved by cyclic Jacobi in one thread's
+// registers; then D levels of merges, the 2^k merges of a level side by side,
+// each by a team of 1024 >> k threads, 16 threads per row.  A merge is the
+// algorithm of the merge kernels above (rank, deflate, secular roots, zhat, U, product).
+// Instead of gathering the kept columns of Q, the rows of U are scattered to
+// Q's column order, with a unit entry for each deflated column, so that one
+// product Q U on MFMA forms every new column; without deflation rotations Q is
+// block diagonal and the product sums over each row's half only.
+//
+// One launch where leaves of 16 rows by QL (one wavefront each, a serial chain
+// of ~220 rotations: 151 us) and ten launches per level took 245 us for 64
+// rows, now 85 us with the
+// kernels around it (2n = 128 solve 540 -> 378 us, 510 2.29 -> 2.11 ms, 1024
+// 4.65 -> 4.52 ms).
+// A leaf is (lo, hi, problem base, problem index).
+// --------------------------------------------------------------------------
+constexpr int BT = 1024;
+constexpr int BQ = BASE + 1;   // column stride of Q and U in LDS (doubles)
+
+__device__ __forceinline__ void jacobi_rot(double (&A)[4][4], double (&V)[4][4], int p, int q, bool& any) {
+  const double apq = A[p][q];
+  if (!(fabs(apq) > DEPS * (fabs(A[p][p]) + fabs(A[q][q])))) return;
+  any = true;
+  const double th = (A[q][q] - A[p][p]) / (2.0 * apq);
+  const double t = copysign(1.0 / (fabs(th) + sqrt(fma(th, th, 1.0))), th);
+  const double c = 1.0 / sqrt(fma(t, t, 1.0)), s = t * c;
+  A[p][p] = fma(-t, apq, A[p][p]);
+  A[q][q] = fma(t, apq, A[q][q]);
+  A[p][q] = A[q][p] = 0.0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (r != p && r != q) {
+      const double x = A[r][p], y = A[r][q];
+      A[r][p] = A[p][r] = c * x - s * y;
+      A[r][q] = A[q][r] = s * x + c * y;
+    }
+    const double x = V[r][p], y = V[r][q];
+    V[r][p] = c * x - s * y;
+    V[r][q] = s * x + c * y;
+  }
+}
+
+__global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, double* __restrict__ lam,
+                                                const double* __restrict__ es, double* __restrict__ Z, int ldz,
+                                                int* __restrict__ info, int cap_leaf, int cap_sec) {
+  typedef double d4 __attribute__((ext_vector_type(4)));
+  __shared__ double Q[BASE * BQ], U[BASE * BQ];   // column-major
+  __shared__ double sl[BASE], se[BASE];           // diagonal / eigenvalues, subdiagonal
+  __shared__ double dk[BASE], zk[BASE];           // sorted d, z of a merge
+  __shared__ double dkk[BASE], zkk[BASE], dv[BASE];   // kept d, z; deflated d
+  __shared__ double tau[BASE], zh[BASE], val[BASE];
+  __shared__ double rot[4 * BASE];
+  __shared__ int src[BASE], keep[BASE], dfl[BASE], org[BASE], pos[BASE];   // pos: by column of Q
+  __shared__ int sK[8], snr[8];
+  __shared__ int bnd[17];
+  const int lo0 = leaves[4 * blockIdx.x], m = leaves[4 * blockIdx.x + 1] - lo0;
+  const int ob = leaves[4 * blockIdx.x + 2], pr = leaves[4 * blockIdx.x + 3];
+  const int tid = threadIdx.x, lane = tid & 63;
+  int D = 0;
+  while ((4 << D) < m) ++D;
+  if (tid < m) sl[tid] = lam[lo0 + tid];
+  if (tid < m - 1) se[tid] = es[lo0 + tid];
+  if (tid <= (1 << D)) {   // leaf boundary: follow the bits from the top
+    int a = 0, b = m;
+    if (tid < (1 << D))
+      for (int k = D - 1; k >= 0; --k) {
+        const int mid = a + (b - a) / 2;
+        if ((tid >> k) & 1) a = mid; else b = mid;
+      }
+    else a = m;
+    bnd[tid] = a;
+  }
+  for (int k = tid; k < BASE * BQ; k += BT) Q[k] = 0.0;
+  __syncthreads();
+  // ---- leaves
+  if (tid < (1 << D)) {
+    const int a = bnd[tid], sz = bnd[tid + 1] - a;
+    double A[4][4], V[4][4];
+    int fail = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        A[i][j] = 0.0;
+        V[i][j] = i == j ? 1.0 : 0.0;
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i < sz) {
+        double v = sl[a + i];   // torn at the splits inside the base block
+        if (i == 0 && a > 0) v -= se[a - 1];
+        if (i == sz - 1 && a + sz < m) v -= se[a + sz - 1];
+        A[i][i] = v;
+      }
+      if (i < 3 && i + 1 < sz) A[i][i + 1] = A[i + 1][i] = se[a + i];
+    }
+    for (int it = 0;;) {
+      bool any = false;
+      jacobi_rot(A, V, 0, 1, any);
+      jacobi_rot(A, V, 2, 3, any);
+      jacobi_rot(A, V, 0, 2, any);
+      jacobi_rot(A, V, 1, 3, any);
+      jacobi_rot(A, V, 0, 3, any);
+      jacobi_rot(A, V, 1, 2, any);
+      if (!any) break;
+      if (++it >= cap_leaf) { fail = 1; break; }
+    }
+    double w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = i < sz ? A[i][i] : DBL_MAX;   // absent rows stay last
+    auto order = [&](int i, int j) {
+      if (w[j] < w[i]) {
+        double t = w[i]; w[i] = w[j]; w[j] = t;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) { t = V[r][i]; V[r][i] = V[r][j]; V[r][j] = t; }
+      }
+    };
+    order(0, 1); order(2, 3); order(0, 2); order(1, 3); order(1, 2);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j < sz) {
+        sl[a + j] = w[j];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (r < sz) Q[(a + j) * BQ + a + r] = V[r][j];
+      }
+    if (fail) atomicMax(info + pr, lo0 - ob + a + 1);
+  }
+  __syncthreads();
+  // ---- merges, 2^k at level k
+  for (int k = D - 1; k >= 0; --k) {
+    const int ts = BT >> k, team = tid / ts, tt = tid - team * ts;
+    const int lo = bnd[team << (D - k)], hi = bnd[(team + 1) << (D - k)];
+    const int mid = bnd[(2 * team + 1) << (D - k - 1)];
+    const int ns = hi - lo, n1 = mid - lo;
+    const int row = tt >> 4, sub = tt & 15;   // 16 lanes per row (row < ns holds work)
+    const double rho = 2.0 * se[mid - 1];
+    // rank of each value in the merged order (stable), z from the rows at the split
+    if (row < ns) {
+      const double v = sl[lo + row];
+      int cnt = 0;
+      if (row < n1) {
+        for (int t = n1 + sub; t < ns; t += 16) cnt += sl[lo + t] < v;
+      } else {
+        for (int t = sub; t < n1; t += 16) cnt += sl[lo + t] <= v;
+      }
+#pragma unroll
+      for (int b = 1; b < 16; b <<= 1) cnt += __shfl_xor(cnt, b, 16);
+      if (sub == 0) {
+        const int r = lo + (row < n1 ? row : row - n1) + cnt;
+        dk[r] = v;
+        zk[r] = 0.70710678118654752440 * Q[(lo + row) * BQ + (row < n1 ? mid - 1 : mid)];
+        src[r] = row;
+      }
+    }
+    __syncthreads();
+    // deflation, by the team's first wave (lane = sorted position)
+    if (tt < 64) {
+      const bool in = lane < ns;
+      double dl = in ? dk[lo + lane] : 0.0, zl = in ? zk[lo + lane] : 0.0;
+      double dm = fabs(dl), zm = fabs(zl);
+#pragma unroll
+      for (int b = 1; b < 64; b <<= 1) {
+        dm = fmax(dm, __shfl_xor(dm, b, 64));
+        zm = fmax(zm, __shfl_xor(zm, b, 64));
+      }
+      const double tol = 8.0 * DEPS * fmax(dm, rho * zm);
+      const bool kept = in && !(rho * fabs(zl) <= tol);
+      const unsigned long long km = __ballot(kept), im = __ballot(in && !kept);
+      const unsigned long long below = (1ull << lane) - 1ull;
+      // the rotation test against the previous kept value; if none passes on the
+      // unrotated values, the scan rotates nowhere
+      const int pv = (km & below) ? 63 - __clzll((long long)(km & below)) : 0;
+      const double zp = __shfl(zl, pv, 64), dp = __shfl(dl, pv, 64);
+      bool rotates = false;
+      if (kept && (km & below)) {
+        const double h = hypot(zl, zp);
+        rotates = fabs((dl - dp) * (zl / h) * (-zp / h)) <= tol;
+      }
+      if (!__any(rotates)) {
+        if (kept) {
+          const int q = __popcll(km & below);
+          keep[lo + q] = lane;
+          dkk[lo + q] = dl;
+          zkk[lo + q] = zl;
+        } else if (in) {
+          const int q = __popcll(im & below);
+          dfl[lo + q] = lane;
+          dv[lo + q] = dl;
+        }
+        if (lane == 0) {
+          sK[team] = __popcll(km);
+          snr[team] = 0;
+        }
+      } else if (lane == 0) {   // the sequential scan of k_merge_prep
+        double *d = dk + lo, *z = zk + lo;
+        int *kp = keep + lo, *df = dfl + lo;
+        int K = 0, nd = 0, nr = 0, pj = -1;
+        for (int j = 0; j < ns; ++j) {
+          if (rho * fabs(z[j]) <= tol) {
+            int q = nd++;
+            while (q > 0 && d[df[q - 1]] > d[j]) { df[q] = df[q - 1]; --q; }
+            df[q] = j;
+            continue;
+          }
+          if (pj < 0) { pj = j; continue; }
+          double s = z[pj], c = z[j];
+          const double h = hypot(c, s);
+          const double t = d[j] - d[pj];
+          c /= h;
+          s = -s / h;
+          if (fabs(t * c * s) <= tol) {
+            z[j] = h;
+            z[pj] = 0.0;
+            double* ro = rot + 4 * (lo + nr++);
+            ro[0] = (double)pj; ro[1] = (double)j; ro[2] = c; ro[3] = s;
+            const double x = d[pj] * c * c + d[j] * s * s;
+            d[j] = d[pj] * s * s + d[j] * c * c;
+            d[pj] = x;
+            int q = nd++;
+            while (q > 0 && d[df[q - 1]] > d[pj]) { df[q] = df[q - 1]; --q; }
+            df[q] = pj;
+          } else {
+            kp[K++] = pj;
+          }
+          pj = j;
+        }
+        if (pj >= 0) kp[K++] = pj;
+        for (int j = 0; j < K; ++j) {
+          dkk[lo + j] = d[kp[j]];
+          zkk[lo + j] = z[kp[j]];
+        }
+        for (int j = 0; j < nd; ++j) dv[lo + j] = d[df[j]];
+        sK[team] = K;
+        snr[team] = nr;
+      }
+    }
+    for (int q = tt; q < ns * BQ; q += ts) U[lo * BQ + q] = 0.0;
+    __syncthreads();
+    const int K = sK[team], nr = snr[team];
+    // the rotations (thread = row of Q; columns lo + src)
+    if (tt < ns)
+      for (int t = 0; t < nr; ++t) {
+        const double* ro = rot + 4 * (lo + t);
+        double* qp = Q + (lo + src[lo + (int)ro[0]]) * BQ + lo + tt;
+        double* qj = Q + (lo + src[lo + (int)ro[1]]) * BQ + lo + tt;
+        const double x = *qp, y = *qj;
+        *qp = ro[2] * x + ro[3] * y;
+        *qj = ro[2] * y - ro[3] * x;
+      }
+    if (row < K) {
+      const SecRoot R = secular_root<16>(rho, cap_sec, K, row, dkk + lo, zkk + lo);
+      if (sub == 0) {
+        org[lo + row] = R.org;
+        tau[lo + row] = R.t;
+        val[lo + row] = dkk[lo + R.org] + R.t;
+        if (!R.conv) atomicMax(info + pr, lo0 - ob + lo + row + 1);
+      }
+    }
+    __syncthreads();
+    if (row < K) {   // Gu-Eisenstat zhat of kept value `row`
+      const double dj = dkk[lo + row];
+      double prod = 1.0;
+      for (int i = sub; i < K; i += 16) {
+        const double num = (dkk[lo + org[lo + i]] - dj) + tau[lo + i];
+        prod *= (i == row) ? num / rho : num / (dkk[lo + i] - dj);
+      }
+#pragma unroll
+      for (int b = 1; b < 16; b <<= 1) prod *= __shfl_xor(prod, b, 16);
+      if (sub == 0) zh[lo + row] = copysign(sqrt(fmax(prod, 0.0)), zkk[lo + row]);
+    } else if (row < ns) {   // final position of deflated value row - K: the roots before it
+      const double v = dv[lo + row - K];
+      int cnt = 0;
+      for (int i = sub; i < K; i += 16) cnt += val[lo + i] <= v;
+#pragma unroll
+      for (int b = 1; b < 16; b <<= 1) cnt += __shfl_xor(cnt, b, 16);
+      if (sub == 0) {
+        const int c = src[lo + dfl[lo + row - K]];
+        pos[lo + row] = row - K + cnt;      // by U's column
+        U[(lo + row) * BQ + lo + c] = 1.0;
+        sl[lo + row - K + cnt] = v;
+      }
+    }
+    __syncthreads();
+    if (row < K) {   // column `row` of U, normalised, and its final position
+      const double dorg = dkk[lo + org[lo + row]], t = tau[lo + row];
+      double u[BASE / 16], ss = 0.0;
+#pragma unroll
+      for (int h = 0; h < BASE / 16; ++h) {
+        const int j = sub + 16 * h;
+        u[h] = j < K ? zh[lo + j] / ((dkk[lo + j] - dorg) - t) : 0.0;
+        ss += u[h] * u[h];
+      }
+      ss = lanes_sum<16>(ss);
+      const double inv = 1.0 / sqrt(ss);
+#pragma unroll
+      for (int h = 0; h < BASE / 16; ++h) {
+        const int j = sub + 16 * h;
+        if (j < K) U[(lo + row) * BQ + lo + src[lo + keep[lo + j]]] = u[h] * inv;
+      }
+      const double v = val[lo + row];
+      int cnt = 0;
+      for (int q = sub; q < ns - K; q += 16) cnt += dv[lo + q] < v;
+#pragma unroll
+      for (int b = 1; b < 16; b <<= 1) cnt += __shfl_xor(cnt, b, 16);
+      if (sub == 0) {
+        pos[lo + row] = row + cnt;
+        sl[lo + row + cnt] = v;
+      }
+    }
+    __syncthreads();
+    // new columns: (Q U) in 16 x 16 tiles, one per wave of the team (a team has
+    // 16 ns / 64 waves or more, and ceil(ns / 16)^2 <= that number of tiles)
+    const int nt = (ns + 15) >> 4;
+    const int wv = tt >> 6, tr = wv % nt, tc = wv / nt;
+    const bool tile = wv < nt * nt;
+    d4 acc = d4{0.0, 0.0, 0.0, 0.0};
+    if (tile) {
+      const int r = 16 * tr + (lane & 15), c = 16 * tc + (lane & 15);
+      int kb = 0, ke = ns;
+      if (nr == 0) {   // block diagonal: the half these rows lie in
+        if (16 * tr >= n1) kb = n1 & ~3;
+        else if (16 * tr + 16 <= n1) ke = n1;
+      }
+      for (int q = kb; q < ke; q += 4) {
+        const int kc = q + (lane >> 4);
+        const double af = (r < ns && kc < ns) ? Q[(lo + kc) * BQ + lo + r] : 0.0;
+        const double bf = (c < ns && kc < ns) ? U[(lo + c) * BQ + lo + kc] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(af, bf, acc, 0, 0, 0);
+      }
+    }
+    __syncthreads();
+    if (tile) {
+      const int c = 16 * tc + (lane & 15);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = 16 * tr + 4 * t + (lane >> 4);
+        if (r < ns && c < ns) Q[(lo + pos[lo + c]) * BQ + lo + r] = acc[t];
+      }
+    }
+    __syncthreads();
+  }
+  if (tid < m) lam[lo0 + tid] = sl[tid];
+  for (int k = tid; k < m * m; k += BT) {
+    const int c = k / m, r = k - c * m;
+    Z[(lo0 + r) + (size_t)(lo0 - ob + c) * ldz] = Q[c * BQ + r];
+  }
 }
 
 // Eigenvalues of a problem whose input held a NaN or an infinity are NaN.
@@ -925,7 +1189,7 @@ int status_out(const int* word, int* out, hipStream_t s) {
 // --------------------------------------------------------------------------
 static void build_tree(int lo, int hi, int ob, int pr, int depth, std::vector<int>& leaves,
                        std::vector<std::vector<MergeDesc>>& lv, std::vector<int>& splits) {
-  if (hi - lo <= LEAF) {
+  if (hi - lo <= BASE) {
     leaves.insert(leaves.end(), {lo, hi, ob, pr});
     return;
   }
@@ -938,9 +1202,9 @@ static void build_tree(int lo, int hi, int ob, int pr, int depth, std::vector<in
 }
 
 size_t stedc_int_slots(int ntot, int nprob) {
-  // per problem of size n at most L = 2 ceil(n / LEAF) leaves (4 ints each),
+  // per problem of size n at most L = 2 ceil(n / BASE) base blocks (4 ints each),
   // L - 1 splits (1 int) and L - 1 merges (5 ints), and (offset, size)
-  return (size_t)22 * (ntot / LEAF + nprob) + 2 * (size_t)nprob + 64;
+  return (size_t)22 * (ntot / BASE + nprob) + 2 * (size_t)nprob + 64;
 }
 
 int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const double* d, const double* e, double* w,
@@ -998,7 +1262,8 @@ int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const dou
   if (!splits.empty())
     hipLaunchKernelGGL(k_dc_tear, dim3(cdiv((int)splits.size(), 256)), dim3(256), 0, s, (int)splits.size(), isplit,
                        sw.es, sw.lam);
-  hipLaunchKernelGGL(k_dc_leaf, dim3(nleaf), dim3(64), 0, s, ileaf, sw.lam, sw.es, sw.Z, ldz, sw.info, sw.cap_leaf);
+  hipLaunchKernelGGL(k_dc_base, dim3(nleaf), dim3(BT), 0, s, ileaf, sw.lam, sw.es, sw.Z, ldz, sw.info, sw.cap_leaf,
+                     sw.cap_secular);
   MergeBufs B{sw.dk, sw.zk, sw.src, sw.keep, sw.dfl, sw.rot, sw.nrot, sw.kcnt, sw.dkk, sw.zkk, sw.dval, sw.rho,
               sw.org, sw.tau, sw.zhat, sw.posK, sw.posD, sw.Qtmp, sw.U, lq, sw.info, sw.cap_secular,
               sw.mix, sw.gpos, sw.ginv, sw.kgrp};

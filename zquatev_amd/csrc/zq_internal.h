@@ -361,7 +361,7 @@ struct StedcWork {
   int* ints;      // tree descriptors
   size_t int_slots;
   Staging* stage; // host staging of the descriptors
-  // iteration caps: QL sweeps per leaf eigenvalue, secular-equation steps
+  // iteration caps: Jacobi sweeps per leaf, secular-equation steps
   // per root, multisection steps per eigenvalue (reaching one is reported
   // as non-convergence, info > 0)
   int cap_leaf = 60, cap_secular = 200, cap_bisect = 64;
