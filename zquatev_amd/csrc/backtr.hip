@@ -23,49 +23,48 @@
 namespace zq {
 
 // phi_0 = 1, phi_{c+1} = r_c phi_c with r_c = e_c / |e_c| (1 where e_c = 0):
-// a prefix product of unit quaternions, chunked over one workgroup.
-constexpr int PH_T = 256;
+// a prefix product of unit quaternions in one workgroup: a chunk per thread,
+// then a scan of the chunks' products over each wave's lanes and over the
+// waves.  (Scanning 256 chunks one after the other, and chunks four times as
+// long, took 14 us at n = 64 and 56 us at n = 4096; now @PH@.)
+constexpr int PH_T = 1024;
+__device__ __forceinline__ quat unit_of(const quat& e) {
+  const double ae = sqrt(qnorm2(e));
+  return (ae > 0.0) ? qscale(e, 1.0 / ae) : quat{1.0, 0.0, 0.0, 0.0};
+}
+__device__ __forceinline__ quat shfl_up_q(const quat& v, int k) {
+  return quat{__shfl_up(v.ar, k, 64), __shfl_up(v.ai, k, 64), __shfl_up(v.br, k, 64), __shfl_up(v.bi, k, 64)};
+}
 __global__ void __launch_bounds__(PH_T) k_phases(int n, const quat* __restrict__ e, quat* __restrict__ phi, ZB zb) {
   if (zb.nvec) {
     n = zb.nvec[blockIdx.z];
     e = zoff(e, zb); phi = zoff(phi, zb);
   }
-  __shared__ quat tot[PH_T];
-  __shared__ quat off[PH_T];
-  const int t = threadIdx.x;
-  const int chunk = (n + PH_T - 1) / PH_T;
-  const int a = t * chunk, b = min(n, a + chunk);
-  // local prefix: L_k = r_{k-1} ... r_a for k in (a, b], L_a = 1
-  quat L = quat{1.0, 0.0, 0.0, 0.0};
+  __shared__ quat tot[PH_T / 64];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const quat one = quat{1.0, 0.0, 0.0, 0.0};
+  // thread t owns phi_k for k in (a, b]: the products r_{k-1} ... r_a
+  const int chunk = (n - 1 + PH_T - 1) / PH_T;
+  const int a = min(n - 1, t * chunk), b = min(n - 1, a + chunk);
+  quat L = one;
+  for (int k = a; k < b; ++k) L = qmul(unit_of(qload(e + k)), L);
+  // inclusive scan over the lanes: later chunks multiply from the left
+#pragma unroll
+  for (int k = 1; k < 64; k <<= 1) {
+    const quat o = shfl_up_q(L, k);
+    if (lane >= k) L = qmul(L, o);
+  }
+  if (lane == 63) tot[wv] = L;
+  __syncthreads();
+  quat base = one;   // the waves before
+  for (int w = 0; w < wv; ++w) base = qmul(tot[w], base);
+  const quat prev = shfl_up_q(L, 1);
+  quat cur = lane == 0 ? base : qmul(prev, base);   // phi_a
+  if (t == 0) qstore(phi, one);
   for (int k = a; k < b; ++k) {
-    if (k > a) {
-      const quat ek = qload(e + k - 1);
-      const double ae = sqrt(qnorm2(ek));
-      const quat r = (ae > 0.0) ? qscale(ek, 1.0 / ae) : quat{1.0, 0.0, 0.0, 0.0};
-      L = qmul(r, L);
-    }
-    qstore(phi + k, L);
+    cur = qmul(unit_of(qload(e + k)), cur);
+    qstore(phi + k + 1, cur);
   }
-  // chunk total maps phi_a to phi_b: T = r_{b-1} L_{b-1}
-  quat T = L;
-  if (b > a && b < n) {
-    const quat ek = qload(e + b - 1);
-    const double ae = sqrt(qnorm2(ek));
-    const quat r = (ae > 0.0) ? qscale(ek, 1.0 / ae) : quat{1.0, 0.0, 0.0, 0.0};
-    T = qmul(r, L);
-  }
-  tot[t] = T;
-  __syncthreads();
-  if (t == 0) {
-    quat cur = quat{1.0, 0.0, 0.0, 0.0};
-    for (int k = 0; k < PH_T; ++k) {
-      off[k] = cur;
-      if (k * chunk < n) cur = qmul(tot[k], cur);
-    }
-  }
-  __syncthreads();
-  const quat o = off[t];
-  for (int k = a; k < b; ++k) qstore(phi + k, qmul(qload(phi + k), o));
 }
 
 // X[i, j] = phi_i Z[i, j]  (in a batch, problem z's Z block starts at row zrow[z])
@@ -94,19 +93,27 @@ __global__ void __launch_bounds__(256) k_sum_parts_b(const SumTask* __restrict__
   qstore_g(t.out + i, s);
 }
 
-// T = (I + triu(G, 1))^{-1} for each block: T[0:j, j] = -T[0:j, 0:j] G[0:j, j],
-// T[j, j] = 1, zero below (the compact-WY recurrence with every tau = 1).
-// G and T are stored per block of sub * WB reflectors (leading dimension
-// sub * WB); workgroup x factors the diagonal WB x WB sub-block h = x % sub
-// of stored block x / sub (problem blockIdx.z) and clears the part of T left
-// of it (rows h WB .. + WB, columns 0 .. h WB).  For sub > 1 the blocks above
-// the diagonal are formed afterwards by GEMMs, pairs of neighbouring
+// T = (I + triu(G, 1))^{-1} for each block (the compact-WY factor with every
+// tau = 1).  G and T are stored per block of sub * WB reflectors (leading
+// dimension sub * WB); workgroup x inverts the diagonal WB x WB sub-block
+// h = x % sub of stored block x / sub (problem blockIdx.z) and clears the part
+// of T left of it (rows h WB .. + WB, columns 0 .. h WB).  For sub > 1 the blocks
+// above the diagonal are formed afterwards by GEMMs, pairs of neighbouring
 // sub-blocks of width w = WB, 2 WB, ... merged level by level:
 // T12 = -T1 (G12 T2).
+//
+// The sub-block is inverted the same way, in place in LDS (above the diagonal
+// G becomes T; the unit diagonal is implied and stored as 0): pairs of width
+// w = 1, 2, .., 32, each level the products P = G12 T2 and T12 = -T1 P with one
+// thread per element.  Lanes run along the index that the triangular factor
+// does not bound, so that a wave's loop ends with its own columns (rows).  Twelve short
+// products instead of the 64-column recurrence (four columns at a time, three
+// barriers each): 65 us -> @TF@.
 constexpr int TF_WB = 64;
-__global__ void __launch_bounds__(256) k_tfactor(int n, const quat* __restrict__ Gall, quat* __restrict__ Tall,
-                                                 int sub, ZB zb) {
-  constexpr int WB = TF_WB;
+constexpr int TF_T = 1024;
+__global__ void __launch_bounds__(TF_T) k_tfactor(int n, const quat* __restrict__ Gall, quat* __restrict__ Tall,
+                                                  int sub, ZB zb) {
+  constexpr int WB = TF_WB, LS = WB + 1;   // LS: column stride
   if (zb.nvec) {
     n = zb.nvec[blockIdx.z];
     Gall = zoff(Gall, zb); Tall = zoff(Tall, zb);
@@ -118,53 +125,41 @@ __global__ void __launch_bounds__(256) k_tfactor(int n, const quat* __restrict__
   const int wdt = min(WB, n - 1 - p);   // <= 0: no reflectors here, T is the identity
   const quat* G = Gall + (size_t)sb * ldt * ldt + (size_t)h * WB * (ldt + 1);
   quat* T = Tall + (size_t)sb * ldt * ldt + (size_t)h * WB * (ldt + 1);
-  // Columns in groups of TB = 256 / WB, one per wave set: thread (r, c) (its
-  // row r of T, column J + c of the group) first applies the columns l < J
-  // (T rows re-read from LDS, the group's G entries staged in LDS); then the
-  // threads of c = 0 run the recurrence inside the group from those
-  // partials.  Every entry sums l = r .. jj-1 in increasing order, as the
-  // column-by-column recurrence does.  T stays in LDS (its rows are re-read
-  // for every later group) and is written out at the end.
-  constexpr int TB = 256 / WB;
-  __shared__ quat gs[TB][WB];
-  __shared__ quat ax[TB][WB];
-  __shared__ quat Ts[WB][WB];   // Ts[col][row]
-  const int r = threadIdx.x % WB, cq = threadIdx.x / WB;
-  for (int J = 0; J < WB; J += TB) {
-    const int jq = J + cq;
-    if (J >= wdt) {   // columns past the block's reflectors: identity (uniform branch)
-      Ts[jq][r] = r == jq ? quat{1.0, 0.0, 0.0, 0.0} : qzero();
-      continue;
-    }
-    gs[cq][r] = (jq < wdt && r < jq) ? qload(G + r + (size_t)jq * ldt) : qzero();
+  __shared__ quat A[WB * LS];   // A[col * LS + row]
+  const int tid = threadIdx.x;
+  for (int idx = tid; idx < WB * WB; idx += TF_T) {
+    const int col = idx / WB, row = idx % WB;
+    A[col * LS + row] = (row < col && col < wdt) ? qload(G + row + (size_t)col * ldt) : qzero();
+  }
+  for (int w = 1; w < WB; w <<= 1) {   // pairs of width w: WB w / 2 elements
+    const bool on = tid < WB / 2 * w;   // whole waves from w = 2
+    const int x = tid & (w - 1), y = (tid / w) & (w - 1), q = tid / (w * w) * 2 * w;   // pair at q, q + w
     __syncthreads();
     quat acc = qzero();
-#pragma unroll 4
-    for (int l = r; l < J; ++l) qfma(acc, Ts[l][r], gs[cq][l]);
-    ax[cq][r] = acc;
-    __syncthreads();
-    if (cq == 0) {
-      quat tb[TB];
-#pragma unroll
-      for (int c = 0; c < TB; ++c) {
-        const int jj = J + c;
-        quat a = ax[c][r];
-#pragma unroll
-        for (int cc = 0; cc < c; ++cc)
-          if (r <= J + cc) qfma(a, tb[cc], gs[c][J + cc]);
-        if (jj < wdt && r < jj) tb[c] = qscale(a, -1.0);
-        else tb[c] = (r == jj) ? quat{1.0, 0.0, 0.0, 0.0} : qzero();
-        Ts[jj][r] = tb[c];
-      }
+    if (on) {   // P(x, y) = G12(x, y) + sum_{k < y} G12(x, k) T2(k, y)
+      const quat* g = A + (q + w) * LS + q + x;          // G12(x, 0); columns LS apart
+      const quat* t2 = A + (q + w + y) * LS + q + w;     // T2(0, y)
+      acc = g[y * LS];
+      for (int k = 0; k < y; ++k) qfma(acc, g[k * LS], t2[k]);
     }
     __syncthreads();
+    if (on) A[(q + w + y) * LS + q + x] = acc;
+    __syncthreads();
+    if (on) {   // T12(y, x) = -(P(y, x) + sum_{k > y} T1(y, k) P(k, x))
+      const quat* pc = A + (q + w + x) * LS + q;         // P(0, x)
+      const quat* t1 = A + q * LS + q + y;               // T1(y, 0); columns LS apart
+      acc = pc[y];
+      for (int k = y + 1; k < w; ++k) qfma(acc, t1[k * LS], pc[k]);
+    }
+    __syncthreads();
+    if (on) A[(q + w + x) * LS + q + y] = qneg(acc);
   }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < WB * WB; idx += 256) {
-    const int col = idx / WB, row = idx - col * WB;
-    qstore(T + row + (size_t)col * ldt, Ts[col][row]);
+  for (int idx = tid; idx < WB * WB; idx += TF_T) {
+    const int col = idx / WB, row = idx % WB;
+    qstore(T + row + (size_t)col * ldt, row == col ? quat{1.0, 0.0, 0.0, 0.0} : A[col * LS + row]);
   }
-  for (int idx = threadIdx.x; idx < WB * h * WB; idx += 256) {   // below the diagonal, left of this sub-block
+  for (int idx = tid; idx < WB * h * WB; idx += TF_T) {   // below the diagonal, left of this sub-block
     const int col = idx / WB, row = idx - col * WB;
     qstore(T - (size_t)h * WB * ldt + row + (size_t)col * ldt, qzero());
   }
@@ -351,7 +346,7 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
   if ((rc = qgemm_tasks(tasks + gt0, ngt, gmaxk, gmaxk, true, false, false, s))) return rc;
   hipLaunchKernelGGL(k_sum_parts_b, dim3(cdiv(wbt * wbt, 256), 1, ngs), dim3(256), 0, s, sums);
   if (wbt < TF_WB || wbt % TF_WB || (tsub & (tsub - 1))) return ZQI_ERR_ARG;
-  hipLaunchKernelGGL(k_tfactor, dim3(nblk * tsub, 1, nprob), dim3(256), 0, s, L, w.G, w.T, tsub, zb);
+  hipLaunchKernelGGL(k_tfactor, dim3(nblk * tsub, 1, nprob), dim3(TF_T), 0, s, L, w.G, w.T, tsub, zb);
   for (size_t li = 0; li < levels.size(); ++li) {
     const int wl = TF_WB << li;
     if ((rc = qgemm_tasks(tasks + levels[li].p0, levels[li].np, wl, wl, false, false, false, s))) return rc;
