@@ -67,17 +67,18 @@ struct Refl {
 };
 __device__ __forceinline__ Refl reflector(const quat& x1, double tail, quat* alpha) {
 #pragma clang fp contract(off)
-  const double ax1 = sqrt(qnorm2(x1));
+  // the two square roots and the reciprocal do not wait for each other
+  const double x2 = qnorm2(x1);
+  const double ax1 = sqrt(x2), nx = sqrt(x2 + tail), ix1 = rsqrt(x2);
   Refl R;
   if (!(tail > 0.0)) {
     R.g = 0.0;
     R.u1 = qzero();
     *alpha = x1;
   } else {
-    const double nx = sqrt(ax1 * ax1 + tail);
-    const quat qph = (ax1 > 0.0) ? qscale(x1, 1.0 / ax1) : quat{1.0, 0.0, 0.0, 0.0};
+    const quat qph = (ax1 > 0.0) ? qscale(x1, ix1) : quat{1.0, 0.0, 0.0, 0.0};
     const double sm = ax1 + nx;
-    R.g = 1.0 / sqrt(nx * sm);
+    R.g = rsqrt(nx * sm);
     R.u1 = qscale(qph, sm * R.g);
     *alpha = qscale(qph, -nx);
   }
@@ -144,9 +145,8 @@ __global__ void __launch_bounds__(SYT) k_symv(
   if (b < 0) {
     // ---- finishing block: reflector, scalars, tall-skinny products
     const bool has_ts = bt < NT;
-    // every load of the block is issued before the first wait: the row-s0
-    // entries of W and V (for the u_1 term of TS), the diagonal entries, and
-    // the partials in batches of 16 per lane (one batch up to m = 2048)
+    // the row-s0 entries of W and V (for the u_1 term of TS), the diagonal
+    // entries, and the partials in batches of 8 per lane
     const int e0 = 64 * bt + 4 * (tid & 15);
     const int lts = e0 >> 3, side = (e0 >> 2) & 1;
     const bool fin = has_ts && tid < 16 && lts < j;
@@ -157,29 +157,27 @@ __global__ void __launch_bounds__(SYT) k_symv(
       mss = M[s0 + (size_t)s0 * ld].ar;
       if (j == 0) mcc = M[c + (size_t)c * ld].ar;
     }
-    double tsacc = 0.0;
+    const quat x1 = qload(M + s0 + (size_t)c * ld);
+    double tail = 0.0, tsacc = 0.0;
     if (has_ts) {
+      // the tail norm from the partials the column kernel left, in wave 0 alone
+      // (it and its reflector then wait for no other wave)
+      if (w == 0)
+        for (int k = lane; k < nparts; k += 64) tail += part[k];
       const int eidx = 64 * bt + lane;
-      constexpr int TB = 16;
+      constexpr int TB = 8;
       for (int k0 = w; k0 < nparts; k0 += NWV * TB) {
         double v[TB];
 #pragma unroll
-        for (int u = 0; u < TB; ++u) {
-          const int k = k0 + NWV * u;
-          v[u] = k < nparts ? TSP[(size_t)k * ldtsp + eidx] : 0.0;
-        }
+        for (int u = 0; u < TB; ++u) v[u] = TSP[(size_t)min(k0 + NWV * u, nparts - 1) * ldtsp + eidx];
 #pragma unroll
-        for (int u = 0; u < TB; ++u) tsacc += v[u];
+        for (int u = 0; u < TB; ++u) tsacc = fma(k0 + NWV * u < nparts ? 1.0 : 0.0, v[u], tsacc);
       }
-    }
-    const quat x1 = qload(M + s0 + (size_t)c * ld);
-    double tail = 0.0;
-    if (j == 0) {   // a panel's first column has no pending update: its tail norm from the column itself
+      tail = wave_sum_d(tail);
+    } else {   // a panel's first column has no pending update: its tail norm from the column itself
       for (int i = c + 2 + tid; i < n; i += SYT) tail += qnorm2(qload(M + i + (size_t)c * ld));
-    } else {        // else from the partials the column kernel left for it
-      for (int k = tid; k < nparts; k += SYT) tail += part[k];
+      tail = block_sum(tail, sh);
     }
-    tail = block_sum(tail, sh);
     quat alpha;
     const Refl R = reflector(x1, tail, &alpha);
     if (bt == 0 && tid == 0) {
@@ -355,26 +353,19 @@ __device__ __forceinline__ ColScalars col_scalars(double qf, double ab, double c
   C.dnext = fma(-2.0, qdot(u1, C.wc1), fma(-2.0, cc, m00));
   return C;
 }
-// The block sums, from the first two waves' lanes (wave 0: lane l < j holds
-// panel column l's coefficients, or with two columns per lane l and l + 64;
-// wave 1: the terms of (M x)_{s0}); x^* M x terms are in every lane.  Each wave
-// sums only what it holds: sh[wave][t] = its sum t.
-__device__ __forceinline__ void col_wave_sums(int wv, double qf, const quat& w0, double ab, const quat& rd, double cc,
-                                              double (*sh)[8]) {
+// The block sums, each wave those whose terms it holds (about a third of the
+// instructions per wave that one wave summing them all would take): wave 0 rd,
+// wave 1 wrow, wave 2 ab and cc, all waves their terms of qf.
+__device__ __forceinline__ void col_wave_sums(int wv, double qf, const quat& v4, double (*sh)[5]) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
-  if (wv == 0) {
-    double v[8] = {qf, ab, cc, rd.ar, rd.ai, rd.br, rd.bi, 0.0};
-    const double t = butterfly_sum<8>(v);
-    if ((lane & 7) == 0) sh[0][lane >> 3] = t;
-  } else if (wv == 1) {
-    double v[8] = {qf, w0.ar, w0.ai, w0.br, w0.bi, 0.0, 0.0, 0.0};
-    const double t = butterfly_sum<8>(v);
-    if ((lane & 7) == 0) sh[1][lane >> 3] = t;
-  } else {
-    const double t = wave_sum_d(qf);
-    if (lane == 0) sh[wv][0] = t;
+  if (wv < 3) {
+    double v[4] = {v4.ar, v4.ai, v4.br, v4.bi};
+    const double t = butterfly_sum<4>(v);
+    if ((lane & 15) == 0) sh[wv][lane >> 4] = t;
   }
+  qf = wave_sum_d(qf);
+  if (lane == 0) sh[wv][4] = qf;
 }
 // One thread's share of a row, over the panel columns l = q + 16 k (its
 // coefficients vv, ww): ps = gamma y - (V a + W b), us = V conj(W(s0)) + W
@@ -506,7 +497,7 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
   }
   __shared__ quat a[NBMAX], b[NBMAX], cw[NBMAX], cv[NBMAX];
   __shared__ __align__(16) double red[RB / 64][RQ][RPAD];   // wave, row, (p | column update) component
-  __shared__ double shr[RB / 64][8];
+  __shared__ double shr[RB / 64][5];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int s0 = c + 1;
@@ -530,10 +521,10 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
   // would share the scalar-load counter with the kernel arguments the gather
   // loop needs, and the loop's loads could not issue before they arrived.
   const double sv = scal[min(lane, 9)];
-  // wave 0: the panel's coefficients, lane l those of columns l + 64 h
+  // waves 0 and 2: the panel's coefficients, lane l those of columns l + 64 h
   constexpr int NH = (16 * KPT + 63) / 64;
   quat al[NH], bl[NH], cwl[NH], cvl[NH];
-  if (wv == 0)
+  if ((wv & 1) == 0)
 #pragma unroll
     for (int h = 0; h < NH; ++h) {
       al[h] = bl[h] = cwl[h] = cvl[h] = qzero();
@@ -595,15 +586,20 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
   for (int bt = 1; bt < nbt; ++bt) gather(bt);
   {
 #pragma clang fp contract(off)
-    quat rd = qzero();
-    double ab = 0.0, cc = 0.0;
+    quat v4 = w0;
     if (wv == 0) {
+      v4 = qzero();
 #pragma unroll
       for (int h = 0; h < NH; ++h) {
-        qfma(rd, cvl[h], al[h]);
-        qfma(rd, cwl[h], bl[h]);
-        ab = h ? ab + qdot(al[h], bl[h]) : qdot(al[h], bl[h]);
-        cc = h ? cc + qdot(cvl[h], cwl[h]) : qdot(cvl[h], cwl[h]);
+        qfma(v4, cvl[h], al[h]);
+        qfma(v4, cwl[h], bl[h]);
+      }
+    } else if (wv == 2) {
+      v4 = qzero();
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        v4.ar += qdot(al[h], bl[h]);
+        v4.ai += qdot(cvl[h], cwl[h]);
         const int l = lane + 64 * h;
         if (l < 16 * KPT) {   // zero beyond j
           a[l] = al[h];
@@ -613,15 +609,15 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
         }
       }
     }
-    col_wave_sums(wv, qf, w0, ab, rd, cc, shr);
+    col_wave_sums(wv, qf, v4, shr);
   }
   __syncthreads();
-  // lane t holds sum t of wave 0 (t < 8), wave 1 (t < 16); to scalar registers
-  const double st = shr[(lane >> 3) & 1][lane & 7];
-  const double qs = ((lane_d(st, 0) + lane_d(st, 8)) + shr[2][0]) + shr[3][0];
-  const ColScalars C = col_scalars(qs, lane_d(st, 1), lane_d(st, 2),
-                                   quat{lane_d(st, 3), lane_d(st, 4), lane_d(st, 5), lane_d(st, 6)},
-                                   quat{lane_d(st, 9), lane_d(st, 10), lane_d(st, 11), lane_d(st, 12)}, lane_d(sv, 0),
+  // lane 5 w + t holds sum t of wave w; to scalar registers
+  const double st = (&shr[0][0])[min(lane, 19)];
+  const double qs = ((lane_d(st, 4) + lane_d(st, 9)) + lane_d(st, 14)) + lane_d(st, 19);
+  const ColScalars C = col_scalars(qs, lane_d(st, 10), lane_d(st, 11),
+                                   quat{lane_d(st, 0), lane_d(st, 1), lane_d(st, 2), lane_d(st, 3)},
+                                   quat{lane_d(st, 5), lane_d(st, 6), lane_d(st, 7), lane_d(st, 8)}, lane_d(sv, 0),
                                    quat{lane_d(sv, 1), lane_d(sv, 2), lane_d(sv, 3), lane_d(sv, 4)},
                                    quat{lane_d(sv, 5), lane_d(sv, 6), lane_d(sv, 7), lane_d(sv, 8)}, lane_d(sv, 9));
   if (blockIdx.x == 0 && tid == 0) {   // row s0
@@ -632,15 +628,16 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
   row_share<KPT>(vv, ww, yi, C.gam, q, j, a, b, cw, cv, red[wv]);
   __syncthreads();
   RowOut o = row_finish(red, r, C, xi, ms);
-  if (q == 0 && i < n) {
-    qstore(W + i + (size_t)j * ldw, o.w);
-    qstore(M + i + (size_t)c * ld, o.u);
-    if (more) qstore(M + i + (size_t)s0 * ld, o.x);
+  // every wave has every row's results (in its lanes 0..15): one store each
+  if (lane < RQ && i < n) {
+    if (wv == 0) qstore(W + i + (size_t)j * ldw, o.w);
+    else if (wv == 1) qstore(M + i + (size_t)c * ld, o.u);
+    else if (wv == 2 && more) qstore(M + i + (size_t)s0 * ld, o.x);
   }
   if (!more) return;   // uniform
   // row s0 + 1 is the updated column's x_1: not in its tail
   if (i <= s0 + 1 || i >= n) o.x = qzero();
-  if (wv == 0) {
+  if (wv == 3) {
     double ss = qnorm2(o.x);   // lanes 0..15: the 16 rows
     ss += xlane<1>(ss);
     ss += xlane<2>(ss);
@@ -673,7 +670,7 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
 // per SIMD having nothing to hide them behind: 64 columns took 242 us, now
 // 150 us (a 2n = 128 solve 679 -> 580 us, 2n = 1024 5.94 -> 5.82 ms).
 // ---------------------------------------------------------------------------
-constexpr int TT = 1024;            // threads: 16 waves
+constexpr int TT = 512;            // threads: 16 waves
 constexpr int TWV = TT / 64;
 constexpr int TKC = TAILN / TWV;    // columns per wave
 static_assert(TAILN == 64 && TKC * TWV == TAILN, "k_tail: lane = row, TKC columns per wave");

@@ -404,7 +404,7 @@ __global__ void __launch_bounds__(256) k_merge_gather(const MergeDesc* __restric
 }
 
 // One root of f(t) = 1 + rho sum_j z_j^2 / (delta_j - t) per group of
-// LANES lanes (64, or a row of 16), which split the sum.  Origin: the nearer pole (chosen by the sign of f
+// LANES lanes (64 or 4), which split the sum.  Origin: the nearer pole (chosen by the sign of f
 // at the midpoint of the interval), so t is small and the differences
 // delta_j - t are formed without cancellation.  Iteration: Newton on the
 // pole-free G(t) = (t - p_lo)(p_hi - t) f(t), safeguarded by a bisection
@@ -419,8 +419,10 @@ __device__ __forceinline__ double lanes_sum(double v) {
   if constexpr (LANES == 64) return wave_sum_d(v);
   v += xlane<1>(v);
   v += xlane<2>(v);
-  v += xlane<4>(v);
-  v += xlane<8>(v);
+  if constexpr (LANES == 16) {
+    v += xlane<4>(v);
+    v += xlane<8>(v);
+  }
   return v;
 }
 
@@ -429,11 +431,11 @@ __device__ __forceinline__ SecSums sec_rest(const double* d, const double* z, in
                                             int plo, int phi) {
   const int lane = threadIdx.x & (LANES - 1);
   double r = 0.0, rp = 0.0;
+#pragma unroll 4
   for (int jj = lane; jj < K; jj += LANES) {
-    if (jj == plo || jj == phi) continue;
     const double zj = z[jj];
     const double inv = 1.0 / ((d[jj] - dorg) - t);
-    const double q = zj * zj * inv;
+    const double q = (jj == plo || jj == phi) ? 0.0 : zj * zj * inv;
     r += q;
     rp += q * inv;
   }
@@ -720,16 +722,19 @@ __global__ void __launch_bounds__(256) k_merge_copydefl(const MergeDesc* __restr
 constexpr int BT = 1024;
 constexpr int BQ = BASE + 1;   // column stride of Q and U in LDS (doubles)
 
-__device__ __forceinline__ void jacobi_rot(double (&A)[4][4], double (&V)[4][4], int p, int q, bool& any) {
+// The rotation that zeroes A[p][q]: c, s, and t = s / c (0 where the entry is
+// negligible).
+__device__ __forceinline__ void jacobi_angle(const double (&A)[4][4], int p, int q, double& c, double& s, double& t,
+                                             bool& any) {
   const double apq = A[p][q];
-  if (!(fabs(apq) > DEPS * (fabs(A[p][p]) + fabs(A[q][q])))) return;
-  any = true;
-  const double th = (A[q][q] - A[p][p]) / (2.0 * apq);
-  const double t = copysign(1.0 / (fabs(th) + sqrt(fma(th, th, 1.0))), th);
-  const double c = 1.0 / sqrt(fma(t, t, 1.0)), s = t * c;
-  A[p][p] = fma(-t, apq, A[p][p]);
-  A[q][q] = fma(t, apq, A[q][q]);
-  A[p][q] = A[q][p] = 0.0;
+  const bool on = fabs(apq) > DEPS * (fabs(A[p][p]) + fabs(A[q][q]));
+  const double th = (A[q][q] - A[p][p]) / (2.0 * (on ? apq : 1.0));
+  t = on ? copysign(1.0 / (fabs(th) + sqrt(fma(th, th, 1.0))), th) : 0.0;
+  c = rsqrt(fma(t, t, 1.0));
+  s = t * c;
+  any |= on;
+}
+__device__ __forceinline__ void jacobi_apply(double (&A)[4][4], double (&V)[4][4], int p, int q, double c, double s) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     if (r != p && r != q) {
@@ -741,6 +746,22 @@ __device__ __forceinline__ void jacobi_rot(double (&A)[4][4], double (&V)[4][4],
     V[r][p] = c * x - s * y;
     V[r][q] = s * x + c * y;
   }
+}
+// Two disjoint rotations: both angles first (their divisions and square roots overlap).
+__device__ __forceinline__ void jacobi_pair(double (&A)[4][4], double (&V)[4][4], int p, int q, int u, int v, bool& any) {
+  double c1, s1, t1, c2, s2, t2;
+  bool a1 = false, a2 = false;
+  jacobi_angle(A, p, q, c1, s1, t1, a1);
+  jacobi_angle(A, u, v, c2, s2, t2, a2);
+  A[p][p] = fma(-t1, A[p][q], A[p][p]);
+  A[q][q] = fma(t1, A[p][q], A[q][q]);
+  A[u][u] = fma(-t2, A[u][v], A[u][u]);
+  A[v][v] = fma(t2, A[u][v], A[v][v]);
+  if (a1) A[p][q] = A[q][p] = 0.0;
+  if (a2) A[u][v] = A[v][u] = 0.0;
+  jacobi_apply(A, V, p, q, c1, s1);
+  jacobi_apply(A, V, u, v, c2, s2);
+  any |= a1 | a2;
 }
 
 __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, double* __restrict__ lam,
@@ -799,12 +820,9 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
     }
     for (int it = 0;;) {
       bool any = false;
-      jacobi_rot(A, V, 0, 1, any);
-      jacobi_rot(A, V, 2, 3, any);
-      jacobi_rot(A, V, 0, 2, any);
-      jacobi_rot(A, V, 1, 3, any);
-      jacobi_rot(A, V, 0, 3, any);
-      jacobi_rot(A, V, 1, 2, any);
+      jacobi_pair(A, V, 0, 1, 2, 3, any);
+      jacobi_pair(A, V, 0, 2, 1, 3, any);
+      jacobi_pair(A, V, 0, 3, 1, 2, any);
       if (!any) break;
       if (++it >= cap_leaf) { fail = 1; break; }
     }
@@ -951,13 +969,17 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
         *qp = ro[2] * x + ro[3] * y;
         *qj = ro[2] * y - ro[3] * x;
       }
-    if (row < K) {
-      const SecRoot R = secular_root<16>(rho, cap_sec, K, row, dkk + lo, zkk + lo);
-      if (sub == 0) {
-        org[lo + row] = R.org;
-        tau[lo + row] = R.t;
-        val[lo + row] = dkk[lo + R.org] + R.t;
-        if (!R.conv) atomicMax(info + pr, lo0 - ob + lo + row + 1);
+    // 4 lanes per root, so the 64 roots of a level are one wave per SIMD: with
+    // 16 the four waves' shares of the scalar work of a step, the same in every
+    // lane, took longer than the shorter sums saved
+    const int root = tt >> 2;
+    if (tt < ts / 4 && root < K) {
+      const SecRoot R = secular_root<4>(rho, cap_sec, K, root, dkk + lo, zkk + lo);
+      if ((tt & 3) == 0) {
+        org[lo + root] = R.org;
+        tau[lo + root] = R.t;
+        val[lo + root] = dkk[lo + R.org] + R.t;
+        if (!R.conv) atomicMax(info + pr, lo0 - ob + lo + root + 1);
       }
     }
     __syncthreads();
