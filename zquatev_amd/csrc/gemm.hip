@@ -40,6 +40,9 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 // The tile shape changes no result: an element's K-sum is one wave's
 // accumulator in the same order in every shape.
 //   64 x 64, GBK 8    the most reuse per fetch, for launches of very many tiles;
+//                     waves of 16 x 64 read 8 fragments per 16 MFMAs where 32 x 32
+//                     ones read 10 (4096 x 4096 x 1024 66.3 -> 67.3 TFLOP/s, and
+//                     65.5 before the loads became branch-free, below);
 //   32 x 64, GBK 8    twice the workgroups (balance, registers);
 //   16 x 32, GBK 16   for launches that leave CUs idle otherwise: a wave's time
 //                     is K x (its 16 x 16 x 4 products) x 64 cycles whatever
@@ -48,9 +51,9 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 //                     cycles at GBK 8) would wait for the next fetch, hence 16.
 //                     C is fetched before the K loop.
 // ---------------------------------------------------------------------------
-template <int TBM_, int TBN_, int GBK_>
+template <int TBM_, int TBN_, int GBK_, int WM_>
 struct QTile {
-  static constexpr int TBM = TBM_, TBN = TBN_, GBK = GBK_;
+  static constexpr int TBM = TBM_, TBN = TBN_, GBK = GBK_, WM = WM_;   // WM of the 4 waves along the rows
   // LDS layouts (doubles).  A: [k][row][component], B: [k][component][column],
   // each k slice padded by 2 doubles, so that fragment reads (16 consecutive
   // doubles per component group) and the stage writes of either operand
@@ -58,34 +61,32 @@ struct QTile {
   static constexpr int ASK = TBM * 4 + 2, BSK = TBN * 4 + 2;
   static constexpr bool PREC = TBM == 16;   // C fetched before the K loop
 };
-using Tile64 = QTile<64, 64, 8>;
-using Tile32 = QTile<32, 64, 8>;
-using Tile16 = QTile<16, 32, 16>;
+using Tile64 = QTile<64, 64, 8, 4>;
+using Tile32 = QTile<32, 64, 8, 2>;
+using Tile16 = QTile<16, 32, 16, 2>;
 
-// Operand elements as stored.  The conjugation of a CT operand is applied
-// when the stage is stashed in LDS, after the current stage's MFMAs: sign
-// flips here, on the freshly loaded registers, would make every prefetch
-// wait for its own data before those MFMAs could start.
-template <bool CT>
-__device__ __forceinline__ quat ld_opA(const QOperand& A, int i, int k, int m, int K) {
-  if (i >= m || k >= K) return qzero();
-  const quat* p = A.p0;
-  int ldp = A.ld0, kk = k;
-  if (k >= A.ksplit) { p = A.p1; ldp = A.ld1; kk = k - A.ksplit; }
-  const int sr = CT ? kk : i, sc = CT ? i : kk;
-  if (!(sr > sc + A.mask_off)) return qzero();
-  return qload_g(p + sr + (size_t)sc * ldp);
+// Operand elements as stored, loaded without a branch at a clamped index (row
+// or column i of the output, 0 <= i < m; k of the sum, within the range): a
+// load in a branch is followed by a wait for it, before the current stage's
+// MFMAs could start (128 x 4096 x 4096 with A transposed 53.2 -> 55.4
+// TFLOP/s, 2n = 8192 solve 147.1 -> 146.1 ms).  What is out of range or masked becomes zero, and a CT operand is
+// conjugated, when the stage is stashed in LDS, after those MFMAs.  A and B
+// are indexed alike: storage element (i, k), for A conj-transposed and plain B (k, i).
+template <bool KROW>
+__device__ __forceinline__ quat ld_op(const QOperand& A, int i, int k) {
+  const bool second = k >= A.ksplit;
+  const quat* p = second ? A.p1 : A.p0;
+  const int ld = second ? A.ld1 : A.ld0, kk = second ? k - A.ksplit : k;
+  return qload_g(p + (KROW ? kk : i) + (size_t)(KROW ? i : kk) * ld);
 }
-
-template <bool CT>
-__device__ __forceinline__ quat ld_opB(const QOperand& B, int k, int j, int K, int nn) {
-  if (k >= K || j >= nn) return qzero();
-  const quat* p = B.p0;
-  int ldp = B.ld0, kk = k;
-  if (k >= B.ksplit) { p = B.p1; ldp = B.ld1; kk = k - B.ksplit; }
-  const int sr = CT ? j : kk, sc = CT ? kk : j;
-  if (!(sr > sc + B.mask_off)) return qzero();
-  return qload_g(p + sr + (size_t)sc * ldp);
+// Whether that element counts: storage (r, c) is used only where r > c + mask_off.
+template <bool KROW>
+__device__ __forceinline__ bool op_on(const QOperand& A, int i, int k) {
+  const int kk = k >= A.ksplit ? k - A.ksplit : k;
+  return KROW ? kk > i + A.mask_off : i > kk + A.mask_off;
+}
+__device__ __forceinline__ quat qselect(bool on, const quat& v) {
+  return quat{on ? v.ar : 0.0, on ? v.ai : 0.0, on ? v.br : 0.0, on ? v.bi : 0.0};
 }
 
 __device__ __forceinline__ double flip_sign(double v, unsigned mask) {
@@ -97,15 +98,16 @@ __device__ __forceinline__ void qgemm2_tile(const QGemmTask& t, int row0, int co
   constexpr int TBM = T::TBM, TBN = T::TBN, GBK = T::GBK;
   constexpr int AH = TBM * GBK / 256;   // A stage elements per thread
   constexpr int BH = TBN * GBK / 256;   // B stage elements per thread
-  constexpr int WR = TBM / 2, WC = TBN / 2;   // quaternion rows and columns per wave
+  constexpr int WM = T::WM, WN = 4 / WM;
+  constexpr int WR = TBM / WM, WC = TBN / WN;   // quaternion rows and columns per wave
   constexpr int NA = WR / 4, NBC = WC / 16;   // MFMA accumulators per wave: NA x NBC
   static_assert(AH * 256 == TBM * GBK && BH * 256 == TBN * GBK && NA * 4 == WR && NBC * 16 == WC, "tile shape");
-  const int m = t.m, nn = t.nn, K = t.K;
+  const int m = t.m, nn = t.nn;
   __shared__ double As[2][GBK * T::ASK];
   __shared__ double Bs[2][GBK * T::BSK];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
-  const int wr = wv >> 1, wc = wv & 1;   // wave tile: rows wr*WR..+WR, cols wc*WC..+WC (quaternions)
+  const int wr = wv / WN, wc = wv % WN;   // wave tile: rows wr*WR..+WR, cols wc*WC..+WC (quaternions)
   const int cr = (lane & 15) >> 2, ck = lane >> 4;
   const int acomp = cr ^ ck;
   const unsigned smask = ((0x428E >> (cr * 4 + ck)) & 1) ? 0x80000000u : 0u;
@@ -127,27 +129,23 @@ __device__ __forceinline__ void qgemm2_tile(const QGemmTask& t, int row0, int co
   quat ra[AH], rb[BH];
   auto fetch = [&](int k0) {
 #pragma unroll
-    for (int h = 0; h < AH; ++h) {
-      const int ka = k0 + ak[h];
-      ra[h] = (ka < kend) ? ld_opA<ACT>(t.A, row0 + ai[h], ka, m, K) : qzero();
-    }
+    for (int h = 0; h < AH; ++h) ra[h] = ld_op<ACT>(t.A, min(row0 + ai[h], m - 1), min(k0 + ak[h], kend - 1));
 #pragma unroll
-    for (int h = 0; h < BH; ++h) {
-      const int kb = k0 + bk[h];
-      rb[h] = (kb < kend) ? ld_opB<BCT>(t.B, kb, col0 + bjj[h], K, nn) : qzero();
-    }
+    for (int h = 0; h < BH; ++h) rb[h] = ld_op<!BCT>(t.B, min(col0 + bjj[h], nn - 1), min(k0 + bk[h], kend - 1));
   };
-  auto stash = [&](int buf) {
+  auto stash = [&](int buf, int k0) {
 #pragma unroll
     for (int h = 0; h < AH; ++h) {
-      const quat a = ACT ? qconj(ra[h]) : ra[h];
+      const int i = row0 + ai[h], k = k0 + ak[h];
+      const quat a = qselect(i < m && k < kend && op_on<ACT>(t.A, i, k), ACT ? qconj(ra[h]) : ra[h]);
       double2* pa = reinterpret_cast<double2*>(&As[buf][ak[h] * T::ASK + ai[h] * 4]);
       pa[0] = make_double2(a.ar, a.ai);
       pa[1] = make_double2(a.br, a.bi);
     }
 #pragma unroll
     for (int h = 0; h < BH; ++h) {
-      const quat bv = BCT ? qconj(rb[h]) : rb[h];
+      const int j = col0 + bjj[h], k = k0 + bk[h];
+      const quat bv = qselect(j < nn && k < kend && op_on<!BCT>(t.B, j, k), BCT ? qconj(rb[h]) : rb[h]);
       double* pb = &Bs[buf][bk[h] * T::BSK + bjj[h]];
       pb[0] = bv.ar;
       pb[TBN] = bv.ai;
@@ -180,7 +178,7 @@ __device__ __forceinline__ void qgemm2_tile(const QGemmTask& t, int row0, int co
   int cur = 0;
   if (kbeg < kend) {
     fetch(kbeg);
-    stash(0);
+    stash(0, kbeg);
   }
   __syncthreads();
   for (int k0 = kbeg; k0 < kend; k0 += GBK) {
@@ -199,7 +197,7 @@ __device__ __forceinline__ void qgemm2_tile(const QGemmTask& t, int row0, int co
         for (int b = 0; b < NBC; ++b)
           acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[a], bf[b], acc[a][b], 0, 0, 0);
     }
-    if (more) stash(cur ^ 1);
+    if (more) stash(cur ^ 1, k0 + GBK);
     __syncthreads();
     cur ^= 1;
   }
