@@ -230,11 +230,13 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
       int kchunk = 0;
       const int nz = splitk_count(k.mr, w.nsplit, &kchunk);
       if ((size_t)(b + 1) * w.nsplit * wbt * wbt > w.part_slots) return ZQI_ERR_ARG;
+      quat* Gb = at(w.G, z) + (size_t)b * wbt * wbt;
       for (int q = 0; q < nz; ++q) {
         const int kb = q * kchunk, ke = std::min(k.mr, kb + kchunk);
-        tt.push_back(QGemmTask{k.wdt, k.wdt, k.mr, kb, ke, wbt, 0, 1.0, 0.0, Vc, Vn, part + (size_t)q * wbt * wbt});
+        quat* out = nz > 1 ? part + (size_t)q * wbt * wbt : Gb;
+        tt.push_back(QGemmTask{k.wdt, k.wdt, k.mr, kb, ke, wbt, 0, 1.0, 0.0, Vc, Vn, out});
       }
-      ss.push_back(SumTask{part, at(w.G, z) + (size_t)b * wbt * wbt, wbt * wbt, nz});
+      if (nz > 1) ss.push_back(SumTask{part, Gb, wbt * wbt, nz});
       gmaxk = std::max(gmaxk, k.wdt);
     }
   const int ngt = (int)tt.size() - gt0;
@@ -316,9 +318,10 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
       if ((size_t)nz * k.wdt * n > w.part_slots) return ZQI_ERR_ARG;
       for (int c = 0; c < nz; ++c) {
         const int kb = c * kchunk, ke = std::min(k.mr, kb + kchunk);
-        tt.push_back(QGemmTask{k.wdt, n, k.mr, kb, ke, k.wdt, 0, 1.0, 0.0, VTc, Xo, part + (size_t)c * k.wdt * n});
+        quat* out = nz > 1 ? part + (size_t)c * k.wdt * n : Y;
+        tt.push_back(QGemmTask{k.wdt, n, k.mr, kb, ke, k.wdt, 0, 1.0, 0.0, VTc, Xo, out});
       }
-      ss.push_back(SumTask{part, Y, k.wdt * n, nz});
+      if (nz > 1) ss.push_back(SumTask{part, Y, k.wdt * n, nz});
       QOperand Vn{V, V, ld, ld, INT_MAX, false, -1};
       QOperand Yo{Y, Y, k.wdt, k.wdt, INT_MAX, false, INT_MIN / 2};
       tx.push_back(QGemmTask{k.mr, n, k.wdt, 0, k.wdt, ldx, 0, -1.0, 1.0, Vn, Yo, Xz + k.r0});
@@ -340,11 +343,11 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
       ss.size() > backtransform_batched_sums(nprob, nh, wbt))
     return ZQI_ERR_ARG;
   int rc = stage_upload(st, tt.data(), tt.size() * sizeof(QGemmTask), tasks, s);
-  if (!rc) rc = stage_upload(st, ss.data(), ss.size() * sizeof(SumTask), sums, s);
+  if (!rc && !ss.empty()) rc = stage_upload(st, ss.data(), ss.size() * sizeof(SumTask), sums, s);
   if (rc) return rc;
   // phase A launches
   if ((rc = qgemm_tasks(tasks + gt0, ngt, gmaxk, gmaxk, true, false, false, s))) return rc;
-  hipLaunchKernelGGL(k_sum_parts_b, dim3(cdiv(wbt * wbt, 256), 1, ngs), dim3(256), 0, s, sums);
+  if (ngs > 0) hipLaunchKernelGGL(k_sum_parts_b, dim3(cdiv(wbt * wbt, 256), 1, ngs), dim3(256), 0, s, sums);
   if (wbt < TF_WB || wbt % TF_WB || (tsub & (tsub - 1))) return ZQI_ERR_ARG;
   hipLaunchKernelGGL(k_tfactor, dim3(nblk * tsub, 1, nprob), dim3(TF_T), 0, s, L, w.G, w.T, tsub, zb);
   for (size_t li = 0; li < levels.size(); ++li) {
@@ -359,7 +362,8 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
       ProfScope ps(PROF_BACKTR, s, q.fy);
       if ((rc = qgemm_tasks(tasks + q.y0, q.ny, q.maxw, q.maxn, true, false, false, s))) return rc;
     }
-    hipLaunchKernelGGL(k_sum_parts_b, dim3(cdiv(q.maxtot, 256), 1, q.ns), dim3(256), 0, s, sums + q.s0);
+    if (q.ns > 0)
+      hipLaunchKernelGGL(k_sum_parts_b, dim3(cdiv(q.maxtot, 256), 1, q.ns), dim3(256), 0, s, sums + q.s0);
     {
       ProfScope ps(PROF_BACKTR, s, q.fx);
       if ((rc = qgemm_tasks(tasks + q.x0, q.nx, q.maxmr, q.maxn, false, false, false, s))) return rc;

@@ -24,6 +24,7 @@
 // (zquatev.cc:86-90).
 #include "zq_internal.h"
 #include <climits>
+#include <algorithm>
 
 namespace zq {
 
@@ -355,7 +356,10 @@ int qgemm_tasks(const QGemmTask* tasks_dev, int ntasks, int maxm, int maxnn, boo
                 hipStream_t s) {
   if (ntasks <= 0 || maxm <= 0 || maxnn <= 0) return ZQI_OK;
   const int n64 = tile_count<Tile64>(maxm, maxnn, lower), n32 = tile_count<Tile32>(maxm, maxnn, lower);
-  switch (tile_rows((long)n64 * ntasks, (long)n32 * ntasks)) {
+  // 64-row tiles by the largest task alone: many smaller ragged tasks lose more
+  // to the padding of their edges than the larger tiles save (the 512-problem
+  // batch 70.3 ms counting all tasks' tiles, 68.8 ms so)
+  switch (tile_rows((long)n64, (long)n32 * ntasks)) {
     case 64: launch_gemm2_batch_t<Tile64>(act, bct, dim3(n64, 1, ntasks), s, tasks_dev); break;
     case 32: launch_gemm2_batch_t<Tile32>(act, bct, dim3(n32, 1, ntasks), s, tasks_dev); break;
     default:
@@ -364,12 +368,15 @@ int qgemm_tasks(const QGemmTask* tasks_dev, int ntasks, int maxm, int maxnn, boo
   return hipGetLastError() == hipSuccess ? ZQI_OK : ZQI_ERR_HIP;
 }
 
-constexpr int KCHUNK = 8;   // split-K chunks are multiples of this
+// Split-K chunks: multiples of KCHUNK, and not shorter than KCHUNK_MIN: below
+// that the partials' traffic and the launch that sums them cost more than the
+// split saves (batch of 512 problems 74.7 ms with chunks from 16, 74.1 from 64,
+// 73.5 from 128; 2n = 510 solve 2.03, 2.03, 2.05 ms).
+constexpr int KCHUNK = 16, KCHUNK_MIN = 64;
 int splitk_count(int K, int nsplit, int* kchunk_out) {
   if (nsplit < 1) nsplit = 1;
   int kchunk = (K + nsplit - 1) / nsplit;
-  kchunk = ((kchunk + KCHUNK - 1) / KCHUNK) * KCHUNK;
-  if (kchunk < KCHUNK) kchunk = KCHUNK;
+  kchunk = std::max(((kchunk + KCHUNK - 1) / KCHUNK) * KCHUNK, KCHUNK_MIN);
   if (kchunk_out) *kchunk_out = kchunk;
   const int nz = (K + kchunk - 1) / kchunk;
   return nz > 0 ? nz : 1;

@@ -659,18 +659,19 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
 // conventions).
 //
 // The whole Hermitian block (both triangles) is held in registers: lane = row,
-// and wave v owns columns v, v + 16, v + 32, v + 48 (cyclic, so that the waves
-// stay evenly loaded as columns retire).  The matrix is never re-read: per
+// and wave v owns columns v, v + 8, ... (cyclic, so that the waves stay
+// evenly loaded as columns retire).  The matrix is never re-read: per
 // column only u, w (broadcast reads) and the waves' partials of y pass
-// through LDS, with three barriers.  Wave cl % 16 owns column cl, so after the
+// through LDS, with three barriers.  Wave cl % 8 owns column cl, so after the
 // update of column cl - 1 it forms the next reflector from its own registers
 // while the other waves are still updating.  Retired and absent rows and
 // columns have u = w = 0, so no lane masks are needed.  A version with the
 // block in LDS and four waves was bound by its re-reads of the block, one wave
 // per SIMD having nothing to hide them behind: 64 columns took 242 us, now
-// 150 us (a 2n = 128 solve 679 -> 580 us, 2n = 1024 5.94 -> 5.82 ms).
+// 138 us (149 with 16 waves, 140 with 4; 149 with the stages in one rolled
+// loop, although that quarters the code).
 // ---------------------------------------------------------------------------
-constexpr int TT = 512;            // threads: 16 waves
+constexpr int TT = 512;            // threads: 8 waves
 constexpr int TWV = TT / 64;
 constexpr int TKC = TAILN / TWV;    // columns per wave
 static_assert(TAILN == 64 && TKC * TWV == TAILN, "k_tail: lane = row, TKC columns per wave");

@@ -11,8 +11,8 @@
 // Tree: halve until a block has at most BASE rows; each split point s couples
 // rows s-1 and s with beta = e[s-1] >= 0, and T = diag(T1', T2') + beta v v^T,
 // v = e_{s-1} + e_s, where T1', T2' have beta subtracted from the touching
-// diagonal entries.  A base block runs its whole divide & conquer (leaves of <=
-// 4 rows, then merges) in one workgroup (k_dc_base); the merges above run
+// diagonal entries.  A base block runs its whole divide & conquer (leaves of 1 or
+// 2 rows, then merges) in one workgroup (k_dc_base); the merges above run
 // level by level (all merges of a level in one launch):
 //   prep   : stable merge of the two sorted spectra, z = [last row of Q1;
 //            first row of Q2]/sqrt(2), rho = 2 beta, deflation scan (small
@@ -404,7 +404,7 @@ __global__ void __launch_bounds__(256) k_merge_gather(const MergeDesc* __restric
 }
 
 // One root of f(t) = 1 + rho sum_j z_j^2 / (delta_j - t) per group of
-// LANES lanes (64 or 4), which split the sum.  Origin: the nearer pole (chosen by the sign of f
+// LANES lanes (64, or a row of 16), which split the sum.  Origin: the nearer pole (chosen by the sign of f
 // at the midpoint of the interval), so t is small and the differences
 // delta_j - t are formed without cancellation.  Iteration: Newton on the
 // pole-free G(t) = (t - p_lo)(p_hi - t) f(t), safeguarded by a bisection
@@ -419,10 +419,8 @@ __device__ __forceinline__ double lanes_sum(double v) {
   if constexpr (LANES == 64) return wave_sum_d(v);
   v += xlane<1>(v);
   v += xlane<2>(v);
-  if constexpr (LANES == 16) {
-    v += xlane<4>(v);
-    v += xlane<8>(v);
-  }
+  if constexpr (LANES >= 8) v += xlane<4>(v);
+  if constexpr (LANES >= 16) v += xlane<8>(v);
   return v;
 }
 
@@ -431,7 +429,8 @@ __device__ __forceinline__ SecSums sec_rest(const double* d, const double* z, in
                                             int plo, int phi) {
   const int lane = threadIdx.x & (LANES - 1);
   double r = 0.0, rp = 0.0;
-#pragma unroll 4
+  constexpr int UNR = LANES == 64 ? 4 : 1;   // a row of 16 has at most 4 terms per lane
+#pragma unroll UNR
   for (int jj = lane; jj < K; jj += LANES) {
     const double zj = z[jj];
     const double inv = 1.0 / ((d[jj] - dorg) - t);
@@ -528,11 +527,15 @@ __device__ __forceinline__ SecRoot secular_root(double rho, int cap, int K, int 
     }
     if (G == 0.0) { a = b = t; conv = true; break; }
     if (G < 0.0) a = t; else b = t;
-    // A Newton correction below the stopping size ends the iteration before
-    // the bracket test: t is an end of the bracket now, and t - dt can round
-    // onto it, which must not be taken for a step out of the bracket.
+    // A Newton correction below 1e-9 of t is the last one.  Newton converges
+    // quadratically here, and G varies on the scale of the distances to the
+    // poles, of which t is the smallest, so the next correction would be of the
+    // order 1e-18 of t (replayed over real merges: 3.5 steps per root instead of
+    // 4.4 and at most 12 instead of 46, f at the roots equally small).  The test
+    // comes before the bracket's: t is an end of the bracket now, and t - dt can
+    // round onto it, which must not be taken for a step out of the bracket.
     const double dt = G / Gp;
-    if (fabs(dt) <= 4.0 * DEPS * fabs(t)) {
+    if (fabs(dt) <= 1e-9 * fabs(t)) {
       const double tc = t - dt;
       if (tc >= a && tc <= b) t = tc;
       conv = true;
@@ -701,10 +704,10 @@ __global__ void __launch_bounds__(256) k_merge_copydefl(const MergeDesc* __restr
 
 // --------------------------------------------------------------------------
 // base block: the divide & conquer of up to BASE rows in one workgroup, with
-// the eigenvectors Q in LDS.  The block is halved D = 0 .. 4 times into 2^D
-// leaves of at most 4 rows (all at the same depth, since sizes at a depth
-// differ by at most one), each solved by cyclic Jacobi in one thread's
-// registers; then D levels of merges, the 2^k merges of a level side by side,
+// the eigenvectors Q in LDS.  The block is halved D = 0 .. 5 times into 2^D
+// leaves of 1 or 2 rows (all at the same depth, since sizes at a depth
+// differ by at most one), each diagonalised by a Jacobi rotation in one
+// thread; then D levels of merges, the 2^k merges of a level side by side,
 // each by a team of 1024 >> k threads, 16 threads per row.  A merge is the
 // algorithm of the merge kernels above (rank, deflate, secular roots, zhat, U, product).
 // Instead of gathering the kept columns of Q, the rows of U are scattered to
@@ -714,55 +717,14 @@ __global__ void __launch_bounds__(256) k_merge_copydefl(const MergeDesc* __restr
 //
 // One launch where leaves of 16 rows by QL (one wavefront each, a serial chain
 // of ~220 rotations: 151 us) and ten launches per level took 245 us for 64
-// rows, now 85 us with the
-// kernels around it (2n = 128 solve 540 -> 378 us, 510 2.29 -> 2.11 ms, 1024
-// 4.65 -> 4.52 ms).
+// rows, with the kernels around them; now 82 us (2n = 128 solve 540 -> 364 us, 510
+// 2.29 -> 2.09 ms, 1024 4.65 -> 4.50 ms).  Most of it is the secular steps (8 or so
+// of the slowest root, ~190 instructions each on every wave): 16 lanes per root
+// beat 8 and 4 (88, 90, 105 us), which leave one wave per SIMD its latencies.
 // A leaf is (lo, hi, problem base, problem index).
 // --------------------------------------------------------------------------
 constexpr int BT = 1024;
 constexpr int BQ = BASE + 1;   // column stride of Q and U in LDS (doubles)
-
-// The rotation that zeroes A[p][q]: c, s, and t = s / c (0 where the entry is
-// negligible).
-__device__ __forceinline__ void jacobi_angle(const double (&A)[4][4], int p, int q, double& c, double& s, double& t,
-                                             bool& any) {
-  const double apq = A[p][q];
-  const bool on = fabs(apq) > DEPS * (fabs(A[p][p]) + fabs(A[q][q]));
-  const double th = (A[q][q] - A[p][p]) / (2.0 * (on ? apq : 1.0));
-  t = on ? copysign(1.0 / (fabs(th) + sqrt(fma(th, th, 1.0))), th) : 0.0;
-  c = rsqrt(fma(t, t, 1.0));
-  s = t * c;
-  any |= on;
-}
-__device__ __forceinline__ void jacobi_apply(double (&A)[4][4], double (&V)[4][4], int p, int q, double c, double s) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    if (r != p && r != q) {
-      const double x = A[r][p], y = A[r][q];
-      A[r][p] = A[p][r] = c * x - s * y;
-      A[r][q] = A[q][r] = s * x + c * y;
-    }
-    const double x = V[r][p], y = V[r][q];
-    V[r][p] = c * x - s * y;
-    V[r][q] = s * x + c * y;
-  }
-}
-// Two disjoint rotations: both angles first (their divisions and square roots overlap).
-__device__ __forceinline__ void jacobi_pair(double (&A)[4][4], double (&V)[4][4], int p, int q, int u, int v, bool& any) {
-  double c1, s1, t1, c2, s2, t2;
-  bool a1 = false, a2 = false;
-  jacobi_angle(A, p, q, c1, s1, t1, a1);
-  jacobi_angle(A, u, v, c2, s2, t2, a2);
-  A[p][p] = fma(-t1, A[p][q], A[p][p]);
-  A[q][q] = fma(t1, A[p][q], A[q][q]);
-  A[u][u] = fma(-t2, A[u][v], A[u][u]);
-  A[v][v] = fma(t2, A[u][v], A[v][v]);
-  if (a1) A[p][q] = A[q][p] = 0.0;
-  if (a2) A[u][v] = A[v][u] = 0.0;
-  jacobi_apply(A, V, p, q, c1, s1);
-  jacobi_apply(A, V, u, v, c2, s2);
-  any |= a1 | a2;
-}
 
 __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, double* __restrict__ lam,
                                                 const double* __restrict__ es, double* __restrict__ Z, int ldz,
@@ -775,13 +737,13 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
   __shared__ double tau[BASE], zh[BASE], val[BASE];
   __shared__ double rot[4 * BASE];
   __shared__ int src[BASE], keep[BASE], dfl[BASE], org[BASE], pos[BASE];   // pos: by column of Q
-  __shared__ int sK[8], snr[8];
-  __shared__ int bnd[17];
+  __shared__ int sK[16], snr[16];
+  __shared__ int bnd[33];
   const int lo0 = leaves[4 * blockIdx.x], m = leaves[4 * blockIdx.x + 1] - lo0;
   const int ob = leaves[4 * blockIdx.x + 2], pr = leaves[4 * blockIdx.x + 3];
   const int tid = threadIdx.x, lane = tid & 63;
   int D = 0;
-  while ((4 << D) < m) ++D;
+  while ((2 << D) < m) ++D;
   if (tid < m) sl[tid] = lam[lo0 + tid];
   if (tid < m - 1) se[tid] = es[lo0 + tid];
   if (tid <= (1 << D)) {   // leaf boundary: follow the bits from the top
@@ -798,53 +760,36 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
   __syncthreads();
   // ---- leaves
   if (tid < (1 << D)) {
-    const int a = bnd[tid], sz = bnd[tid + 1] - a;
-    double A[4][4], V[4][4];
+    const int a = bnd[tid], sz = bnd[tid + 1] - a;   // 1 or 2 rows
     int fail = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        A[i][j] = 0.0;
-        V[i][j] = i == j ? 1.0 : 0.0;
-      }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (i < sz) {
-        double v = sl[a + i];   // torn at the splits inside the base block
-        if (i == 0 && a > 0) v -= se[a - 1];
-        if (i == sz - 1 && a + sz < m) v -= se[a + sz - 1];
-        A[i][i] = v;
-      }
-      if (i < 3 && i + 1 < sz) A[i][i + 1] = A[i + 1][i] = se[a + i];
+    // torn at the splits inside the base block
+    const double tl = a > 0 ? se[a - 1] : 0.0, tr = a + sz < m ? se[a + sz - 1] : 0.0;
+    double p = sl[a] - tl, q = 0.0, r = 0.0, c = 1.0, s = 0.0;   // [p r; r q] and its vectors (c, -s), (s, c)
+    if (sz == 1) p -= tr;
+    if (sz == 2) {
+      q = sl[a + 1] - tr;
+      r = se[a];
     }
-    for (int it = 0;;) {
-      bool any = false;
-      jacobi_pair(A, V, 0, 1, 2, 3, any);
-      jacobi_pair(A, V, 0, 2, 1, 3, any);
-      jacobi_pair(A, V, 0, 3, 1, 2, any);
-      if (!any) break;
+    // Jacobi: one rotation makes the off-diagonal entry 0
+    for (int it = 0; fabs(r) > DEPS * (fabs(p) + fabs(q));) {
+      const double th = (q - p) / (2.0 * r);
+      const double t = copysign(1.0 / (fabs(th) + sqrt(fma(th, th, 1.0))), th);
+      c = rsqrt(fma(t, t, 1.0));
+      s = t * c;
+      p = fma(-t, r, p);
+      q = fma(t, r, q);
+      r = 0.0;
       if (++it >= cap_leaf) { fail = 1; break; }
     }
-    double w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = i < sz ? A[i][i] : DBL_MAX;   // absent rows stay last
-    auto order = [&](int i, int j) {
-      if (w[j] < w[i]) {
-        double t = w[i]; w[i] = w[j]; w[j] = t;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) { t = V[r][i]; V[r][i] = V[r][j]; V[r][j] = t; }
-      }
-    };
-    order(0, 1); order(2, 3); order(0, 2); order(1, 3); order(1, 2);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j < sz) {
-        sl[a + j] = w[j];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (r < sz) Q[(a + j) * BQ + a + r] = V[r][j];
-      }
+    const bool sw = sz == 2 && q < p;   // ascending
+    sl[a] = sw ? q : p;
+    Q[a * BQ + a] = sw ? s : c;
+    if (sz == 2) {
+      sl[a + 1] = sw ? p : q;
+      Q[a * BQ + a + 1] = sw ? c : -s;
+      Q[(a + 1) * BQ + a] = sw ? c : s;
+      Q[(a + 1) * BQ + a + 1] = sw ? -s : c;
+    }
     if (fail) atomicMax(info + pr, lo0 - ob + a + 1);
   }
   __syncthreads();
@@ -895,7 +840,7 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
       const double zp = __shfl(zl, pv, 64), dp = __shfl(dl, pv, 64);
       bool rotates = false;
       if (kept && (km & below)) {
-        const double h = hypot(zl, zp);
+        const double h = sqrt(zl * zl + zp * zp);   // neither is below 8 roundoffs of the largest z
         rotates = fabs((dl - dp) * (zl / h) * (-zp / h)) <= tol;
       }
       if (!__any(rotates)) {
@@ -926,7 +871,7 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
           }
           if (pj < 0) { pj = j; continue; }
           double s = z[pj], c = z[j];
-          const double h = hypot(c, s);
+          const double h = sqrt(c * c + s * s);
           const double t = d[j] - d[pj];
           c /= h;
           s = -s / h;
@@ -969,17 +914,13 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
         *qp = ro[2] * x + ro[3] * y;
         *qj = ro[2] * y - ro[3] * x;
       }
-    // 4 lanes per root, so the 64 roots of a level are one wave per SIMD: with
-    // 16 the four waves' shares of the scalar work of a step, the same in every
-    // lane, took longer than the shorter sums saved
-    const int root = tt >> 2;
-    if (tt < ts / 4 && root < K) {
-      const SecRoot R = secular_root<4>(rho, cap_sec, K, root, dkk + lo, zkk + lo);
-      if ((tt & 3) == 0) {
-        org[lo + root] = R.org;
-        tau[lo + root] = R.t;
-        val[lo + root] = dkk[lo + R.org] + R.t;
-        if (!R.conv) atomicMax(info + pr, lo0 - ob + lo + root + 1);
+    if (row < K) {
+      const SecRoot R = secular_root<16>(rho, cap_sec, K, row, dkk + lo, zkk + lo);
+      if (sub == 0) {
+        org[lo + row] = R.org;
+        tau[lo + row] = R.t;
+        val[lo + row] = dkk[lo + R.org] + R.t;
+        if (!R.conv) atomicMax(info + pr, lo0 - ob + lo + row + 1);
       }
     }
     __syncthreads();
@@ -988,7 +929,7 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
       double prod = 1.0;
       for (int i = sub; i < K; i += 16) {
         const double num = (dkk[lo + org[lo + i]] - dj) + tau[lo + i];
-        prod *= (i == row) ? num / rho : num / (dkk[lo + i] - dj);
+        prod *= num / (i == row ? rho : dkk[lo + i] - dj);
       }
 #pragma unroll
       for (int b = 1; b < 16; b <<= 1) prod *= __shfl_xor(prod, b, 16);
