@@ -352,14 +352,21 @@ int qgemm(int m, int nn, int k, double alpha, const QOperand& A, const QOperand&
   return hipGetLastError() == hipSuccess ? ZQI_OK : ZQI_ERR_HIP;
 }
 
-int qgemm_tasks(const QGemmTask* tasks_dev, int ntasks, int maxm, int maxnn, bool act, bool bct, bool lower,
+// Task lists whose every sum is at least LONG_K long take 64-row tiles already
+// from two per CU, where they all run at once: the back-transform's Y products at
+// n >= 4096 (1024 32-row tiles make one and a third rounds of three per CU, 512
+// 64-row ones one round of two; 2n = 8192 back-transform 39.3 -> 38.4 ms).
+constexpr int LONG_K = 384;
+int qgemm_tasks(const QGemmTask* tasks_dev, int ntasks, int maxm, int maxnn, int kmin, bool act, bool bct, bool lower,
                 hipStream_t s) {
   if (ntasks <= 0 || maxm <= 0 || maxnn <= 0) return ZQI_OK;
   const int n64 = tile_count<Tile64>(maxm, maxnn, lower), n32 = tile_count<Tile32>(maxm, maxnn, lower);
   // 64-row tiles by the largest task alone: many smaller ragged tasks lose more
   // to the padding of their edges than the larger tiles save (the 512-problem
   // batch 70.3 ms counting all tasks' tiles, 68.8 ms so)
-  switch (tile_rows((long)n64, (long)n32 * ntasks)) {
+  int rows = tile_rows((long)n64, (long)n32 * ntasks);
+  if (rows == 32 && kmin >= LONG_K && (long)n64 * ntasks >= 2L * device_cus()) rows = 64;
+  switch (rows) {
     case 64: launch_gemm2_batch_t<Tile64>(act, bct, dim3(n64, 1, ntasks), s, tasks_dev); break;
     case 32: launch_gemm2_batch_t<Tile32>(act, bct, dim3(n32, 1, ntasks), s, tasks_dev); break;
     default:
