@@ -468,7 +468,6 @@ int solve_device(zq_context* ctx, int n, double* dD, int ld2, double* deig, bool
   if ((rc = zq::load_left_half(n, dD, ld2, p.M, p.ldm, p.sw.info, s))) return rc;
   ZQ_HIP_CHECK(mark(1));
   if ((rc = zq::reduce(p.M, n, p.ldm, nb, p.d, p.e, p.rw, s))) return rc;
-  if ((rc = zq::offdiag_abs(n, p.e, p.ea, s))) return rc;
   ZQ_HIP_CHECK(mark(2));
   ctx->info_dev = p.sw.info;
   ctx->last_kind = 1;
@@ -481,10 +480,12 @@ int solve_device(zq_context* ctx, int n, double* dD, int ld2, double* deig, bool
   const int zero = 0;
   p.sw.stage = &ctx->stage;
   apply_caps(ctx, p.sw);
-  if ((rc = zq::stedc(1, &zero, &n, n, n, p.d, p.ea, deig, p.sw, vectors, s))) return rc;
+  p.sw.phase_e = p.e;
+  p.sw.phi = vectors ? p.bw.phi : nullptr;
+  if ((rc = zq::stedc(1, &zero, &n, n, n, p.d, nullptr, p.e, deig, p.sw, vectors, s))) return rc;
   ZQ_HIP_CHECK(mark(3));
   if (vectors) {
-    if ((rc = zq::backtransform_batched(1, &n, zq::ZB{nullptr, 0}, nullptr, p.M, p.ldm, p.e, p.sw.Z, n, p.X, n, p.bw,
+    if ((rc = zq::backtransform_batched(1, &n, zq::ZB{nullptr, 0}, nullptr, p.M, p.ldm, p.sw.Z, n, p.X, n, p.bw,
                                         p.btasks, p.bsums, ctx->stage, s)))
       return rc;
     ZQ_HIP_CHECK(mark(4));
@@ -580,11 +581,14 @@ int solve_group(zq_context* ctx, std::vector<zq::BatchProb>& P, int nb, int tsm,
   if ((rc = zq::gather_tridiag_batched(nprob, L, bp.probs, bp.slab.d, bp.slab.e, zb, bp.dall, bp.eall, s))) return rc;
   bp.sw.stage = &st;
   apply_caps(ctx, bp.sw);
-  if ((rc = zq::stedc(nprob, zrow.data(), nh.data(), ntot, L, bp.dall, bp.eall, bp.wall, bp.sw, vectors, s)))
+  bp.sw.phase_e = bp.slab.e;
+  bp.sw.phi = vectors ? bp.slab.bw.phi : nullptr;
+  bp.sw.phase_zs = bp.zs;
+  if ((rc = zq::stedc(nprob, zrow.data(), nh.data(), ntot, L, bp.dall, bp.eall, nullptr, bp.wall, bp.sw, vectors, s)))
     return rc;
   if ((rc = zq::scatter_eig_batched(nprob, L, bp.probs, bp.wall, s))) return rc;
   if (vectors) {
-    if ((rc = zq::backtransform_batched(nprob, nh.data(), zb, bp.zrow, bp.slab.M, L, bp.slab.e, bp.sw.Z, ntot,
+    if ((rc = zq::backtransform_batched(nprob, nh.data(), zb, bp.zrow, bp.slab.M, L, bp.sw.Z, ntot,
                                         bp.slab.X, L, bp.slab.bw, bp.btasks, bp.sums, st, s)))
       return rc;
     if ((rc = zq::store_vectors_batched(nprob, L, bp.probs, bp.slab.X, L, zb, s))) return rc;
@@ -1448,7 +1452,7 @@ int zq_tridiag_eig(zq_context* c, int n, const double* dd, const double* de, dou
   p.sw.stage = &c->stage;
   apply_caps(c, p.sw);
   if ((rc = zq::stage_begin(c->stage))) return rc;
-  if ((rc = zq::stedc(1, &zero, &n, n, n, dd, de, dw, p.sw, vec, s))) return rc;
+  if ((rc = zq::stedc(1, &zero, &n, n, n, dd, de, nullptr, dw, p.sw, vec, s))) return rc;
   if ((rc = zq::stage_end(c->stage, s))) return rc;
   if (vec) ZQ_HIP_CHECK(hipMemcpyAsync(dZ, p.sw.Z, (size_t)n * n * sizeof(double), hipMemcpyDeviceToDevice, s));
   return ZQ_OK;

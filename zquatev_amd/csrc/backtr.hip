@@ -22,51 +22,6 @@
 
 namespace zq {
 
-// phi_0 = 1, phi_{c+1} = r_c phi_c with r_c = e_c / |e_c| (1 where e_c = 0):
-// a prefix product of unit quaternions in one workgroup: a chunk per thread,
-// then a scan of the chunks' products over each wave's lanes and over the
-// waves.  (Scanning 256 chunks one after the other, and chunks four times as
-// long, took 14 us at n = 64 and 56 us at n = 4096; now @PH@.)
-constexpr int PH_T = 1024;
-__device__ __forceinline__ quat unit_of(const quat& e) {
-  const double ae = sqrt(qnorm2(e));
-  return (ae > 0.0) ? qscale(e, 1.0 / ae) : quat{1.0, 0.0, 0.0, 0.0};
-}
-__device__ __forceinline__ quat shfl_up_q(const quat& v, int k) {
-  return quat{__shfl_up(v.ar, k, 64), __shfl_up(v.ai, k, 64), __shfl_up(v.br, k, 64), __shfl_up(v.bi, k, 64)};
-}
-__global__ void __launch_bounds__(PH_T) k_phases(int n, const quat* __restrict__ e, quat* __restrict__ phi, ZB zb) {
-  if (zb.nvec) {
-    n = zb.nvec[blockIdx.z];
-    e = zoff(e, zb); phi = zoff(phi, zb);
-  }
-  __shared__ quat tot[PH_T / 64];
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const quat one = quat{1.0, 0.0, 0.0, 0.0};
-  // thread t owns phi_k for k in (a, b]: the products r_{k-1} ... r_a
-  const int chunk = (n - 1 + PH_T - 1) / PH_T;
-  const int a = min(n - 1, t * chunk), b = min(n - 1, a + chunk);
-  quat L = one;
-  for (int k = a; k < b; ++k) L = qmul(unit_of(qload(e + k)), L);
-  // inclusive scan over the lanes: later chunks multiply from the left
-#pragma unroll
-  for (int k = 1; k < 64; k <<= 1) {
-    const quat o = shfl_up_q(L, k);
-    if (lane >= k) L = qmul(L, o);
-  }
-  if (lane == 63) tot[wv] = L;
-  __syncthreads();
-  quat base = one;   // the waves before
-  for (int w = 0; w < wv; ++w) base = qmul(tot[w], base);
-  const quat prev = shfl_up_q(L, 1);
-  quat cur = lane == 0 ? base : qmul(prev, base);   // phi_a
-  if (t == 0) qstore(phi, one);
-  for (int k = a; k < b; ++k) {
-    cur = qmul(unit_of(qload(e + k)), cur);
-    qstore(phi + k + 1, cur);
-  }
-}
-
 // X[i, j] = phi_i Z[i, j]  (in a batch, problem z's Z block starts at row zrow[z])
 __global__ void __launch_bounds__(256) k_phase_apply(int n, const quat* __restrict__ phi, const double* __restrict__ Z,
                                                      int ldz, quat* __restrict__ X, int ldx, ZB zb,
@@ -108,7 +63,7 @@ __global__ void __launch_bounds__(256) k_sum_parts_b(const SumTask* __restrict__
 // thread per element.  Lanes run along the index that the triangular factor
 // does not bound, so that a wave's loop ends with its own columns (rows).  Twelve short
 // products instead of the 64-column recurrence (four columns at a time, three
-// barriers each): 65 us -> @TF@.
+// barriers each): 65 us -> 19 us.
 constexpr int TF_WB = 64;
 constexpr int TF_T = 1024;
 __global__ void __launch_bounds__(TF_T) k_tfactor(int n, const quat* __restrict__ Gall, quat* __restrict__ Tall,
@@ -185,13 +140,12 @@ size_t backtransform_batched_sums(int nprob, const int* nh, int wbt) {
   return (size_t)nprob * cdiv(nh[0] - 1, wbt) * 2 + 1;
 }
 
-int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, const quat* M, int ld, const quat* e,
-                          const double* Z, int ldz, quat* X, int ldx, const BacktrWork& w, QGemmTask* tasks,
-                          SumTask* sums, Staging& st, hipStream_t s) {
+int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, const quat* M, int ld, const double* Z,
+                          int ldz, quat* X, int ldx, const BacktrWork& w, QGemmTask* tasks, SumTask* sums, Staging& st,
+                          hipStream_t s) {
   if (nprob <= 0) return ZQI_OK;
   const int L = nh[0];
   const int wbt = w.wbt;
-  hipLaunchKernelGGL(k_phases, dim3(1, 1, nprob), dim3(PH_T), 0, s, L, e, w.phi, zb);
   hipLaunchKernelGGL(k_phase_apply, dim3(cdiv(L, 256), L, nprob), dim3(256), 0, s, L, w.phi, Z, ldz, X, ldx, zb,
                      zrow_d);
   if (hipGetLastError() != hipSuccess) return ZQI_ERR_HIP;

@@ -408,12 +408,22 @@ constexpr int DBM = 64, DBN = 64, DBK = 16;
 __global__ void __launch_bounds__(256) k_dgemm_merge(const MergeDesc* __restrict__ descs, const int* __restrict__ kcnt,
                                                      const int* __restrict__ kgrp, const double* __restrict__ Qtmp,
                                                      const double* __restrict__ U, int lq, double* __restrict__ Z,
-                                                     int ldz, const int* __restrict__ posK) {
+                                                     int ldz, const int* __restrict__ posK,
+                                                     const int* __restrict__ posD) {
   const MergeDesc md = descs[blockIdx.z];
   const int K = kcnt[blockIdx.z];
   const int m = md.hi - md.lo, n1 = md.mid - md.lo;
   const int row0 = blockIdx.x * DBM, col0 = blockIdx.y * DBN;
-  if (col0 >= K || row0 >= m) return;
+  if (col0 >= m || row0 >= m) return;
+  if (col0 + DBN > K) {
+    // columns K .. of Qtmp are the deflated ones: copied to their final columns
+    const int i = row0 + (threadIdx.x & (DBM - 1));
+    if (i < m)
+      for (int j = max(col0, K) + (threadIdx.x >> 6); j < min(col0 + DBN, m); j += 4)
+        Z[md.lo + i + (size_t)(md.lo - md.ob + posD[md.lo + j - K]) * ldz] =
+            Qtmp[(size_t)md.lo * lq + i + (size_t)j * m];
+    if (col0 >= K) return;
+  }
   // the sum's range for this tile's rows (the full range for a tile across the halves)
   const int kb = row0 >= n1 ? kgrp[2 * blockIdx.z] : 0;
   const int ke = row0 + DBM <= n1 ? kgrp[2 * blockIdx.z + 1] : K;
@@ -492,10 +502,11 @@ __global__ void __launch_bounds__(256) k_dgemm_merge(const MergeDesc* __restrict
 }
 
 int dgemm_merges(const MergeDesc* descs_dev, int nmerge, int nsmax, const int* kcnt, const int* kgrp,
-                 const double* Qtmp, const double* U, int lq, double* Z, int ldz, const int* posK, hipStream_t s) {
+                 const double* Qtmp, const double* U, int lq, double* Z, int ldz, const int* posK, const int* posD,
+                 hipStream_t s) {
   if (nmerge <= 0 || nsmax <= 0) return ZQI_OK;
   dim3 grid((nsmax + DBM - 1) / DBM, (nsmax + DBN - 1) / DBN, nmerge);
-  launch_k(k_dgemm_merge, grid, dim3(256), 0, s, descs_dev, kcnt, kgrp, Qtmp, U, lq, Z, ldz, posK);
+  launch_k(k_dgemm_merge, grid, dim3(256), 0, s, descs_dev, kcnt, kgrp, Qtmp, U, lq, Z, ldz, posK, posD);
   return hipGetLastError() == hipSuccess ? ZQI_OK : ZQI_ERR_HIP;
 }
 

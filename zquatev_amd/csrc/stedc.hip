@@ -38,29 +38,30 @@ constexpr double DEPS = DBL_EPSILON * 0.5;   // unit roundoff
 
 static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
+// The subdiagonal: magnitudes e, or (q set) the quaternions whose magnitudes they are.
+struct SubDiag {
+  const double* e;
+  const quat* q;
+  __device__ __forceinline__ double operator[](int i) const { return q ? sqrt(qnorm2(qload(q + i))) : fabs(e[i]); }
+};
+
 // --------------------------------------------------------------------------
-// scale: s = max(max|d|, max|e|) per problem; d, e scaled by 1/s into lam, es.
+// scale (eigenvalues only; with vectors each base block does the same for its
+// rows): s = max(max|d|, max|e|) per problem; d, e scaled by 1/s into lam, es.
 // probs holds (offset, size) per problem, one workgroup each.  A tridiagonal
 // holding a NaN or an infinity (an input entry of that kind, or an overflow
 // in the reduction) is replaced by zeros and marks the problem's status word:
 // the merges rank values by comparisons, which a NaN would make inconsistent.
 // --------------------------------------------------------------------------
-__global__ void __launch_bounds__(1024) k_dc_scale(const int* __restrict__ probs, const double* __restrict__ d,
-                                                   const double* __restrict__ e, double* __restrict__ lam,
-                                                   double* __restrict__ es, double* __restrict__ scal,
-                                                   int* __restrict__ info) {
-  const int o = probs[2 * blockIdx.x], n = probs[2 * blockIdx.x + 1];
-  d += o; e += o; lam += o; es += o;
+// (The scale helper is for workgroups of 1024 threads; bad: not all finite.)
+__device__ __forceinline__ double tridiag_scale(int o, int n, const double* d, const SubDiag& e, int& bad) {
   __shared__ double sh[16];
   double m = 0.0;
-  int bad = 0;
+  bad = 0;
   for (int i = threadIdx.x; i < n; i += 1024) {
-    m = fmax(m, fabs(d[i]));
-    bad |= !isfinite(d[i]);
-  }
-  for (int i = threadIdx.x; i < n - 1; i += 1024) {
-    m = fmax(m, fabs(e[i]));
-    bad |= !isfinite(e[i]);
+    const double di = d[o + i], ei = i < n - 1 ? e[o + i] : 0.0;
+    m = fmax(m, fmax(fabs(di), ei));
+    bad |= !isfinite(di) || !isfinite(ei);
   }
 #pragma unroll
   for (int k = 32; k >= 1; k >>= 1) m = fmax(m, __shfl_xor(m, k, 64));
@@ -68,25 +69,23 @@ __global__ void __launch_bounds__(1024) k_dc_scale(const int* __restrict__ probs
   bad = __syncthreads_or(bad);
   double s = 0.0;
   for (int k = 0; k < 16; ++k) s = fmax(s, sh[k]);
-  if (!(s > 0.0) || bad) s = 1.0;
+  return (!(s > 0.0) || bad) ? 1.0 : s;
+}
+
+__global__ void __launch_bounds__(1024) k_dc_scale(const int* __restrict__ probs, const double* __restrict__ d,
+                                                   SubDiag e, double* __restrict__ lam,
+                                                   double* __restrict__ es, double* __restrict__ scal,
+                                                   int* __restrict__ info) {
+  const int o = probs[2 * blockIdx.x], n = probs[2 * blockIdx.x + 1];
+  int bad;
+  const double s = tridiag_scale(o, n, d, e, bad);
   const double inv = 1.0 / s;
-  for (int i = threadIdx.x; i < n; i += 1024) lam[i] = bad ? 0.0 : d[i] * inv;
-  for (int i = threadIdx.x; i < n - 1; i += 1024) es[i] = bad ? 0.0 : fabs(e[i]) * inv;
+  for (int i = threadIdx.x; i < n; i += 1024) lam[o + i] = bad ? 0.0 : d[o + i] * inv;
+  for (int i = threadIdx.x; i < n - 1; i += 1024) es[o + i] = bad ? 0.0 : e[o + i] * inv;
   if (threadIdx.x == 0) {
     scal[blockIdx.x] = s;
     if (bad) atomicOr(info + blockIdx.x, ZQI_INFO_NONFINITE);
   }
-}
-
-// subtract the coupling beta = es[s-1] from the diagonal entries beside each split s
-__global__ void k_dc_tear(int nsplit, const int* __restrict__ splits, const double* __restrict__ es,
-                          double* __restrict__ lam) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nsplit) return;
-  const int s = splits[t];
-  const double b = es[s - 1];
-  lam[s - 1] -= b;
-  lam[s] -= b;
 }
 
 // --------------------------------------------------------------------------
@@ -124,7 +123,17 @@ struct MergeBufs {
   int* gpos;     // per kept index: its GEMM position
   int* ginv;     // per GEMM position: the kept index
   int* kgrp;     // per merge: end of the first-half group, end of the both-halves group
+  // a problem's last merge also writes its eigenvalues w, unscaled
+  const int* probs;
+  const double* scal;
+  double* w;
 };
+// Eigenvalue lam of problem pr at position i (global) of its spectrum, unscaled;
+// NaN where the problem's input held a NaN or an infinity.
+__device__ __forceinline__ void put_eigenvalue(double* w, const double* scal, const int* info, int pr, int i,
+                                               double lam) {
+  w[i] = (info[pr] & ZQI_INFO_NONFINITE) ? __builtin_nan("") : lam * scal[pr];
+}
 
 __device__ __forceinline__ int count_less(const double* a, int len, double v) {
   int lo = 0, hi = len;
@@ -308,22 +317,15 @@ __global__ void __launch_bounds__(256) k_merge_prep(const MergeDesc* __restrict_
     }
     if (inl) B.mix[lo + t] = mix[t];
   }
-}
-
-// GEMM order of the kept columns (one workgroup per merge): first-half
-// columns, then the ones mixing both halves, then second-half columns, each
-// group in kept order (stable ranks from block scans over contiguous chunks).
-__global__ void __launch_bounds__(256) k_merge_types(const MergeDesc* __restrict__ descs, MergeBufs B) {
-  const MergeDesc md = descs[blockIdx.x];
-  const int lo = md.lo, n1 = md.mid - md.lo;
-  const int K = B.kcnt[blockIdx.x];
-  const int* keep = B.keep + lo;
+  // GEMM order of the kept columns: first-half columns, then the ones mixing
+  // both halves, then second-half columns, each group in kept order (stable
+  // ranks from block scans over contiguous chunks).
   auto type_of = [&](int k) {
     const int sp = keep[k];
-    return B.mix[lo + sp] ? 1 : (B.src[lo + sp] < n1 ? 0 : 2);
+    return mix[sp] ? 1 : (src[sp] < n1 ? 0 : 2);
   };
-  const int C = (K + 255) / 256;
-  const int k0 = min(K, (int)threadIdx.x * C), k1 = min(K, k0 + C);
+  const int CK = (K + 255) / 256;
+  const int k0 = min(K, (int)threadIdx.x * CK), k1 = min(K, k0 + CK);
   int c[3] = {0, 0, 0};
   for (int k = k0; k < k1; ++k) ++c[type_of(k)];
   __shared__ int sc[3][256];
@@ -339,16 +341,16 @@ __global__ void __launch_bounds__(256) k_merge_types(const MergeDesc* __restrict
     for (int g = 0; g < 3; ++g) sc[g][threadIdx.x] += v[g];
     __syncthreads();
   }
-  const int n0 = sc[0][255], nm = sc[1][255];
-  int pos[3] = {sc[0][threadIdx.x] - c[0], n0 + sc[1][threadIdx.x] - c[1], n0 + nm + sc[2][threadIdx.x] - c[2]};
+  const int c0 = sc[0][255], cm = sc[1][255];
+  int at[3] = {sc[0][threadIdx.x] - c[0], c0 + sc[1][threadIdx.x] - c[1], c0 + cm + sc[2][threadIdx.x] - c[2]};
   for (int k = k0; k < k1; ++k) {
-    const int p = pos[type_of(k)]++;
+    const int p = at[type_of(k)]++;
     B.gpos[lo + k] = p;
     B.ginv[lo + p] = k;
   }
   if (threadIdx.x == 0) {
-    B.kgrp[2 * blockIdx.x] = n0;
-    B.kgrp[2 * blockIdx.x + 1] = n0 + nm;
+    B.kgrp[2 * blockIdx.x] = c0;
+    B.kgrp[2 * blockIdx.x + 1] = c0 + cm;
   }
 }
 
@@ -602,13 +604,59 @@ __global__ void __launch_bounds__(64 * ROOTS) k_merge_secular(const MergeDesc* _
   }
 }
 
+// The merged spectrum: final columns of the roots (posK) and of the deflated
+// values (posD), the eigenvalues in order, and at a problem's last merge its w.
+// zk is free by now and holds the root values.
+__device__ __forceinline__ void merge_order(const MergeDesc& md, double* lam, const MergeBufs& B) {
+  const int lo = md.lo, ns = md.hi - md.lo;
+  const int K = B.kcnt[blockIdx.y];
+  const int nd = ns - K;
+  // roots are written to lam only after every thread has read the deflated list
+  double* dv = B.dval + lo;
+  const bool last = ns == B.probs[2 * md.pr + 1];   // uniform
+  const double* d = B.dkk + lo;
+  for (int t = threadIdx.x; t < ns; t += 256) {
+    if (t < K) {
+      const double v = d[B.org[lo + t]] + B.tau[lo + t];
+      B.posK[lo + t] = t + count_less(dv, nd, v);
+      B.zk[lo + t] = v;
+    }
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < ns; t += 256) {
+    if (t < nd) {
+      const double v = dv[t];
+      // number of roots <= v: roots are sorted ascending
+      int a = 0, b = K;
+      while (a < b) {
+        const int m = (a + b) >> 1;
+        if (B.zk[lo + m] <= v) a = m + 1; else b = m;
+      }
+      B.posD[lo + t] = t + a;
+    }
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < ns; t += 256) {
+    const int q = lo + (t < K ? B.posK[lo + t] : B.posD[lo + t - K]);
+    const double v = t < K ? B.zk[lo + t] : dv[t - K];
+    lam[q] = v;
+    if (last) put_eigenvalue(B.w, B.scal, B.info, md.pr, q, v);
+  }
+}
+
 // Gu-Eisenstat: zhat_j^2 = prod_i (lambda_i - d_j) / (rho prod_{i != j} (d_i - d_j)),
-// one wavefront per j, the lanes splitting the product.
-__global__ void __launch_bounds__(256) k_merge_zhat(const MergeDesc* __restrict__ descs, MergeBufs B) {
+// one wavefront per j, the lanes splitting the product.  The first block of each
+// merge orders its spectrum meanwhile.
+__global__ void __launch_bounds__(256) k_merge_zhat(const MergeDesc* __restrict__ descs, double* __restrict__ lam,
+                                                    MergeBufs B) {
   const MergeDesc md = descs[blockIdx.y];
+  if (blockIdx.x == 0) {
+    merge_order(md, lam, B);
+    return;
+  }
   const int lo = md.lo;
   const int K = B.kcnt[blockIdx.y];
-  const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int j = (blockIdx.x - 1) * 4 + (threadIdx.x >> 6);
   if (j >= K) return;   // wave-uniform
   const int lane = threadIdx.x & 63;
   const double rho = B.rho[blockIdx.y];
@@ -653,55 +701,6 @@ __global__ void __launch_bounds__(256) k_merge_buildU(const MergeDesc* __restric
   for (int j = threadIdx.x; j < K; j += 256) Ucol[j] *= inv;
 }
 
-__global__ void __launch_bounds__(256) k_merge_order(const MergeDesc* __restrict__ descs, double* __restrict__ lam,
-                                                     MergeBufs B) {
-  const MergeDesc md = descs[blockIdx.x];
-  const int lo = md.lo, ns = md.hi - md.lo;
-  const int K = B.kcnt[blockIdx.x];
-  const int nd = ns - K;
-  // roots are written to lam only after every thread has read the deflated list
-  double* dv = B.dval + lo;
-  const double* d = B.dkk + lo;
-  for (int t = threadIdx.x; t < ns; t += 256) {
-    if (t < K) {
-      const double v = d[B.org[lo + t]] + B.tau[lo + t];
-      B.posK[lo + t] = t + count_less(dv, nd, v);
-      B.zhat[lo + t] = v;  // zhat no longer needed: keep the root value
-    }
-  }
-  __syncthreads();
-  for (int t = threadIdx.x; t < ns; t += 256) {
-    if (t < nd) {
-      const double v = dv[t];
-      // number of roots <= v: roots are sorted ascending
-      int a = 0, b = K;
-      while (a < b) {
-        const int m = (a + b) >> 1;
-        if (B.zhat[lo + m] <= v) a = m + 1; else b = m;
-      }
-      B.posD[lo + t] = t + a;
-    }
-  }
-  __syncthreads();
-  for (int t = threadIdx.x; t < ns; t += 256) {
-    if (t < K) lam[lo + B.posK[lo + t]] = B.zhat[lo + t];
-    else lam[lo + B.posD[lo + t - K]] = dv[t - K];
-  }
-}
-
-__global__ void __launch_bounds__(256) k_merge_copydefl(const MergeDesc* __restrict__ descs, double* __restrict__ Z,
-                                                        int ldz, MergeBufs B) {
-  const MergeDesc md = descs[blockIdx.z];
-  const int lo = md.lo, ns = md.hi - md.lo;
-  const int K = B.kcnt[blockIdx.z];
-  const int t = blockIdx.y;
-  if (t >= ns - K) return;
-  const int r = blockIdx.x * 256 + threadIdx.x;
-  if (r >= ns) return;
-  const double* Q = B.Qtmp + (size_t)lo * B.lq;
-  Z[(lo + r) + (size_t)(lo - md.ob + B.posD[lo + t]) * ldz] = Q[r + (size_t)(K + t) * ns];
-}
-
 // --------------------------------------------------------------------------
 // base block: the divide & conquer of up to BASE rows in one workgroup, with
 // the eigenvectors Q in LDS.  The block is halved D = 0 .. 5 times into 2^D
@@ -726,9 +725,65 @@ __global__ void __launch_bounds__(256) k_merge_copydefl(const MergeDesc* __restr
 constexpr int BT = 1024;
 constexpr int BQ = BASE + 1;   // column stride of Q and U in LDS (doubles)
 
-__global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, double* __restrict__ lam,
-                                                const double* __restrict__ es, double* __restrict__ Z, int ldz,
-                                                int* __restrict__ info, int cap_leaf, int cap_sec) {
+// The phases of the quaternion subdiagonal (backtr.hip uses them) ride along
+// with the base blocks: problem z's subdiagonal and phi at z zs bytes.
+struct PhaseJob {
+  const quat* e;
+  quat* phi;
+  size_t zs;
+};
+// phi_0 = 1, phi_{c+1} = r_c phi_c with r_c = e_c / |e_c| (1 where e_c = 0):
+// a prefix product of unit quaternions in one workgroup: a chunk per thread,
+// then a scan of the chunks' products over each wave's lanes and over the
+// waves.  A launch of its own, with 256 chunks scanned one after the other, took
+// 14 us at n = 64 and 56 us at n = 4096; here it ends before the base blocks do.
+constexpr int PH_T = BT;
+__device__ __forceinline__ quat unit_of(const quat& e) {
+  const double ae = sqrt(qnorm2(e));
+  return (ae > 0.0) ? qscale(e, 1.0 / ae) : quat{1.0, 0.0, 0.0, 0.0};
+}
+__device__ __forceinline__ quat shfl_up_q(const quat& v, int k) {
+  return quat{__shfl_up(v.ar, k, 64), __shfl_up(v.ai, k, 64), __shfl_up(v.br, k, 64), __shfl_up(v.bi, k, 64)};
+}
+__device__ __forceinline__ void phases_block(int n, const quat* e, quat* phi) {
+  __shared__ quat tot[PH_T / 64];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const quat one = quat{1.0, 0.0, 0.0, 0.0};
+  // thread t owns phi_k for k in (a, b]: the products r_{k-1} ... r_a
+  const int chunk = (n - 1 + PH_T - 1) / PH_T;
+  const int a = min(n - 1, t * chunk), b = min(n - 1, a + chunk);
+  quat L = one;
+  for (int k = a; k < b; ++k) L = qmul(unit_of(qload(e + k)), L);
+  // inclusive scan over the lanes: later chunks multiply from the left
+#pragma unroll
+  for (int k = 1; k < 64; k <<= 1) {
+    const quat o = shfl_up_q(L, k);
+    if (lane >= k) L = qmul(L, o);
+  }
+  if (lane == 63) tot[wv] = L;
+  __syncthreads();
+  quat base = one;   // the waves before
+  for (int w = 0; w < wv; ++w) base = qmul(tot[w], base);
+  const quat prev = shfl_up_q(L, 1);
+  quat cur = lane == 0 ? base : qmul(prev, base);   // phi_a
+  if (t == 0) qstore(phi, one);
+  for (int k = a; k < b; ++k) {
+    cur = qmul(unit_of(qload(e + k)), cur);
+    qstore(phi + k + 1, cur);
+  }
+}
+
+__global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, int nleaf,
+                                                const int* __restrict__ probs, const double* d, SubDiag e,
+                                                PhaseJob ph, double* __restrict__ lam, double* __restrict__ es,
+                                                double* __restrict__ scal, double* __restrict__ Z, int ldz,
+                                                int* __restrict__ info, double* w, int cap_leaf, int cap_sec) {
+  if ((int)blockIdx.x >= nleaf) {   // the blocks after the base blocks: the problems' phases
+    const int z = blockIdx.x - nleaf;
+    phases_block(probs[2 * z + 1], reinterpret_cast<const quat*>(reinterpret_cast<const char*>(ph.e) + z * ph.zs),
+                 reinterpret_cast<quat*>(reinterpret_cast<char*>(ph.phi) + z * ph.zs));
+    return;
+  }
   typedef double d4 __attribute__((ext_vector_type(4)));
   __shared__ double Q[BASE * BQ], U[BASE * BQ];   // column-major
   __shared__ double sl[BASE], se[BASE];           // diagonal / eigenvalues, subdiagonal
@@ -744,8 +799,25 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
   const int tid = threadIdx.x, lane = tid & 63;
   int D = 0;
   while ((2 << D) < m) ++D;
-  if (tid < m) sl[tid] = lam[lo0 + tid];
-  if (tid < m - 1) se[tid] = es[lo0 + tid];
+  // the problem's scale (each of its blocks finds it for itself), and this
+  // block's rows, torn at its ends
+  const int n = probs[2 * pr + 1];
+  int bad;
+  const double scale = tridiag_scale(ob, n, d, e, bad), inv = 1.0 / scale;
+  const bool torn0 = lo0 > ob, torn1 = lo0 + m < ob + n;
+  if (tid < m) {
+    const double ei = (tid < m - 1 || torn1) && !bad ? e[lo0 + tid] * inv : 0.0;
+    double v = bad ? 0.0 : d[lo0 + tid] * inv;
+    if (tid == 0 && torn0 && !bad) v -= e[lo0 - 1] * inv;
+    if (tid == m - 1 && torn1) v -= ei;
+    sl[tid] = v;
+    if (tid < m - 1) se[tid] = ei;
+    es[lo0 + tid] = ei;
+  }
+  if (tid == 0 && !torn0) {
+    scal[pr] = scale;
+    if (bad) atomicOr(info + pr, ZQI_INFO_NONFINITE);
+  }
   if (tid <= (1 << D)) {   // leaf boundary: follow the bits from the top
     int a = 0, b = m;
     if (tid < (1 << D))
@@ -1006,20 +1078,15 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
     }
     __syncthreads();
   }
-  if (tid < m) lam[lo0 + tid] = sl[tid];
+  if (tid < m) {
+    lam[lo0 + tid] = sl[tid];
+    if (!torn0 && !torn1)   // the whole problem (its status word holds the load's findings)
+      w[lo0 + tid] = (bad || (info[pr] & ZQI_INFO_NONFINITE)) ? __builtin_nan("") : sl[tid] * scale;
+  }
   for (int k = tid; k < m * m; k += BT) {
     const int c = k / m, r = k - c * m;
     Z[(lo0 + r) + (size_t)(lo0 - ob + c) * ldz] = Q[c * BQ + r];
   }
-}
-
-// Eigenvalues of a problem whose input held a NaN or an infinity are NaN.
-__global__ void k_dc_unscale(const int* __restrict__ probs, const double* __restrict__ lam,
-                             const double* __restrict__ scal, const int* __restrict__ info, double* __restrict__ w) {
-  const int o = probs[2 * blockIdx.y], n = probs[2 * blockIdx.y + 1];
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  const bool bad = (info[blockIdx.y] & ZQI_INFO_NONFINITE) != 0;
-  if (i < n) w[o + i] = bad ? __builtin_nan("") : lam[o + i] * scal[blockIdx.y];
 }
 
 // --------------------------------------------------------------------------
@@ -1138,7 +1205,8 @@ int eigvals_one(int n, const double* d, const double* e, double* w, const StedcW
   if (n <= 0) return ZQI_OK;
   int* iprob = sw.ints;   // (offset, size) written by a kernel: nothing is uploaded from the host
   hipLaunchKernelGGL(k_set_prob, dim3(1), dim3(1), 0, s, iprob, 0, n);
-  hipLaunchKernelGGL(k_dc_scale, dim3(1), dim3(1024), 0, s, iprob, d, e, sw.lam, sw.es, sw.scal, sw.info);
+  hipLaunchKernelGGL(k_dc_scale, dim3(1), dim3(1024), 0, s, iprob, d, SubDiag{e, nullptr}, sw.lam, sw.es, sw.scal,
+                     sw.info);
   return values_kernels(1, n, n, iprob, w, sw, s);
 }
 
@@ -1151,7 +1219,7 @@ int status_out(const int* word, int* out, hipStream_t s) {
 
 // --------------------------------------------------------------------------
 static void build_tree(int lo, int hi, int ob, int pr, int depth, std::vector<int>& leaves,
-                       std::vector<std::vector<MergeDesc>>& lv, std::vector<int>& splits) {
+                       std::vector<std::vector<MergeDesc>>& lv) {
   if (hi - lo <= BASE) {
     leaves.insert(leaves.end(), {lo, hi, ob, pr});
     return;
@@ -1159,19 +1227,18 @@ static void build_tree(int lo, int hi, int ob, int pr, int depth, std::vector<in
   const int mid = lo + (hi - lo) / 2;
   if ((int)lv.size() <= depth) lv.resize(depth + 1);
   lv[depth].push_back(MergeDesc{lo, mid, hi, ob, pr});
-  splits.push_back(mid);
-  build_tree(lo, mid, ob, pr, depth + 1, leaves, lv, splits);
-  build_tree(mid, hi, ob, pr, depth + 1, leaves, lv, splits);
+  build_tree(lo, mid, ob, pr, depth + 1, leaves, lv);
+  build_tree(mid, hi, ob, pr, depth + 1, leaves, lv);
 }
 
 size_t stedc_int_slots(int ntot, int nprob) {
   // per problem of size n at most L = 2 ceil(n / BASE) base blocks (4 ints each),
-  // L - 1 splits (1 int) and L - 1 merges (5 ints), and (offset, size)
+  // L - 1 merges (5 ints), and (offset, size)
   return (size_t)22 * (ntot / BASE + nprob) + 2 * (size_t)nprob + 64;
 }
 
-int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const double* d, const double* e, double* w,
-          const StedcWork& sw, bool vectors, hipStream_t s) {
+int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const double* d, const double* e, const quat* eq,
+          double* w, const StedcWork& sw, bool vectors, hipStream_t s) {
   if (nprob <= 0 || ntot <= 0) return ZQI_OK;
   int nmax = 0;
   std::vector<int> probs(2 * (size_t)nprob);
@@ -1181,12 +1248,12 @@ int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const dou
     nmax = std::max(nmax, ns[z]);
   }
   if (nmax <= 0) return ZQI_OK;
-  std::vector<int> leaves, splits;
+  std::vector<int> leaves;
   std::vector<std::vector<MergeDesc>> levels;
   if (vectors)
     for (int z = 0; z < nprob; ++z)
-      if (ns[z] > 0) build_tree(offs[z], offs[z] + ns[z], offs[z], z, 0, leaves, levels, splits);
-  // device table: merge descriptors (deepest level first), leaves, splits, problems
+      if (ns[z] > 0) build_tree(offs[z], offs[z] + ns[z], offs[z], z, 0, leaves, levels);
+  // device table: merge descriptors (deepest level first), base blocks, problems
   std::vector<MergeDesc> flat;
   std::vector<size_t> level_off;
   for (int dpt = (int)levels.size() - 1; dpt >= 0; --dpt) {
@@ -1194,7 +1261,7 @@ int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const dou
     for (auto& md : levels[dpt]) flat.push_back(md);
   }
   static_assert(sizeof(MergeDesc) == 5 * sizeof(int), "MergeDesc is uploaded as 5 ints");
-  std::vector<int> host(5 * flat.size() + leaves.size() + splits.size() + probs.size());
+  std::vector<int> host(5 * flat.size() + leaves.size() + probs.size());
   size_t o = 0;
   for (auto& md : flat) {
     host[o++] = md.lo;
@@ -1205,8 +1272,6 @@ int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const dou
   }
   const size_t o_leaf = o;
   for (int v : leaves) host[o++] = v;
-  const size_t o_split = o;
-  for (int v : splits) host[o++] = v;
   const size_t o_prob = o;
   for (int v : probs) host[o++] = v;
   if (host.size() > sw.int_slots) return ZQI_ERR_ARG;
@@ -1214,22 +1279,23 @@ int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const dou
   if (rc) return rc;
   const MergeDesc* idesc = reinterpret_cast<const MergeDesc*>(sw.ints);
   const int* ileaf = sw.ints + o_leaf;
-  const int* isplit = sw.ints + o_split;
   const int* iprob = sw.ints + o_prob;
 
-  hipLaunchKernelGGL(k_dc_scale, dim3(nprob), dim3(1024), 0, s, iprob, d, e, sw.lam, sw.es, sw.scal, sw.info);
-  if (!vectors) return values_kernels(nprob, nmax, ntot, iprob, w, sw, s);
+  const SubDiag sub{e, eq};
+  if (!vectors) {
+    hipLaunchKernelGGL(k_dc_scale, dim3(nprob), dim3(1024), 0, s, iprob, d, sub, sw.lam, sw.es, sw.scal, sw.info);
+    return values_kernels(nprob, nmax, ntot, iprob, w, sw, s);
+  }
   const int nleaf = (int)leaves.size() / 4;
   const int ldz = ntot;
-  if ((rc = fill_zero(sw.Z, (size_t)ntot * lq * sizeof(double), s))) return rc;
-  if (!splits.empty())
-    hipLaunchKernelGGL(k_dc_tear, dim3(cdiv((int)splits.size(), 256)), dim3(256), 0, s, (int)splits.size(), isplit,
-                       sw.es, sw.lam);
-  hipLaunchKernelGGL(k_dc_base, dim3(nleaf), dim3(BT), 0, s, ileaf, sw.lam, sw.es, sw.Z, ldz, sw.info, sw.cap_leaf,
-                     sw.cap_secular);
+  // merges read whole columns of the blocks' eigenvectors
+  if (nmax > BASE && (rc = fill_zero(sw.Z, (size_t)ntot * lq * sizeof(double), s))) return rc;
+  hipLaunchKernelGGL(k_dc_base, dim3(nleaf + (sw.phi ? nprob : 0)), dim3(BT), 0, s, ileaf, nleaf, iprob, d, sub,
+                     PhaseJob{sw.phase_e, sw.phi, sw.phase_zs}, sw.lam, sw.es, sw.scal, sw.Z, ldz, sw.info, w,
+                     sw.cap_leaf, sw.cap_secular);
   MergeBufs B{sw.dk, sw.zk, sw.src, sw.keep, sw.dfl, sw.rot, sw.nrot, sw.kcnt, sw.dkk, sw.zkk, sw.dval, sw.rho,
               sw.org, sw.tau, sw.zhat, sw.posK, sw.posD, sw.Qtmp, sw.U, lq, sw.info, sw.cap_secular,
-              sw.mix, sw.gpos, sw.ginv, sw.kgrp};
+              sw.mix, sw.gpos, sw.ginv, sw.kgrp, iprob, sw.scal, w};
   for (size_t li = 0; li < level_off.size(); ++li) {
     const size_t off = level_off[li];
     const size_t cnt = (li + 1 < level_off.size() ? level_off[li + 1] : flat.size()) - off;
@@ -1239,7 +1305,6 @@ int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const dou
     const int nm = (int)cnt;
     hipLaunchKernelGGL(k_merge_prep, dim3(nm), dim3(256), 0, s, dd, sw.lam, sw.es, sw.Z, ldz, B);
     hipLaunchKernelGGL(k_merge_rot, dim3(cdiv(nsmax, 256), nm), dim3(256), 0, s, dd, sw.Z, ldz, B);
-    hipLaunchKernelGGL(k_merge_types, dim3(nm), dim3(256), 0, s, dd, B);
     hipLaunchKernelGGL(k_merge_gather, dim3(cdiv(nsmax, 256), cdiv(nsmax, GATHER_COLS), nm), dim3(256), 0, s, dd,
                        sw.Z, ldz, B);
     {
@@ -1250,17 +1315,14 @@ int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const dou
       else
         hipLaunchKernelGGL(k_merge_secular<16>, dim3(cdiv(nsmax, 16), nm), dim3(1024), shm, s, dd, B, kst);
     }
-    hipLaunchKernelGGL(k_merge_zhat, dim3(cdiv(nsmax, 4), nm), dim3(256), 0, s, dd, B);
+    hipLaunchKernelGGL(k_merge_zhat, dim3(1 + cdiv(nsmax, 4), nm), dim3(256), 0, s, dd, sw.lam, B);
     hipLaunchKernelGGL(k_merge_buildU, dim3(nsmax, nm), dim3(256), 0, s, dd, B);
-    hipLaunchKernelGGL(k_merge_order, dim3(nm), dim3(256), 0, s, dd, sw.lam, B);
     {
       ProfScope ps(PROF_MERGE, s, 0.0);
-      rc = dgemm_merges(dd, nm, nsmax, sw.kcnt, sw.kgrp, sw.Qtmp, sw.U, lq, sw.Z, ldz, sw.posK, s);
+      rc = dgemm_merges(dd, nm, nsmax, sw.kcnt, sw.kgrp, sw.Qtmp, sw.U, lq, sw.Z, ldz, sw.posK, sw.posD, s);
     }
     if (rc) return rc;
-    hipLaunchKernelGGL(k_merge_copydefl, dim3(cdiv(nsmax, 256), nsmax, nm), dim3(256), 0, s, dd, sw.Z, ldz, B);
   }
-  hipLaunchKernelGGL(k_dc_unscale, dim3(cdiv(nmax, 256), nprob), dim3(256), 0, s, iprob, sw.lam, sw.scal, sw.info, w);
   return hipGetLastError() == hipSuccess ? ZQI_OK : ZQI_ERR_HIP;
 }
 

@@ -361,6 +361,11 @@ struct StedcWork {
   int* ints;      // tree descriptors
   size_t int_slots;
   Staging* stage; // host staging of the descriptors
+  // with vectors, when phi is set: the phases of the quaternion subdiagonals
+  // are formed too (problem z's e and phi phase_zs bytes after problem z-1's)
+  const quat* phase_e = nullptr;
+  quat* phi = nullptr;
+  size_t phase_zs = 0;
   // iteration caps: Jacobi sweeps per leaf, secular-equation steps
   // per root, multisection steps per eigenvalue (reaching one is reported
   // as non-convergence, info > 0)
@@ -368,10 +373,11 @@ struct StedcWork {
 };
 size_t stedc_int_slots(int ntot, int nprob);
 // offs/ns (host): problem offsets and sizes; ntot = sum of ns; lq >= max ns.
-// d, e: concatenated diagonals and |subdiagonals| (e[o_z + i], i < n_z - 1);
+// d, e: concatenated diagonals and |subdiagonals| (e[o_z + i], i < n_z - 1; or
+// eq, not null: quaternions whose magnitudes they are);
 // w (ntot): eigenvalues ascending per problem.  Z (when vectors) is ld ntot.
-int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const double* d, const double* e, double* w,
-          const StedcWork& sw, bool vectors, hipStream_t s);
+int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const double* d, const double* e, const quat* eq,
+          double* w, const StedcWork& sw, bool vectors, hipStream_t s);
 // Eigenvalues of one tridiagonal of order n, the kernels stedc runs for it
 // without vectors, with nothing staged from the host (sw.ints holds the
 // problem's (offset, size), written by a kernel).
@@ -404,7 +410,7 @@ void stage_free(Staging& st);
 // backtr.hip: X = Q Phi Z with the reflectors u_c kept in M, applied in
 // blocks of wbt consecutive reflectors (compact WY, I - V T V^*).
 struct BacktrWork {
-  quat* phi;          // n
+  quat* phi;          // n, formed by stedc
   quat* part;         // split-K partials: part_slots
   size_t part_slots;  // >= nsplit * wbt * n
   int nsplit;
@@ -429,8 +435,7 @@ size_t backtransform_batched_sums(int nprob, const int* nh, int wbt);
 // ZB{nullptr, 0}); problem z's real eigenvectors are Z + zrow[z] (ld ldz),
 // zrow_d the device copy (null for a single solve).  tasks / sums: device
 // room for the task tables.
-int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, const quat* M, int ld, const quat* e,
-                          const double* Z, int ldz, quat* X, int ldx, const BacktrWork& w, QGemmTask* tasks,
+int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, const quat* M, int ld, const double* Z, int ldz, quat* X, int ldx, const BacktrWork& w, QGemmTask* tasks,
                           SumTask* sums, Staging& st, hipStream_t s);
 
 // layout.hip
@@ -515,7 +520,8 @@ int splitk_count(int K, int nsplit, int* kchunk_out);
 // kgrp: per merge the GEMM positions ending the first-half and both-halves
 // groups of kept columns
 int dgemm_merges(const MergeDesc* descs_dev, int nmerge, int nsmax, const int* kcnt, const int* kgrp,
-                 const double* Qtmp, const double* U, int lq, double* Z, int ldz, const int* posK, hipStream_t s);
+                 const double* Qtmp, const double* U, int lq, double* Z, int ldz, const int* posK, const int* posD,
+                 hipStream_t s);
 int mfma_probe(const double* a, const double* b, double* out, hipStream_t s);
 
 // api.hip hooks for the serving loop (serve.hip)
