@@ -69,6 +69,24 @@ def test_batch_equals_solo_bitwise(gpu_ctx):
         inv.assert_solution(H, Xs[k], eigs[k])
 
 
+@pytest.mark.parametrize("switch", [0, 100, -1])
+@pytest.mark.parametrize("sizes", [[97], [150, 66], [190, 129, 67], [161, 160, 96, 96, 65]])
+def test_batch_folded_grids(gpu_ctx, sizes, switch):
+    """Large and small members share a row of blocks: odd and even numbers of
+    active members, both strip widths in one column.  Bitwise, as above."""
+    _say(f"case: folded batch sizes {sizes} switch {switch}")
+    gpu_ctx.set_tile_shape(matvec_switch=switch)
+    try:
+        Ds = [gen.uniform_case(n, 6100 + k) for k, n in enumerate(sizes)]
+        rc, info, Xs, eigs = _batch(gpu_ctx, Ds)
+        assert rc == 0 and info == [0] * len(sizes)
+        for k, D in enumerate(Ds):
+            Xs1, e1 = _solo(gpu_ctx, D)
+            assert np.array_equal(eigs[k], e1) and np.array_equal(Xs[k], Xs1)
+    finally:
+        gpu_ctx.set_tile_shape()
+
+
 def test_batch_fock_workload(gpu_ctx):
     """A small draw of the batched workload: Fock-like matrices, 2n uniform over even [64, 1024]."""
     n2s = [int(v) for v in gen.batched_sizes(10, 1002)]

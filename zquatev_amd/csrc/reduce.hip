@@ -39,6 +39,9 @@ constexpr int TSM_MAX = 2048;
 __host__ __device__ constexpr int matvec_spg(int m, int tsm) { return m <= tsm ? 4 : 2; }
 // matvec tiles of a trailing size with G row groups: group g holds spg (g + 1) strips
 __host__ __device__ constexpr int ntiles(int G, int spg) { return spg * G * (G + 1) / 2; }
+// blocks of k_symv (nf of them finishing blocks) and of k_wcol at trailing size sz
+__host__ __device__ constexpr int symv_blocks(int sz, int spg, int nf) { return ntiles((sz + SG - 1) / SG, spg) + nf; }
+__host__ __device__ constexpr int wcol_blocks(int sz) { return sz - 1 > RQ ? (sz - 1 + RQ - 1) / RQ : 1; }
 constexpr int NBMAX = 128;   // largest supported panel width
 constexpr int TAILN = 64;    // trailing size from which one workgroup finishes (k_tail)
 
@@ -122,14 +125,14 @@ __global__ void __launch_bounds__(SYT) k_symv(
   static_assert(SW <= SG && SG % SW == 0 && SW % NWV == 0, "matvec tile shape");
   const int NT = j > 0 ? (8 * j + 63) / 64 : 0;
   const int NF = NT > 0 ? NT : 1;
+  int bt = blockIdx.x;
   if constexpr (BT) {
-    n = zb.nvec[blockIdx.z];
+    int z;
+    if (!fold_member(zb, [=](int m) { return symv_blocks(m - c - 1, SPG, NF); }, z, n, bt)) return;
     nparts = (n - c - 1 + RQ - 1) / RQ;
-    const int Gz = (n - c - 1 + SG - 1) / SG;
-    if ((int)blockIdx.x >= ntiles(Gz, SPG) + NF) return;
-    M = zoff(M, zb); W = zoff(W, zb); part = zoff(part, zb); scal = zoff(scal, zb); d = zoff(d, zb);
-    e = zoff(e, zb); Prow = zoff(Prow, zb); Pcol = zoff(Pcol, zb); TS = zoff(TS, zb); TSP = zoff(TSP, zb);
-    QF = zoff(QF, zb);
+    M = zoff(M, zb, z); W = zoff(W, zb, z); part = zoff(part, zb, z); scal = zoff(scal, zb, z); d = zoff(d, zb, z);
+    e = zoff(e, zb, z); Prow = zoff(Prow, zb, z); Pcol = zoff(Pcol, zb, z); TS = zoff(TS, zb, z);
+    TSP = zoff(TSP, zb, z); QF = zoff(QF, zb, z);
   }
   __shared__ double sh[SYT / 64];
   __shared__ double sqf[SYT / 64];
@@ -140,7 +143,6 @@ __global__ void __launch_bounds__(SYT) k_symv(
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: its column loads are scalar
   // blocks [0, NF) finish the column (dispatched first, so they overlap the
   // tiles), blocks NF + b take tile b
-  const int bt = blockIdx.x;
   const int b = bt - NF;
   if (b < 0) {
     // ---- finishing block: reflector, scalars, tall-skinny products
@@ -489,11 +491,12 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
     int n, int p, int c, int j, int ldw, int ldp, int nb, const quat* __restrict__ TS, const double* __restrict__ scal,
     const double* __restrict__ QF, double* __restrict__ part, double* __restrict__ TSP, double* __restrict__ d,
     int ldtsp, int tsm, ZB zb) {
+  int bx = blockIdx.x;
   if constexpr (BT) {
-    n = zb.nvec[blockIdx.z];
-    if (blockIdx.x > 0 && c + 2 + (int)blockIdx.x * RQ >= n) return;
-    M = zoff(M, zb); W = zoff(W, zb); Prow = zoff(Prow, zb); TS = zoff(TS, zb);
-    scal = zoff(scal, zb); QF = zoff(QF, zb); part = zoff(part, zb); TSP = zoff(TSP, zb); d = zoff(d, zb);
+    int z;
+    if (!fold_member(zb, [=](int m) { return wcol_blocks(m - c - 1); }, z, n, bx)) return;
+    M = zoff(M, zb, z); W = zoff(W, zb, z); Prow = zoff(Prow, zb, z); TS = zoff(TS, zb, z);
+    scal = zoff(scal, zb, z); QF = zoff(QF, zb, z); part = zoff(part, zb, z); TSP = zoff(TSP, zb, z); d = zoff(d, zb, z);
   }
   __shared__ quat a[NBMAX], b[NBMAX], cw[NBMAX], cv[NBMAX];
   __shared__ __align__(16) double red[RB / 64][RQ][RPAD];   // wave, row, (p | column update) component
@@ -503,7 +506,7 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
   const int s0 = c + 1;
   const bool more = (j + 1 < nb) && (c + 1 <= n - 2);   // uniform
   const int r = tid & (RQ - 1), q = tid >> 4;
-  const int i = s0 + 1 + blockIdx.x * RQ + r;
+  const int i = s0 + 1 + bx * RQ + r;
   const int ic = min(i, n - 1);
   const int jl = j > 0 ? j - 1 : 0;
   // ---- loads, all issued up front
@@ -620,7 +623,7 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
                                    quat{lane_d(st, 5), lane_d(st, 6), lane_d(st, 7), lane_d(st, 8)}, lane_d(sv, 0),
                                    quat{lane_d(sv, 1), lane_d(sv, 2), lane_d(sv, 3), lane_d(sv, 4)},
                                    quat{lane_d(sv, 5), lane_d(sv, 6), lane_d(sv, 7), lane_d(sv, 8)}, lane_d(sv, 9));
-  if (blockIdx.x == 0 && tid == 0) {   // row s0
+  if (bx == 0 && tid == 0) {   // row s0
     qstore(M + s0 + (size_t)c * ld, C.u1);
     qstore(W + s0 + (size_t)j * ldw, C.wc1);
     if (more) d[s0] = C.dnext;
@@ -643,9 +646,9 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
     ss += xlane<2>(ss);
     ss += xlane<4>(ss);
     ss += xlane<8>(ss);
-    if (lane == 0) part[blockIdx.x] = ss;
+    if (lane == 0) part[bx] = ss;
   }
-  row_tsp<KPT>(vv, ww, o.u, o.w, o.x, q, j, TSP + (size_t)blockIdx.x * ldtsp);
+  row_tsp<KPT>(vv, ww, o.u, o.w, o.x, q, j, TSP + (size_t)bx * ldtsp);
 }
 
 // ---------------------------------------------------------------------------
@@ -842,7 +845,7 @@ int reduce(quat* M, int n, int ld, int nb, double* d, quat* e, const ReduceWork&
           launch_k(k_symv<512, 32, false>, dim3(nmain), dim3(512), 0, s, M, w.W, w.TSP, w.part, ld, n, p, c, j, ldw,
                    nparts, w.ldtsp, w.scal, d, e, w.Prow, w.Pcol, n, nb, w.TS, w.QF, ZB{nullptr, 0});
       }
-      launch_wcol<false>(kpt, sz, dim3(std::max(1, cdiv(sz - 1, RQ))), s, M, w.W, w.Prow, w.pcs, ld, n, p, c, j, ldw,
+      launch_wcol<false>(kpt, sz, dim3(wcol_blocks(sz)), s, M, w.W, w.Prow, w.pcs, ld, n, p, c, j, ldw,
                          n, nb, w.TS, w.scal, w.QF, w.part, w.TSP, d, w.ldtsp, w.tsm, ZB{nullptr, 0});
     }
     // trailing update of rows/cols [p+wdt, n): M -= [V W] [W V]^*  (lower triangle)
@@ -939,20 +942,24 @@ int reduce_batched(int nprob, const int* nh, ZB zb, quat* M, int ld, int nb, dou
     };
     if (k1 > 0) {
       ProfScope ps(PROF_SYMV, s, tri_bytes(0, k1));
-      launch_k(k_symv<512, 32, true>, dim3(ntiles(cdiv(sz, SG), 2) + NF, 1, k1), dim3(512), 0, s, M, w.W, w.TSP,
-               w.part, ld, L, p, c, j, ldw, nparts, w.ldtsp, w.scal, d, e, w.Prow, w.Pcol, ld, nb, w.TS, w.QF, zb);
+      const int gx = fold_width(k1, [&](int z) { return symv_blocks(nh[z] - c - 1, 2, NF); });
+      launch_k(k_symv<512, 32, true>, dim3(gx, 1, (k1 + 1) / 2), dim3(512), 0, s, M, w.W, w.TSP,
+               w.part, ld, L, p, c, j, ldw, nparts, w.ldtsp, w.scal, d, e, w.Prow, w.Pcol, ld, nb, w.TS, w.QF,
+               ZB{zb.nvec, zb.zs, k1});
     }
     if (k1 < act) {
       const size_t sh = (size_t)k1 * zb.zs;
-      const int szn = nh[k1] - c - 1;
+      const int gx = fold_width(act - k1, [&](int z) { return symv_blocks(nh[k1 + z] - c - 1, 4, NF); });
       ProfScope ps(PROF_SYMV, s, tri_bytes(k1, act));
-      launch_k(k_symv<256, 16, true>, dim3(ntiles(cdiv(szn, SG), 4) + NF, 1, act - k1), dim3(256), 0, s, zshift(M,
+      launch_k(k_symv<256, 16, true>, dim3(gx, 1, (act - k1 + 1) / 2), dim3(256), 0, s, zshift(M,
                sh), zshift(w.W, sh), zshift(w.TSP, sh), zshift(w.part, sh), ld, L, p, c, j, ldw, nparts, w.ldtsp,
                zshift(w.scal, sh), zshift(d, sh), zshift(e, sh), zshift(w.Prow, sh), zshift(w.Pcol, sh), ld, nb,
-               zshift(w.TS, sh), zshift(w.QF, sh), ZB{zb.nvec + k1, zb.zs});
+               zshift(w.TS, sh), zshift(w.QF, sh), ZB{zb.nvec + k1, zb.zs, act - k1});
     }
-    launch_wcol<true>(kpt, sz, dim3(std::max(1, cdiv(sz - 1, RQ)), 1, act), s, M, w.W, w.Prow, w.pcs, ld, L, p, c, j,
-                      ldw, ld, nb, w.TS, w.scal, w.QF, w.part, w.TSP, d, w.ldtsp, w.tsm, zb);
+    const int gw = fold_width(act, [&](int z) { return wcol_blocks(nh[z] - c - 1); });
+    launch_wcol<true>(kpt, sz, dim3(gw, 1, (act + 1) / 2), s, M, w.W, w.Prow, w.pcs, ld, L, p, c, j,
+                      ldw, ld, nb, w.TS, w.scal, w.QF, w.part, w.TSP, d, w.ldtsp, w.tsm,
+                      ZB{zb.nvec, zb.zs, act});
     if (j == nb - 1 || c == cend - 1) {
       const int P = c / nb;
       const int cnt = toff[P + 1] - toff[P];
