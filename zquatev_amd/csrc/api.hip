@@ -989,9 +989,10 @@ int zq_tuned_panel_width(int n) {
   // measured on MI355X (eigenvalues only, 16 / 24 / 32): 2n = 2048 9.36 / 9.74 /
   // 9.71 ms, 4096 27.2 / 27.6 / 27.5, 6000 55.8 / 56.4 / 56.2, 8192 109.3 / 109.6 /
   // 109.1 (16's column kernel holds half the panel coefficients per thread; 32
-  // halves the passes of the trailing update, which is the larger part only at
-  // the top).  zq_autotune refines it per size bucket (floor(log2 n)).
-  return n < 4096 ? 16 : 32;
+  // halves the passes of the trailing update over the matrix, the larger part
+  // only beyond).  One width for n <= 4096 also keeps a batch of such sizes in
+  // one lockstep group.  zq_autotune refines it per size bucket (floor(log2 n)).
+  return n <= 4096 ? 16 : 32;
 }
 
 int zq_create(zq_context** out, int device) try {
