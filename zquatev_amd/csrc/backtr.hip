@@ -302,27 +302,30 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
   if (!rc && !ss.empty()) rc = stage_upload(st, ss.data(), ss.size() * sizeof(SumTask), sums, s);
   if (rc) return rc;
   // phase A launches
-  if ((rc = qgemm_tasks(tasks + gt0, ngt, gmaxk, gmaxk, 0, true, false, false, s))) return rc;
+  const QGemmTask* th = tt.data();
+  if ((rc = qgemm_tasks(tasks + gt0, th + gt0, ngt, gmaxk, gmaxk, 0, true, false, false, s))) return rc;
   if (ngs > 0) hipLaunchKernelGGL(k_sum_parts_b, dim3(cdiv(wbt * wbt, 256), 1, ngs), dim3(256), 0, s, sums);
   if (wbt < TF_WB || wbt % TF_WB || (tsub & (tsub - 1))) return ZQI_ERR_ARG;
   hipLaunchKernelGGL(k_tfactor, dim3(nblk * tsub, 1, nprob), dim3(TF_T), 0, s, L, w.G, w.T, tsub, zb);
   for (size_t li = 0; li < levels.size(); ++li) {
     const int wl = TF_WB << li;
-    if ((rc = qgemm_tasks(tasks + levels[li].p0, levels[li].np, wl, wl, 0, false, false, false, s))) return rc;
-    if ((rc = qgemm_tasks(tasks + levels[li].t0, levels[li].nt, wl, wl, 0, false, false, false, s))) return rc;
+    if ((rc = qgemm_tasks(tasks + levels[li].p0, th + levels[li].p0, levels[li].np, wl, wl, 0, false, false, false,
+                          s))) return rc;
+    if ((rc = qgemm_tasks(tasks + levels[li].t0, th + levels[li].t0, levels[li].nt, wl, wl, 0, false, false, false,
+                          s))) return rc;
   }
-  if ((rc = qgemm_tasks(tasks + vt0, nvt, vtmaxm, wbt, 0, false, true, false, s))) return rc;
+  if ((rc = qgemm_tasks(tasks + vt0, th + vt0, nvt, vtmaxm, wbt, 0, false, true, false, s))) return rc;
   // phase B launches
   for (const Step& q : steps) {
     {
       ProfScope ps(PROF_BACKTR, s, q.fy);
-      if ((rc = qgemm_tasks(tasks + q.y0, q.ny, q.maxw, q.maxn, q.kmin, true, false, false, s))) return rc;
+      if ((rc = qgemm_tasks(tasks + q.y0, th + q.y0, q.ny, q.maxw, q.maxn, q.kmin, true, false, false, s))) return rc;
     }
     if (q.ns > 0)
       hipLaunchKernelGGL(k_sum_parts_b, dim3(cdiv(q.maxtot, 256), 1, q.ns), dim3(256), 0, s, sums + q.s0);
     {
       ProfScope ps(PROF_BACKTR, s, q.fx);
-      if ((rc = qgemm_tasks(tasks + q.x0, q.nx, q.maxmr, q.maxn, 0, false, false, false, s))) return rc;
+      if ((rc = qgemm_tasks(tasks + q.x0, th + q.x0, q.nx, q.maxmr, q.maxn, 0, false, false, false, s))) return rc;
     }
   }
   return hipGetLastError() == hipSuccess ? ZQI_OK : ZQI_ERR_HIP;

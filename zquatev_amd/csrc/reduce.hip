@@ -964,7 +964,9 @@ int reduce_batched(int nprob, const int* nh, ZB zb, quat* M, int ld, int nb, dou
       const int P = c / nb;
       const int cnt = toff[P + 1] - toff[P];
       ProfScope ps(PROF_TRAIL, s, tflops[P]);
-      if (cnt > 0 && (rc = qgemm_tasks(tasks + toff[P], cnt, tmaxm[P], tmaxm[P], 0, false, true, true, s))) return rc;
+      if (cnt > 0 && (rc = qgemm_tasks(tasks + toff[P], tt.data() + toff[P], cnt, tmaxm[P], tmaxm[P], 0, false, true,
+                                       true, s)))
+        return rc;
     }
   }
   // problems without a tail take d[n-1] here; the tails overwrite theirs

@@ -534,11 +534,12 @@ struct QGemmTask {
   QOperand A, B;
   quat* C;
 };
-// ntasks independent tasks (device array) in one launch; maxm / maxnn bound
-// their shapes, kmin (0: unknown) the lengths of their sums from below; every task has the given operand conjugation flags.  Each task
-// computes exactly what qgemm would for it.
-int qgemm_tasks(const QGemmTask* tasks_dev, int ntasks, int maxm, int maxnn, int kmin, bool a_conj_trans, bool b_conj_trans,
-                bool lower_only, hipStream_t s);
+// ntasks independent tasks (device array, and the same on the host) in one
+// launch; maxm / maxnn bound their shapes, kmin (0: unknown) the lengths of
+// their sums from below; every task has the given operand conjugation flags.
+// Each task computes exactly what qgemm would for it.
+int qgemm_tasks(const QGemmTask* tasks_dev, const QGemmTask* tasks_host, int ntasks, int maxm, int maxnn, int kmin,
+                bool a_conj_trans, bool b_conj_trans, bool lower_only, hipStream_t s);
 // GEMM tile rows: 64-row tiles for launches of at least `g_tile64_per_cu`
 // 64 x 64 tiles per compute unit, else 32-row tiles.  A tuning parameter of
 // the calling thread (set per solve from its context; 16 by default): the
