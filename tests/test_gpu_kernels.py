@@ -174,6 +174,37 @@ def test_qgemm_small_tiles(gpu_ctx, m, n, k, ta, tb, lower):
     assert torch.equal(dC[:, m:, :], before[:, m:, :])
 
 
+@pytest.mark.parametrize("m", [1504, 1505, 1567])
+@pytest.mark.parametrize("k", [1, 8, 33])
+def test_qgemm_lower_tiles(gpu_ctx, m, k):
+    """Lower-triangle products from two 32 x 64 tiles per CU on (32 x 32 tiles):
+    bound as above, every entry against torch's FP64 products, the strict
+    upper triangle untouched."""
+    import torch
+    _say(f"case: qgemm lower tiles m={m} k={k}")
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+
+    def rand(r, c):   # [column, row, component]
+        return 2.0 * torch.rand(c, r, 4, dtype=torch.float64, device="cuda", generator=g) - 1.0
+
+    A, B, C = rand(m, k), rand(m, k), rand(m, m)
+    out = C.clone()
+    torch.cuda.synchronize()
+    assert gpu_ctx.qgemm_device("N", "C", m, m, k, -1.0, A.data_ptr(), m, B.data_ptr(), m, 1.0, out.data_ptr(), m,
+                                True) == 0
+    gpu_ctx.synchronize()
+    # (a1, b1)(a2, b2)^* with (a, b)^* = (conj a, -b): a1 conj a2 + conj b1 b2, b1 conj a2 - conj a1 b2
+    a1, b1 = (torch.complex(A[..., 2 * h], A[..., 2 * h + 1]).T for h in range(2))
+    a2, b2 = (torch.complex(B[..., 2 * h], B[..., 2 * h + 1]).T for h in range(2))
+    pa = a1 @ a2.mH.contiguous() + b1.conj() @ b2.T.contiguous()
+    pb = b1 @ a2.mH.contiguous() - a1.conj() @ b2.T.contiguous()
+    ref = C - torch.stack([pa.real.T, pa.imag.T, pb.real.T, pb.imag.T], -1)
+    low = torch.ones(m, m, dtype=torch.bool, device="cuda").triu()   # [column, row]: row >= column
+    bound = (4 * k + 2) * (4 * k + 1) * np.finfo(float).eps / 4
+    assert (out - ref)[low].abs().max().item() <= max(bound, 1e-14)
+    assert torch.equal(out[~low], C[~low])
+
+
 def test_qgemm_argument_errors(gpu_ctx):
     assert gpu_ctx.qgemm_device("X", "N", 2, 2, 2, 1.0, 0, 2, 0, 2, 0.0, 0, 2) == -2
     assert gpu_ctx.qgemm_device("N", "N", -1, 2, 2, 1.0, 0, 2, 0, 2, 0.0, 0, 2) == -4

@@ -45,6 +45,12 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 //                     ones read 10 (4096 x 4096 x 1024 66.3 -> 67.3 TFLOP/s, and
 //                     65.5 before the loads became branch-free, below);
 //   32 x 64, GBK 8    twice the workgroups (balance, registers);
+//   32 x 32, GBK 8    the same for lower-triangle products, whose K is a panel's
+//                     two widths: less of the tiles above the diagonal, and four
+//                     workgroups per CU (97 registers, 33 KB) to cover the
+//                     reads of C.  2n = 8192 solve 144.9 -> 144.3 ms, 4096 31.93 ->
+//                     31.78, batch of 512 72.6 -> 71.9; other products lose by the
+//                     extra operand traffic (batch 72.0 -> 72.9);
 //   16 x 32, GBK 16   for launches that leave CUs idle otherwise: a wave's time
 //                     is K x (its 16 x 16 x 4 products) x 64 cycles whatever
 //                     the other CUs do -- 14 us for 32 x 64 at K = 64, a
@@ -64,6 +70,7 @@ struct QTile {
 };
 using Tile64 = QTile<64, 64, 8, 4>;
 using Tile32 = QTile<32, 64, 8, 2>;
+using Tile32L = QTile<32, 32, 8, 2>;
 using Tile16 = QTile<16, 32, 16, 2>;
 
 // Operand elements as stored, loaded without a branch at a clamped index (row
@@ -340,7 +347,10 @@ static void launch_gemm2(bool act, bool bct, hipStream_t s, const QGemmTask& t, 
   const bool low = t.lower_only;
   switch (tile_rows((long)tile_count<Tile64>(t.m, t.nn, low) * nz, (long)tile_count<Tile32>(t.m, t.nn, low) * nz)) {
     case 64: launch_gemm2_t<Tile64>(act, bct, s, t, nz, kchunk, cstride); break;
-    case 32: launch_gemm2_t<Tile32>(act, bct, s, t, nz, kchunk, cstride); break;
+    case 32:
+      if (low) launch_gemm2_t<Tile32L>(act, bct, s, t, nz, kchunk, cstride);
+      else launch_gemm2_t<Tile32>(act, bct, s, t, nz, kchunk, cstride);
+      break;
     default: launch_gemm2_t<Tile16>(act, bct, s, t, nz, kchunk, cstride); break;
   }
 }
@@ -391,7 +401,13 @@ int qgemm_tasks(const QGemmTask* tasks_dev, const QGemmTask* tasks_host, int nta
   if (rows == 32 && kmin >= LONG_K && (long)n64 * ntasks >= 2L * device_cus()) rows = 64;
   switch (rows) {
     case 64: launch_gemm2_batch_t<Tile64>(act, bct, ntasks, n64, s, tasks_dev, tasks_host); break;
-    case 32: launch_gemm2_batch_t<Tile32>(act, bct, ntasks, n32, s, tasks_dev, tasks_host); break;
+    case 32:
+      if (lower)
+        launch_gemm2_batch_t<Tile32L>(act, bct, ntasks, tile_count<Tile32L>(maxm, maxnn, lower), s, tasks_dev,
+                                      tasks_host);
+      else
+        launch_gemm2_batch_t<Tile32>(act, bct, ntasks, n32, s, tasks_dev, tasks_host);
+      break;
     default:
       launch_gemm2_batch_t<Tile16>(act, bct, ntasks, tile_count<Tile16>(maxm, maxnn, lower), s, tasks_dev, tasks_host);
   }
