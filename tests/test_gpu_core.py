@@ -156,6 +156,38 @@ def test_tridiag_eig_one_block(gpu_ctx, n, kind):
     assert np.abs(Z.T @ Z - np.eye(n)).max() <= tol
 
 
+@pytest.mark.parametrize("kind", ["clement", "constant", "integer"])
+def test_tridiag_eig_structured(gpu_ctx, kind):
+    """Tridiagonals whose secular equations have roots within a rounding of an
+    end of their first bracket (the midpoint of two poles, or the bound of the
+    last root), where a Newton step that ends the iteration can round out of the
+    bracket.  Bound as for one block, with a merge level more per doubling."""
+    import torch
+    rng = np.random.default_rng(5)
+    for n in list(range(2, 65)) + [65, 80, 96, 100, 127, 128, 129, 130]:
+        _say(f"case: tridiag_eig {kind} n={n}")
+        k = np.arange(n - 1)
+        if kind == "clement":      # eigenvalues -(n - 1), -(n - 3), ..., n - 1
+            d, e = np.zeros(n), np.sqrt((k + 1.0) * (n - 1 - k))
+        elif kind == "constant":
+            d, e = rng.integers(0, 5, n).astype(float), np.full(n - 1, 0.1 * rng.integers(1, 60))
+        else:
+            d, e = rng.integers(0, 3, n).astype(float), rng.integers(0, 3, n - 1).astype(float)
+        dd, de = torch.from_numpy(d).cuda(), torch.from_numpy(np.r_[e, 0.0]).cuda()
+        dw = torch.zeros(n, dtype=torch.float64, device="cuda")
+        dz = torch.zeros(n * n, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        assert gpu_ctx.tridiag_eig_device(n, dd.data_ptr(), de.data_ptr(), dw.data_ptr(), dz.data_ptr()) == 0
+        assert gpu_ctx.last_info() == 0
+        w, Z = dw.cpu().numpy(), dz.cpu().numpy().reshape(n, n).T
+        T = np.diag(d) + np.diag(e, 1) + np.diag(e, -1)
+        tol = 8 * np.finfo(float).eps * (np.ceil(np.log2(n)) + n)
+        tn = max(np.linalg.norm(T, 2), 1e-300)
+        assert np.abs(w - np.linalg.eigvalsh(T)).max() <= tol * tn
+        assert np.abs(T @ Z - Z * w[None, :]).max() <= tol * tn
+        assert np.abs(Z.T @ Z - np.eye(n)).max() <= tol
+
+
 @pytest.mark.parametrize("n2", [2, 4, 6, 8, 16, 22, 42, 44, 64, 128, 130, 400, 510, 512])
 def test_zquatev_host(gpu_ctx, n2):
     _say(f"case: zquatev host 2n={n2}")

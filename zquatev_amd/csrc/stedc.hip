@@ -536,10 +536,12 @@ __device__ __forceinline__ SecRoot secular_root(double rho, int cap, int K, int 
     // 4.4 and at most 12 instead of 46, f at the roots equally small).  The test
     // comes before the bracket's: t is an end of the bracket now, and t - dt can
     // round onto it, which must not be taken for a step out of the bracket.
+    // A last step that rounds past the other end (a root within a rounding of
+    // the two poles' midpoint or of the last root's bound) stops there: that end
+    // is as good as the root, where t itself is up to 1e-9 of t off.
     const double dt = G / Gp;
     if (fabs(dt) <= 1e-9 * fabs(t)) {
-      const double tc = t - dt;
-      if (tc >= a && tc <= b) t = tc;
+      t = fmin(fmax(t - dt, a), b);
       conv = true;
       break;
     }
