@@ -147,9 +147,10 @@ int zq_zquatev_device(zq_context* ctx, int n2, double* dD, int nld2, double* dei
  * reference solves one matrix per call (zquatev.cc:42-72); a caller with many
  * matrices loops over ts::zquatev.  Problem i is (n2[i], D[i], ld2[i],
  * eig[i]) with the meaning of zq_zquatev_device's arguments; n2[i] = 0 is
- * skipped.  Problems are grouped by panel width and each group runs its
- * columns in lockstep, so every problem's result is bitwise the result of its
- * own zq_zquatev_device call on the same context.
+ * skipped.  Problems are grouped by panel width (and a few large ones apart
+ * from many small ones) and each group runs its columns in lockstep, so every
+ * problem's result is bitwise the result of its own zq_zquatev_device call on
+ * the same context.
  * Device-memory variant: asynchronous on the context's stream unless info is
  * given (host array of count ints), in which case it waits and stores each
  * problem's status there (0, or > 0: tridiagonal solver did not converge).
@@ -321,7 +322,7 @@ int zq_set_workspace_limit(zq_context* ctx, size_t bytes);
 
 /* Device workspace bytes a batched call of these sizes (jobz 'V' or 'N')
  * needs on ctx (NULL: the built-in panel-width table), split into runs that
- * fit `budget` bytes (0: one run per panel-width group).  *bytes receives
+ * fit `budget` bytes (0: one run per group).  *bytes receives
  * the largest run's workspace, run[i] (optional, count ints) problem i's run
  * (-1 for an empty problem).  Returns the number of runs, or -2 count < 0,
  * -3 bad sizes, -4 bad jobz.  Host arithmetic only: no device call. */

@@ -12,6 +12,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+import zquatev_amd as zq  # noqa: E402
 from zquatev_amd import gen  # noqa: E402
 from tests import invariants as inv  # noqa: E402
 
@@ -85,6 +86,20 @@ def test_batch_folded_grids(gpu_ctx, sizes, switch):
             assert np.array_equal(eigs[k], e1) and np.array_equal(Xs[k], Xs1)
     finally:
         gpu_ctx.set_tile_shape()
+
+
+def test_batch_large_member_apart(gpu_ctx):
+    """One large member among many small ones of its panel and block widths: the
+    group is cut between them.  Bitwise, as above."""
+    sizes = [449, 1024, 460, 449, 452, 470, 449, 455, 461, 449, 463]
+    _say(f"case: batch cut below its large member sizes {sizes}")
+    assert zq.batch_workspace([2 * n for n in sizes], "V")[1] == 2
+    Ds = [gen.uniform_case(n, 6200 + k) for k, n in enumerate(sizes)]
+    rc, info, Xs, eigs = _batch(gpu_ctx, Ds)
+    assert rc == 0 and info == [0] * len(sizes)
+    for k, D in enumerate(Ds):
+        Xs1, e1 = _solo(gpu_ctx, D)
+        assert np.array_equal(eigs[k], e1) and np.array_equal(Xs[k], Xs1)
 
 
 def test_batch_fock_workload(gpu_ctx):

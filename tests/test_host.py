@@ -182,6 +182,29 @@ def test_batch_workspace_split_plan():
         zq.batch_workspace([63], "V")
 
 
+@pytest.mark.parametrize("large,small,count", [(8192, 1800, 100), (8192, 1000, 50), (4096, 1000, 200),
+                                               (8192, 64, 400), (4096, 2046, 30)])
+def test_batch_workspace_of_a_few_large_members(large, small, count):
+    """Groups are solved one after the other, so a batch needs its largest group.
+    A large member does not size the slabs of many small ones: the batch needs
+    no more than its large members alone and its small members alone."""
+    for jobz in ("V", "N"):
+        whole, _, run = zq.batch_workspace([large] + [small] * count, jobz)
+        alone = zq.batch_workspace([large], jobz)[0], zq.batch_workspace([small] * count, jobz)[0]
+        assert whole == max(alone)
+        assert run[0] not in run[1:]
+
+
+def test_batch_workspace_of_an_even_mix():
+    """Large and small members in like numbers share a group, padded to at most
+    three times their squares (the workspace's leading term)."""
+    sizes = [3000, 2000, 1000] * 6
+    for jobz in ("V", "N"):
+        whole, runs, _ = zq.batch_workspace(sizes, jobz)
+        assert runs == 1
+        assert whole <= 3.0 * sum(zq.batch_workspace([s], jobz)[0] for s in sizes)
+
+
 def test_dropin_caller_is_built():
     exe = os.path.join(ROOT, "tests", "dropin", "zquatev_caller")
     assert os.path.exists(exe), "built by zquatev_amd/csrc/Makefile (__graft_entry__.build)"
