@@ -65,8 +65,9 @@ def _ct(a, b):
     (1500, 1500, 64, "N", "C", True, -1.0, 1.0)])
 @pytest.mark.parametrize("t64", [0, 1])
 def test_qgemm_against_complex_embedding(gpu_ctx, m, n, k, ta, tb, lower, alpha, beta, t64):
-    """t64 = 1: 64-row tiles for every launch of at least one 64 x 64 tile per
-    compute unit (0: the context's default threshold, 32-row tiles here)."""
+    """Small products (16 x 32 tiles whatever t64 is) and two with more than two
+    32 x 64 tiles per compute unit: t64 = 1 gives them 64-row tiles, 0 (the
+    context's default threshold) 32-row ones."""
     import torch
     _say(f"case: qgemm m={m} n={n} k={k} {ta}{tb} lower={lower} alpha={alpha} beta={beta} t64={t64}")
     rng = np.random.default_rng(m * 1000 + n + k)
@@ -203,6 +204,55 @@ def test_qgemm_lower_tiles(gpu_ctx, m, k):
     bound = (4 * k + 2) * (4 * k + 1) * np.finfo(float).eps / 4
     assert (out - ref)[low].abs().max().item() <= max(bound, 1e-14)
     assert torch.equal(out[~low], C[~low])
+
+
+# shape, lower, threshold of 64-row tiles (0: the default): the tiles that 256 CUs take
+@pytest.mark.parametrize("m,n,lower,t64", [
+    (1027, 1031, False, 0),   # 32 x 64: two per CU
+    (1027, 1031, False, 1),   # 64 x 64
+    (1409, 1409, True, 0),    # 32 x 32
+    (1409, 1409, True, 1)])   # 64 x 64
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("C", "N"), ("N", "C"), ("C", "C")])
+def test_qgemm_tile_shapes(gpu_ctx, m, n, lower, t64, ta, tb):
+    """Every tile shape, all conjugations, K at and off a stage's end (1, 7, 8,
+    33), beta = 0 over a C of NaNs (which it must not read) and beta != 0.
+    Bound as above (|alpha| < 1, |beta C| <= 1.25), against torch's FP64 products."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+
+    def rand(r, c):   # [column, row, component]
+        return 2.0 * torch.rand(c, r, 4, dtype=torch.float64, device="cuda", generator=g) - 1.0
+
+    def op(Q, conj):   # complex components (a, b) of op(Q)
+        a, b = (torch.complex(Q[..., 2 * h], Q[..., 2 * h + 1]).T.contiguous() for h in range(2))
+        return (a.mH.resolve_conj().contiguous(), -b.T.contiguous()) if conj else (a, b)
+
+    low = torch.ones(n, m, dtype=torch.bool, device="cuda")   # [column, row]: the entries written
+    if lower:
+        low = low.triu()
+    gpu_ctx.set_tile_shape(-1, t64)
+    try:
+        for k, alpha, beta in ((1, -1.0, 0.0), (7, -0.75, 1.25), (8, 1.0, 0.0), (33, 0.5, -1.25)):
+            _say(f"case: qgemm tile shapes m={m} n={n} k={k} {ta}{tb} lower={lower} t64={t64} beta={beta}")
+            A = rand(k, m) if ta == "C" else rand(m, k)
+            B = rand(n, k) if tb == "C" else rand(k, n)
+            C = rand(m, n) if beta else torch.full((n, m, 4), float("nan"), dtype=torch.float64, device="cuda")
+            out = C.clone()
+            torch.cuda.synchronize()
+            assert gpu_ctx.qgemm_device(ta, tb, m, n, k, alpha, A.data_ptr(), A.shape[1], B.data_ptr(), B.shape[1],
+                                        beta, out.data_ptr(), m, lower) == 0
+            gpu_ctx.synchronize()
+            (a1, b1), (a2, b2) = op(A, ta == "C"), op(B, tb == "C")
+            pa = a1 @ a2 - b1.conj().resolve_conj() @ b2
+            pb = b1 @ a2 + a1.conj().resolve_conj() @ b2
+            ref = alpha * torch.stack([pa.real.T, pa.imag.T, pb.real.T, pb.imag.T], -1)
+            if beta:
+                ref = ref + beta * C
+            bound = (4 * k + 2) * (4 * k + 2) * np.finfo(float).eps / 4
+            assert (out - ref)[low].abs().max().item() <= max(bound, 1e-14)
+            assert torch.equal(out[~low].view(torch.int64), C[~low].view(torch.int64))
+    finally:
+        gpu_ctx.set_tile_shape(-1, 0)
 
 
 def test_qgemm_argument_errors(gpu_ctx):
