@@ -96,9 +96,11 @@ int zq_panel_width(zq_context* ctx, int n);
  * strips (16 quaternions) for trailing sizes up to this many rows, wide (32)
  * above; candidates 512, 768, 1024, 1536; default 768 -- and the quaternion
  * GEMM's tile rows -- 64-row tiles for launches of at least this many
- * 64 x 64 tiles per compute unit, else 32-row tiles (16-row tiles for launches
- * too small to occupy the device); candidates 4, 16, 64;
- * default 16.  zq_set_tile_shape overrides both (switch -1 and threshold 0
+ * 64 x 64 tiles per compute unit, else 32-row tiles; candidates 4, 16, 64;
+ * default 16.  Two kinds of launch take their tiles whatever the threshold:
+ * 16-row ones where 32-row tiles would not fill two rounds of the device, and
+ * 64-row ones for the back-transform's split sums of K >= 384 with at least two
+ * 64 x 64 tiles per compute unit.  zq_set_tile_shape overrides both (switch -1 and threshold 0
  * restore the tuned values; switch 0..2048, -2 / -3 when out of range).
  * The switch changes the matvec's summation order, so a batch groups its
  * problems by it (as by panel width); the tile rows change no result.

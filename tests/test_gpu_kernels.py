@@ -208,6 +208,8 @@ def test_qgemm_lower_tiles(gpu_ctx, m, k):
 
 # shape, lower, threshold of 64-row tiles (0: the default): the tiles that 256 CUs take
 @pytest.mark.parametrize("m,n,lower,t64", [
+    (896, 1024, False, 0),    # 16 x 32: 7 of them per CU
+    (897, 1024, False, 0),    # 32 x 64: 16 x 32 would be more than 7 per CU
     (1027, 1031, False, 0),   # 32 x 64: two per CU
     (1027, 1031, False, 1),   # 64 x 64
     (1409, 1409, True, 0),    # 32 x 32

@@ -327,9 +327,14 @@ thread_local int g_tile64_per_cu = 16;
 // 33.4 ms, below 2 2.30, 4.65, 10.78, 33.2 ms, below 4 2.30, 4.65, 10.82, 33.8
 // ms, below 8 the 2n = 8192 solve too is slower (149.0 -> 151.9 ms): more
 // operand traffic per product once every CU is busy.
-constexpr int SMALL_PER_CU = 2;
-static int tile_rows(long tiles64, long tiles32) {
-  if (tiles32 < (long)SMALL_PER_CU * device_cus()) return 16;
+// And of at most SMALL_ROUNDS 16 x 32 tiles per unit: a launch's time goes by the
+// tiles of its fullest unit, and 8 small ones take longer than the 2 large ones
+// that a full round holds.  16 x 32 over 32 x 64, K = 16, 64, 256, 1024: at 5
+// tiles per unit 0.71, 0.72, 0.70, 0.70, at 6 0.80, 0.82, 0.83, 0.83, at 7 0.87,
+// 0.93, 0.96, 0.97, at 8 0.92, 1.03, 1.09, 1.10 (960 x 1000 x 1000: 541 and 598 us).
+constexpr int SMALL_PER_CU = 2, SMALL_ROUNDS = 7;
+static int tile_rows(long tiles64, long tiles32, long tiles16) {
+  if (tiles32 < (long)SMALL_PER_CU * device_cus() && tiles16 <= (long)SMALL_ROUNDS * device_cus()) return 16;
   return tiles64 >= (long)g_tile64_per_cu * device_cus() ? 64 : 32;
 }
 
@@ -345,7 +350,8 @@ static void launch_gemm2_t(bool act, bool bct, hipStream_t s, const QGemmTask& t
 
 static void launch_gemm2(bool act, bool bct, hipStream_t s, const QGemmTask& t, int nz, int kchunk, size_t cstride) {
   const bool low = t.lower_only;
-  switch (tile_rows((long)tile_count<Tile64>(t.m, t.nn, low) * nz, (long)tile_count<Tile32>(t.m, t.nn, low) * nz)) {
+  switch (tile_rows((long)tile_count<Tile64>(t.m, t.nn, low) * nz, (long)tile_count<Tile32>(t.m, t.nn, low) * nz,
+                    (long)tile_count<Tile16>(t.m, t.nn, low) * nz)) {
     case 64: launch_gemm2_t<Tile64>(act, bct, s, t, nz, kchunk, cstride); break;
     case 32:
       if (low) launch_gemm2_t<Tile32L>(act, bct, s, t, nz, kchunk, cstride);
@@ -397,7 +403,7 @@ int qgemm_tasks(const QGemmTask* tasks_dev, const QGemmTask* tasks_host, int nta
   // 64-row tiles by the largest task alone: many smaller ragged tasks lose more
   // to the padding of their edges than the larger tiles save (the 512-problem
   // batch 70.3 ms counting all tasks' tiles, 68.8 ms so)
-  int rows = tile_rows((long)n64, (long)n32 * ntasks);
+  int rows = tile_rows((long)n64, (long)n32 * ntasks, (long)tile_count<Tile16>(maxm, maxnn, lower) * ntasks);
   if (rows == 32 && kmin >= LONG_K && (long)n64 * ntasks >= 2L * device_cus()) rows = 64;
   switch (rows) {
     case 64: launch_gemm2_batch_t<Tile64>(act, bct, ntasks, n64, s, tasks_dev, tasks_host); break;
