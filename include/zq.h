@@ -17,8 +17,8 @@
  *
  * Return codes: 0 success; -i argument i is invalid (LAPACK style); > 0 the
  * tridiagonal eigensolver did not converge (as zhbev's info at zquatev.cc:84,
- * :99: a leaf's Jacobi iteration, a secular-equation root or an eigenvalue bracket
- * that did not converge; the value is 1 + a local row or root index);
+ * :99: a secular-equation root or an eigenvalue bracket that did not converge;
+ * the value is 1 + a local root index);
  * ZQ_ERR_* below for runtime errors and for a non-finite input.
  */
 #ifndef ZQ_H
@@ -100,8 +100,9 @@ int zq_panel_width(zq_context* ctx, int n);
  * default 16.  Two kinds of launch take their tiles whatever the threshold:
  * 16-row ones where 32-row tiles would not fill two rounds of the device, and
  * 64-row ones for the back-transform's split sums of K >= 384 with at least two
- * 64 x 64 tiles per compute unit.  zq_set_tile_shape overrides both (switch -1 and threshold 0
- * restore the tuned values; switch 0..2048, -2 / -3 when out of range).
+ * 64 x 64 tiles per compute unit.  zq_set_tile_shape overrides both (switch -1
+ * and threshold 0 restore the tuned values; switch 0..2048, -2 / -3 when out of
+ * range).
  * The switch changes the matvec's summation order, so a batch groups its
  * problems by it (as by panel width); the tile rows change no result.
  * zq_tile_shape reports what a solve of half-dimension n uses now. */
@@ -307,9 +308,9 @@ int zq_synchronize(zq_context* ctx);
 int zq_last_info(zq_context* ctx);
 
 /* Iteration caps of the tridiagonal eigensolver on ctx (0 = default):
- * Jacobi sweeps per divide & conquer leaf (60), safeguarded Newton
- * steps per secular-equation root (200), multisection steps per eigenvalue
- * of the eigenvalues-only path (64).  A cap reached is reported as
+ * safeguarded Newton steps per secular-equation root (200), multisection steps
+ * per eigenvalue of the eigenvalues-only path (64); leaf is accepted and has no
+ * effect (a divide & conquer leaf of one or two rows takes one rotation).  A cap reached is reported as
  * non-convergence (info > 0), as zhbev reports a QL failure (zquatev.cc:84).
  * Meant for tests of that path; -2 for a negative cap. */
 int zq_set_iteration_caps(zq_context* ctx, int leaf, int secular, int bisect);

@@ -241,8 +241,9 @@ class Context:
         return int(_fn("zq_last_info")(self._h))
 
     def set_iteration_caps(self, leaf=0, secular=0, bisect=0):
-        """Iteration caps of the tridiagonal solver (0: default 60 / 200 / 64);
-        reaching one is reported as non-convergence (info > 0)."""
+        """Iteration caps of the tridiagonal solver's secular roots and multisection
+        (0: default 200 / 64); reaching one is reported as non-convergence
+        (info > 0).  leaf has no effect."""
         _check(_fn("zq_set_iteration_caps")(self._h, int(leaf), int(secular), int(bisect)),
                "zq_set_iteration_caps")
 

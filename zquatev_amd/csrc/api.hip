@@ -70,7 +70,7 @@ struct zq_context {
   bool have_times = false;
   int* info_dev = nullptr;  // status word of the last single solve (device)
   int last_kind = 0;        // 0 none, 1 single solve (info_dev), 2 batch (binfo, last_count entries)
-  int caps[3] = {0, 0, 0};  // iteration caps of the tridiagonal solver (0: default)
+  int caps[2] = {0, 0};   // iteration caps of the tridiagonal solver: secular steps, multisection (0: default)
   int last_count = 0;
   zq::ProfState prof;
   zq::Staging stage;
@@ -422,9 +422,8 @@ int make_plan(zq_context* ctx, int n, int nb, bool vectors, Plan* p) {
 }
 
 void apply_caps(const zq_context* ctx, zq::StedcWork& sw) {
-  if (ctx->caps[0] > 0) sw.cap_leaf = ctx->caps[0];
-  if (ctx->caps[1] > 0) sw.cap_secular = ctx->caps[1];
-  if (ctx->caps[2] > 0) sw.cap_bisect = ctx->caps[2];
+  if (ctx->caps[0] > 0) sw.cap_secular = ctx->caps[0];
+  if (ctx->caps[1] > 0) sw.cap_bisect = ctx->caps[1];
 }
 
 // Makes the context's device current and, when the context runs on its own
@@ -1564,9 +1563,8 @@ int zq_last_info(zq_context* c) try {
 int zq_set_iteration_caps(zq_context* c, int leaf, int secular, int bisect) {
   if (!c) return ZQ_ERR_ARG;
   if (leaf < 0 || secular < 0 || bisect < 0) return -2;
-  c->caps[0] = leaf;
-  c->caps[1] = secular;
-  c->caps[2] = bisect;
+  c->caps[0] = secular;
+  c->caps[1] = bisect;
   return ZQ_OK;
 }
 

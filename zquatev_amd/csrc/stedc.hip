@@ -779,7 +779,7 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
                                                 const int* __restrict__ probs, const double* d, SubDiag e,
                                                 PhaseJob ph, double* __restrict__ lam, double* __restrict__ es,
                                                 double* __restrict__ scal, double* __restrict__ Z, int ldz,
-                                                int* __restrict__ info, double* w, int cap_leaf, int cap_sec) {
+                                                int* __restrict__ info, double* w, int cap_sec) {
   if ((int)blockIdx.x >= nleaf) {   // the blocks after the base blocks: the problems' phases
     const int z = blockIdx.x - nleaf;
     phases_block(probs[2 * z + 1], reinterpret_cast<const quat*>(reinterpret_cast<const char*>(ph.e) + z * ph.zs),
@@ -835,7 +835,6 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
   // ---- leaves
   if (tid < (1 << D)) {
     const int a = bnd[tid], sz = bnd[tid + 1] - a;   // 1 or 2 rows
-    int fail = 0;
     // torn at the splits inside the base block
     const double tl = a > 0 ? se[a - 1] : 0.0, tr = a + sz < m ? se[a + sz - 1] : 0.0;
     double p = sl[a] - tl, q = 0.0, r = 0.0, c = 1.0, s = 0.0;   // [p r; r q] and its vectors (c, -s), (s, c)
@@ -844,16 +843,14 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
       q = sl[a + 1] - tr;
       r = se[a];
     }
-    // Jacobi: one rotation makes the off-diagonal entry 0
-    for (int it = 0; fabs(r) > DEPS * (fabs(p) + fabs(q));) {
+    // one Jacobi rotation makes the off-diagonal entry 0
+    if (fabs(r) > DEPS * (fabs(p) + fabs(q))) {
       const double th = (q - p) / (2.0 * r);
       const double t = copysign(1.0 / (fabs(th) + sqrt(fma(th, th, 1.0))), th);
       c = rsqrt(fma(t, t, 1.0));
       s = t * c;
       p = fma(-t, r, p);
       q = fma(t, r, q);
-      r = 0.0;
-      if (++it >= cap_leaf) { fail = 1; break; }
     }
     const bool sw = sz == 2 && q < p;   // ascending
     sl[a] = sw ? q : p;
@@ -864,7 +861,6 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
       Q[(a + 1) * BQ + a] = sw ? c : s;
       Q[(a + 1) * BQ + a + 1] = sw ? -s : c;
     }
-    if (fail) atomicMax(info + pr, lo0 - ob + a + 1);
   }
   __syncthreads();
   // ---- merges, 2^k at level k
@@ -1294,7 +1290,7 @@ int stedc(int nprob, const int* offs, const int* ns, int ntot, int lq, const dou
   if (nmax > BASE && (rc = fill_zero(sw.Z, (size_t)ntot * lq * sizeof(double), s))) return rc;
   hipLaunchKernelGGL(k_dc_base, dim3(nleaf + (sw.phi ? nprob : 0)), dim3(BT), 0, s, ileaf, nleaf, iprob, d, sub,
                      PhaseJob{sw.phase_e, sw.phi, sw.phase_zs}, sw.lam, sw.es, sw.scal, sw.Z, ldz, sw.info, w,
-                     sw.cap_leaf, sw.cap_secular);
+                     sw.cap_secular);
   MergeBufs B{sw.dk, sw.zk, sw.src, sw.keep, sw.dfl, sw.rot, sw.nrot, sw.kcnt, sw.dkk, sw.zkk, sw.dval, sw.rho,
               sw.org, sw.tau, sw.zhat, sw.posK, sw.posD, sw.Qtmp, sw.U, lq, sw.info, sw.cap_secular,
               sw.mix, sw.gpos, sw.ginv, sw.kgrp, iprob, sw.scal, w};

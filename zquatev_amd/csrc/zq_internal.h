@@ -401,10 +401,10 @@ struct StedcWork {
   const quat* phase_e = nullptr;
   quat* phi = nullptr;
   size_t phase_zs = 0;
-  // iteration caps: Jacobi sweeps per leaf, secular-equation steps
+  // iteration caps: secular-equation steps
   // per root, multisection steps per eigenvalue (reaching one is reported
   // as non-convergence, info > 0)
-  int cap_leaf = 60, cap_secular = 200, cap_bisect = 64;
+  int cap_secular = 200, cap_bisect = 64;
 };
 size_t stedc_int_slots(int ntot, int nprob);
 // offs/ns (host): problem offsets and sizes; ntot = sum of ns; lq >= max ns.
