@@ -188,7 +188,7 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
       for (int q = 0; q < nz; ++q) {
         const int kb = q * kchunk, ke = std::min(k.mr, kb + kchunk);
         quat* out = nz > 1 ? part + (size_t)q * wbt * wbt : Gb;
-        tt.push_back(QGemmTask{k.wdt, k.wdt, k.mr, kb, ke, wbt, 0, 1.0, 0.0, Vc, Vn, out});
+        tt.push_back(QGemmTask{k.wdt, k.wdt, kb, ke, wbt, 0, 1.0, 0.0, Vc, Vn, out});
       }
       if (nz > 1) ss.push_back(SumTask{part, Gb, wbt * wbt, nz});
       gmaxk = std::max(gmaxk, k.wdt);
@@ -217,12 +217,12 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
               const quat* T2 = T + (q + wl) + (size_t)(q + wl) * wbt;
               QOperand Ga{G12, G12, wbt, wbt, INT_MAX, false, INT_MIN / 2};
               QOperand Tb{T2, T2, wbt, wbt, INT_MAX, false, INT_MIN / 2};
-              tt.push_back(QGemmTask{w1, w2, w2, 0, w2, wl, 0, 1.0, 0.0, Ga, Tb, P});
+              tt.push_back(QGemmTask{w1, w2, 0, w2, wl, 0, 1.0, 0.0, Ga, Tb, P});
             } else {
               const quat* T1 = T + q + (size_t)q * wbt;
               QOperand Ta{T1, T1, wbt, wbt, INT_MAX, false, INT_MIN / 2};
               QOperand Pb{P, P, wl, wl, INT_MAX, false, INT_MIN / 2};
-              tt.push_back(QGemmTask{w1, w2, w1, 0, w1, wbt, 0, -1.0, 0.0, Ta, Pb, T + q + (size_t)(q + wl) * wbt});
+              tt.push_back(QGemmTask{w1, w2, 0, w1, wbt, 0, -1.0, 0.0, Ta, Pb, T + q + (size_t)(q + wl) * wbt});
             }
           }
         }
@@ -245,16 +245,16 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
       const quat* T = at(w.T, z) + (size_t)b * wbt * wbt;
       QOperand Vn{V, V, ld, ld, INT_MAX, false, -1};
       QOperand Tc{T, T, wbt, wbt, INT_MAX, true, INT_MIN / 2};
-      tt.push_back(QGemmTask{k.mr, k.wdt, k.wdt, 0, k.wdt, k.mr, 0, 1.0, 0.0, Vn, Tc, at(w.VT, z) + k.vt});
+      tt.push_back(QGemmTask{k.mr, k.wdt, 0, k.wdt, k.mr, 0, 1.0, 0.0, Vn, Tc, at(w.VT, z) + k.vt});
       vtmaxm = std::max(vtmaxm, k.mr);
     }
   const int nvt = (int)tt.size() - vt0;
   // ---- phase B, last block first: Y = VT^* X[r0:, :] (split), sums, X[r0:, :] -= V Y
-  struct Step { int y0, ny, s0, ns, x0, nx, maxw, maxn, maxtot, maxmr, kmin; double fy, fx; };
+  struct Step { int y0, ny, s0, ns, x0, nx, maxw, maxn, maxtot, maxmr, kchunk; double fy, fx; };
   std::vector<Step> steps;
   for (int b = nblk - 1; b >= 0; --b) {
     Step q{};
-    q.kmin = INT_MAX;
+    q.kchunk = INT_MAX;
     q.y0 = (int)tt.size();
     q.s0 = (int)ss.size();
     std::vector<QGemmTask> tx;
@@ -274,14 +274,14 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
       for (int c = 0; c < nz; ++c) {
         const int kb = c * kchunk, ke = std::min(k.mr, kb + kchunk);
         quat* out = nz > 1 ? part + (size_t)c * k.wdt * n : Y;
-        tt.push_back(QGemmTask{k.wdt, n, k.mr, kb, ke, k.wdt, 0, 1.0, 0.0, VTc, Xo, out});
+        tt.push_back(QGemmTask{k.wdt, n, kb, ke, k.wdt, 0, 1.0, 0.0, VTc, Xo, out});
       }
       if (nz > 1) ss.push_back(SumTask{part, Y, k.wdt * n, nz});
       QOperand Vn{V, V, ld, ld, INT_MAX, false, -1};
       QOperand Yo{Y, Y, k.wdt, k.wdt, INT_MAX, false, INT_MIN / 2};
-      tx.push_back(QGemmTask{k.mr, n, k.wdt, 0, k.wdt, ldx, 0, -1.0, 1.0, Vn, Yo, Xz + k.r0});
+      tx.push_back(QGemmTask{k.mr, n, 0, k.wdt, ldx, 0, -1.0, 1.0, Vn, Yo, Xz + k.r0});
       q.maxw = std::max(q.maxw, k.wdt);
-      q.kmin = std::min(q.kmin, kchunk);
+      q.kchunk = std::min(q.kchunk, std::min(kchunk, k.mr));
       q.maxn = std::max(q.maxn, n);
       q.maxtot = std::max(q.maxtot, k.wdt * n);
       q.maxmr = std::max(q.maxmr, k.mr);
@@ -319,7 +319,7 @@ int backtransform_batched(int nprob, const int* nh, ZB zb, const int* zrow_d, co
   for (const Step& q : steps) {
     {
       ProfScope ps(PROF_BACKTR, s, q.fy);
-      if ((rc = qgemm_tasks(tasks + q.y0, th + q.y0, q.ny, q.maxw, q.maxn, q.kmin, true, false, false, s))) return rc;
+      if ((rc = qgemm_tasks(tasks + q.y0, th + q.y0, q.ny, q.maxw, q.maxn, q.kchunk, true, false, false, s))) return rc;
     }
     if (q.ns > 0)
       hipLaunchKernelGGL(k_sum_parts_b, dim3(cdiv(q.maxtot, 256), 1, q.ns), dim3(256), 0, s, sums + q.s0);

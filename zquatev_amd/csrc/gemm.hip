@@ -386,17 +386,18 @@ static void launch_gemm2_batch_t(bool act, bool bct, int ntasks, int tiles, hipS
 int qgemm(int m, int nn, int k, double alpha, const QOperand& A, const QOperand& B, double beta, quat* C, int ldc,
           bool lower_only, hipStream_t s) {
   if (m <= 0 || nn <= 0) return ZQI_OK;
-  QGemmTask t{m, nn, k, 0, k, ldc, lower_only ? 1 : 0, alpha, beta, A, B, C};
+  QGemmTask t{m, nn, 0, k, ldc, lower_only ? 1 : 0, alpha, beta, A, B, C};
   launch_gemm2(A.conj_trans, B.conj_trans, s, t, 1, k, (size_t)0);
   return hipGetLastError() == hipSuccess ? ZQI_OK : ZQI_ERR_HIP;
 }
 
-// Task lists whose every sum is at least LONG_K long take 64-row tiles already
-// from two per CU, where they all run at once: the back-transform's Y products at
-// n >= 4096 (1024 32-row tiles make one and a third rounds of three per CU, 512
-// 64-row ones one round of two; 2n = 8192 back-transform 39.3 -> 38.4 ms).
+// Task lists of split-K chunks of at least LONG_K (but for a sum's last chunk)
+// take 64-row tiles already from two per CU, where they all run at once: the
+// back-transform's Y products at n >= 4096 (1024 32-row tiles make one and a third
+// rounds of three per CU, 512 64-row ones one round of two; 2n = 8192
+// back-transform 39.3 -> 38.4 ms).
 constexpr int LONG_K = 384;
-int qgemm_tasks(const QGemmTask* tasks_dev, const QGemmTask* tasks_host, int ntasks, int maxm, int maxnn, int kmin,
+int qgemm_tasks(const QGemmTask* tasks_dev, const QGemmTask* tasks_host, int ntasks, int maxm, int maxnn, int kchunk,
                 bool act, bool bct, bool lower, hipStream_t s) {
   if (ntasks <= 0 || maxm <= 0 || maxnn <= 0) return ZQI_OK;
   const int n64 = tile_count<Tile64>(maxm, maxnn, lower), n32 = tile_count<Tile32>(maxm, maxnn, lower);
@@ -404,7 +405,7 @@ int qgemm_tasks(const QGemmTask* tasks_dev, const QGemmTask* tasks_host, int nta
   // to the padding of their edges than the larger tiles save (the 512-problem
   // batch 70.3 ms counting all tasks' tiles, 68.8 ms so)
   int rows = tile_rows((long)n64, (long)n32 * ntasks, (long)tile_count<Tile16>(maxm, maxnn, lower) * ntasks);
-  if (rows == 32 && kmin >= LONG_K && (long)n64 * ntasks >= 2L * device_cus()) rows = 64;
+  if (rows == 32 && kchunk >= LONG_K && (long)n64 * ntasks >= 2L * device_cus()) rows = 64;
   switch (rows) {
     case 64: launch_gemm2_batch_t<Tile64>(act, bct, ntasks, n64, s, tasks_dev, tasks_host); break;
     case 32:

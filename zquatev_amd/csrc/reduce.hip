@@ -911,7 +911,7 @@ int reduce_batched(int nprob, const int* nh, ZB zb, quat* M, int ld, int nb, dou
       quat* Wz = reinterpret_cast<quat*>(reinterpret_cast<char*>(w.W) + (size_t)z * zb.zs);
       QOperand A{Mz + r0 + (size_t)p * ld, Wz + r0, ld, ldw, wdt, false, INT_MIN / 2};
       QOperand B{Wz + r0, Mz + r0 + (size_t)p * ld, ldw, ld, wdt, true, INT_MIN / 2};
-      tt.push_back(QGemmTask{mt, mt, 2 * wdt, 0, 2 * wdt, ld, 1, -1.0, 1.0, A, B, Mz + r0 + (size_t)r0 * ld});
+      tt.push_back(QGemmTask{mt, mt, 0, 2 * wdt, ld, 1, -1.0, 1.0, A, B, Mz + r0 + (size_t)r0 * ld});
       tmaxm[P] = std::max(tmaxm[P], mt);
       tflops[P] += 32.0 * 0.5 * (double)mt * (mt + 1) * 2.0 * wdt;
     }

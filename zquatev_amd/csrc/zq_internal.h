@@ -513,7 +513,9 @@ int matvec_tile_slots(int nmax);
 // gemm.hip: C = beta C + alpha opA(A) opB(B) for quaternion operands (FP64 MFMA).
 // An operand is the column concatenation [p0 | p1] split at ksplit along K;
 // conj_trans selects conj-transpose use of the storage; storage element
-// (r, c) is read only when r > c + mask_off (INT_MIN/2 disables the mask).
+// (r, c) counts as zero unless r > c + mask_off (INT_MIN/2 disables the mask).
+// Masked elements are loaded all the same: the whole rectangle that the shape
+// spans must be allocated, whatever it holds.
 struct QOperand {
   const quat* p0;
   const quat* p1;
@@ -525,20 +527,20 @@ struct QOperand {
 int qgemm(int m, int nn, int k, double alpha, const QOperand& A, const QOperand& B, double beta, quat* C, int ldc,
           bool lower_only, hipStream_t s);
 // One quaternion GEMM piece: C = beta C + alpha opA(A) opB(B) summed over
-// logical k in [kbeg, kend); K bounds the operand reads; lower_only writes
-// only i >= j.
+// logical k in [kbeg, kend); lower_only writes only i >= j.
 struct QGemmTask {
-  int m, nn, K, kbeg, kend;
+  int m, nn, kbeg, kend;
   int ldc, lower_only;
   double alpha, beta;
   QOperand A, B;
   quat* C;
 };
 // ntasks independent tasks (device array, and the same on the host) in one
-// launch; maxm / maxnn bound their shapes, kmin (0: unknown) the lengths of
-// their sums from below; every task has the given operand conjugation flags.
-// Each task computes exactly what qgemm would for it.
-int qgemm_tasks(const QGemmTask* tasks_dev, const QGemmTask* tasks_host, int ntasks, int maxm, int maxnn, int kmin,
+// launch; maxm / maxnn bound their shapes, kchunk (0: unknown) is the least
+// length of their split-K chunks (a sum's last chunk may be shorter); every task
+// has the given operand conjugation flags.  Each task computes exactly what qgemm
+// would for it.
+int qgemm_tasks(const QGemmTask* tasks_dev, const QGemmTask* tasks_host, int ntasks, int maxm, int maxnn, int kchunk,
                 bool a_conj_trans, bool b_conj_trans, bool lower_only, hipStream_t s);
 // GEMM tile rows: 64-row tiles for launches of at least `g_tile64_per_cu`
 // 64 x 64 tiles per compute unit, else 32-row tiles.  A tuning parameter of
