@@ -115,10 +115,6 @@ __device__ __forceinline__ void qfma_cr(quat& acc, const quat& x, const quat& y)
   qfma(acc, x, qconj(y));
 }
 
-__device__ __forceinline__ double shfl_xor_d(double v, int m) {
-  return __shfl_xor(v, m, 64);
-}
-
 // ---- cross-lane exchanges without the LDS crossbar (gfx950) ----------------
 // lane bits 0 .. 3 inside a 16-lane row through DPP; the row-crossing steps of a
 // butterfly through v_permlane16_swap / v_permlane32_swap.
@@ -225,9 +221,6 @@ __device__ __forceinline__ double wave_sum_d(double v) {
   v += xlane<8>(v);
   v = bf16(v, v);
   return bf32(v, v);
-}
-__device__ __forceinline__ quat wave_sum(quat v) {
-  return quat{wave_sum_d(v.ar), wave_sum_d(v.ai), wave_sum_d(v.br), wave_sum_d(v.bi)};
 }
 
 }  // namespace zq
