@@ -188,6 +188,36 @@ def test_tridiag_eig_structured(gpu_ctx, kind):
         assert np.abs(Z.T @ Z - np.eye(n)).max() <= tol
 
 
+@pytest.mark.parametrize("kind", ["ones", "decay"])
+def test_vanishing_columns(gpu_ctx, kind):
+    """Matrices whose columns shrink during the reduction until their squares
+    leave the normal range: equal entries (a roundoff per column) and entries
+    10^(-6 (i + j)).  The vectors stay orthonormal."""
+    for n in list(range(2, 65)) + [65, 80, 100, 128, 224, 300]:
+        _say(f"case: vanishing columns {kind} n={n}")
+        A = np.ones((n, n)) if kind == "ones" else np.outer(10.0 ** (-6.0 * np.arange(n)), 10.0 ** (-6.0 * np.arange(n)))
+        D = np.zeros((2 * n, 2 * n), dtype=np.complex128, order="F")
+        D[:n, :n] = A
+        H = inv.full_h(D, n)
+        info, eig = gpu_ctx.zquatev(D)
+        assert info == 0
+        inv.assert_solution(H, D, eig)
+
+
+@pytest.mark.parametrize("exponent", [-300, -160, 150])
+def test_tail_scale(gpu_ctx, exponent):
+    """Up to n = 64 the reduction takes matrices of any scale, up to the overflow
+    of the columns' squared norms."""
+    for n in (2, 5, 17, 64):
+        _say(f"case: tail scale 1e{exponent} n={n}")
+        D = gen.uniform_case(n, 3900 + n)
+        H = inv.full_h(D, n)
+        X = np.array(D * 10.0 ** exponent, order="F")
+        info, eig = gpu_ctx.zquatev(X)
+        assert info == 0
+        inv.assert_solution(H, X, eig / 10.0 ** exponent)
+
+
 @pytest.mark.parametrize("n2", [2, 4, 6, 8, 16, 22, 42, 44, 64, 128, 130, 400, 510, 512])
 def test_zquatev_host(gpu_ctx, n2):
     _say(f"case: zquatev host 2n={n2}")

@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(256) k_store_vec(int n, const quat* __restrict
 
 __global__ void k_offdiag_abs(int n, const quat* __restrict__ e, double* __restrict__ ea) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n - 1) ea[i] = sqrt(qnorm2(qload(e + i)));
+  if (i < n - 1) ea[i] = qabs(qload(e + i));
 }
 
 // ---- batches: problem blockIdx.z, its table entry P[z], its buffers by zb ----

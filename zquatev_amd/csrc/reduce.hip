@@ -703,18 +703,26 @@ __global__ void __launch_bounds__(TT) k_tail(quat* __restrict__ M, int ld, int n
       if (tx == j) a[k] = quat{a[k].ar, 0.0, 0.0, 0.0};
     }
   }
-  // the reflector of column cl from its owner's registers (column x)
-  auto reflect = [&](int cl, const quat& x) {
+  // The reflector of column cl from its owner's registers (column x).  A block
+  // may shrink by a roundoff per column (equal entries: what is left of each
+  // column is the rounding of equal sums), down to where squares lose digits and
+  // u^* u is no longer 2; there the column is scaled up first.
+  auto reflect = [&](int cl, quat x) {
     const int r0 = cl + 1;
     const bool row = tx >= r0 && tx < ms;
-    const double tail = wave_sum_d(tx > r0 && tx < ms ? qnorm2(x) : 0.0);
-    const quat x1 = quat{lane_d(x.ar, r0), lane_d(x.ai, r0), lane_d(x.br, r0), lane_d(x.bi, r0)};
+    if (tx == cl) d[p + cl] = x.ar;
+    double tail, down = 1.0;
+    quat x1;
+    for (;;) {
+      tail = wave_sum_d(tx > r0 && tx < ms ? qnorm2(x) : 0.0);
+      x1 = quat{lane_d(x.ar, r0), lane_d(x.ai, r0), lane_d(x.br, r0), lane_d(x.bi, r0)};
+      if (!(qnorm2(x1) + tail < TINY_SQ) || down != 1.0) break;   // uniform
+      x = qscale(x, UPSCALE);
+      down = 1.0 / UPSCALE;
+    }
     quat alpha;
     const Refl R = reflector(x1, tail, &alpha);
-    if (tx == cl) {
-      d[p + cl] = x.ar;
-      qstore(e + p + cl, alpha);
-    }
+    if (tx == cl) qstore(e + p + cl, qscale(alpha, down));
     const quat ui = row ? (tx == r0 ? R.u1 : qscale(x, R.g)) : qzero();
     us[cl & 1][tx] = ui;
     if (row) qstore(M + (p + tx) + (size_t)(p + cl) * ld, ui);

@@ -42,7 +42,7 @@ static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 struct SubDiag {
   const double* e;
   const quat* q;
-  __device__ __forceinline__ double operator[](int i) const { return q ? sqrt(qnorm2(qload(q + i))) : fabs(e[i]); }
+  __device__ __forceinline__ double operator[](int i) const { return q ? qabs(qload(q + i)) : fabs(e[i]); }
 };
 
 // --------------------------------------------------------------------------
@@ -740,7 +740,8 @@ struct PhaseJob {
 // waves.  A launch of its own, with 256 chunks scanned one after the other, took
 // 14 us at n = 64 and 56 us at n = 4096; here it ends before the base blocks do.
 constexpr int PH_T = BT;
-__device__ __forceinline__ quat unit_of(const quat& e) {
+__device__ __forceinline__ quat unit_of(quat e) {
+  if (qnorm2(e) < TINY_SQ) e = qscale(e, UPSCALE);
   const double ae = sqrt(qnorm2(e));
   return (ae > 0.0) ? qscale(e, 1.0 / ae) : quat{1.0, 0.0, 0.0, 0.0};
 }
@@ -807,10 +808,13 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
   int bad;
   const double scale = tridiag_scale(ob, n, d, e, bad), inv = 1.0 / scale;
   const bool torn0 = lo0 > ob, torn1 = lo0 + m < ob + n;
+  // entries below 1e-130 of the largest count as zero: the secular equations
+  // multiply two differences of them and a squared weight
+  auto rel = [=](double v) { return bad || fabs(v * inv) < 1e-130 ? 0.0 : v * inv; };
   if (tid < m) {
-    const double ei = (tid < m - 1 || torn1) && !bad ? e[lo0 + tid] * inv : 0.0;
-    double v = bad ? 0.0 : d[lo0 + tid] * inv;
-    if (tid == 0 && torn0 && !bad) v -= e[lo0 - 1] * inv;
+    const double ei = tid < m - 1 || torn1 ? rel(e[lo0 + tid]) : 0.0;
+    double v = rel(d[lo0 + tid]);
+    if (tid == 0 && torn0) v -= rel(e[lo0 - 1]);
     if (tid == m - 1 && torn1) v -= ei;
     sl[tid] = v;
     if (tid < m - 1) se[tid] = ei;

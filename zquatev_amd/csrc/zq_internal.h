@@ -81,6 +81,14 @@ __device__ __forceinline__ double qdot(const quat& x, const quat& y) {
   return fma(x.bi, y.bi, fma(x.br, y.br, fma(x.ai, y.ai, x.ar * y.ar)));
 }
 __device__ __forceinline__ double qnorm2(const quat& x) { return qdot(x, x); }
+// Sums of squares below TINY_SQ may hold squares that lost digits below the normal
+// range; UPSCALE takes every such (nonzero) component's square back into it.
+constexpr double TINY_SQ = 1e-280, UPSCALE = 0x1p600;
+// |x|, also for such x
+__device__ __forceinline__ double qabs(const quat& x) {
+  const double s = qnorm2(x);
+  return s < TINY_SQ ? sqrt(qnorm2(qscale(x, UPSCALE))) * (1.0 / UPSCALE) : sqrt(s);
+}
 // x + s y
 __device__ __forceinline__ quat qaxpy(const quat& x, double s, const quat& y) {
   return quat{fma(s, y.ar, x.ar), fma(s, y.ai, x.ai), fma(s, y.br, x.br), fma(s, y.bi, x.bi)};
