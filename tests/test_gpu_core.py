@@ -188,20 +188,34 @@ def test_tridiag_eig_structured(gpu_ctx, kind):
         assert np.abs(Z.T @ Z - np.eye(n)).max() <= tol
 
 
-@pytest.mark.parametrize("kind", ["ones", "decay"])
+@pytest.mark.parametrize("kind", ["ones", "bipartite", "decay1.5", "decay2.5", "decay5", "decay6"])
 def test_vanishing_columns(gpu_ctx, kind):
     """Matrices whose columns shrink during the reduction until their squares
-    leave the normal range: equal entries (a roundoff per column) and entries
-    10^(-6 (i + j)).  The vectors stay orthonormal."""
-    for n in list(range(2, 65)) + [65, 80, 100, 128, 224, 300]:
+    leave the normal range: equal entries (a roundoff per column or panel) and
+    entries 10^(-a (i + j)).  The vectors stay orthonormal, and eigenvalues only
+    finds the same spectrum."""
+    import torch
+    for n in (list(range(2, 65)) if kind in ("ones", "decay6") else [12, 33, 63, 64]) + [65, 96, 129, 224, 300]:
         _say(f"case: vanishing columns {kind} n={n}")
-        A = np.ones((n, n)) if kind == "ones" else np.outer(10.0 ** (-6.0 * np.arange(n)), 10.0 ** (-6.0 * np.arange(n)))
+        i = np.arange(n)
+        if kind == "ones":
+            A = np.ones((n, n))
+        elif kind == "bipartite":
+            A = 1.0 * ((i[:, None] + i[None, :]) % 2)
+        else:
+            A = np.outer(10.0 ** (-float(kind[5:]) * i), 10.0 ** (-float(kind[5:]) * i))
         D = np.zeros((2 * n, 2 * n), dtype=np.complex128, order="F")
         D[:n, :n] = A
         H = inv.full_h(D, n)
+        Dt = torch.from_numpy(np.ascontiguousarray(D.T)).cuda()
+        ev = torch.zeros(n, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        assert gpu_ctx.zquatev_device(2 * n, Dt.data_ptr(), 2 * n, ev.data_ptr(), "N") == 0
+        assert gpu_ctx.last_info() == 0
         info, eig = gpu_ctx.zquatev(D)
         assert info == 0
         inv.assert_solution(H, D, eig)
+        assert np.abs(ev.cpu().numpy() - eig).max() <= inv.EIG_TOL * np.linalg.norm(H, 2)
 
 
 @pytest.mark.parametrize("exponent", [-300, -160, 150])

@@ -60,6 +60,13 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
   return r;
 }
 
+// Whether an entry of the tridiagonal's first c columns exceeds v (one thread)
+__device__ __forceinline__ bool any_above(const double* d, const quat* e, int c, double v) {
+  for (int k = 0; k < c; ++k)
+    if (fabs(d[k]) > v || qabs(qload(e + k)) > v) return true;
+  return false;
+}
+
 // Reflector for column c: x = M[c+1:, c].  H x = alpha e_1 with
 // alpha = -q |x|, q = x_1/|x_1|; u = gamma (x - alpha e_1), gamma = 1/sqrt(|x| (|x| + |x_1|)),
 // so u^* u = 2.  A zero tail gives u = 0 and alpha = x_1.  Computed identically
@@ -180,9 +187,17 @@ __global__ void __launch_bounds__(SYT) k_symv(
       for (int i = c + 2 + tid; i < n; i += SYT) tail += qnorm2(qload(M + i + (size_t)c * ld));
       tail = block_sum(tail, sh);
     }
+    // A column whose squares lose digits counts as reduced (u = 0): it is at most
+    // 1e-140, and neither its norm nor x^* M x is known.  One that is not zero and
+    // below the reach of gamma^2 is told apart from a matrix of that scale, which
+    // this reduction cannot take (not finite, as its gamma^2), by a larger entry of
+    // d or e so far.
+    const double s = qnorm2(x1) + tail;
+    const bool drop = s < TINY_SQ;
     quat alpha;
-    const Refl R = reflector(x1, tail, &alpha);
+    const Refl R = reflector(x1, drop ? 0.0 : tail, &alpha);
     if (bt == 0 && tid == 0) {
+      if (drop && s > 0.0 && s < 3e-309 && !any_above(d, e, c, 1e-130)) alpha.ar = __builtin_nan("");
       scal[0] = R.g;
       scal[1] = R.u1.ar; scal[2] = R.u1.ai; scal[3] = R.u1.br; scal[4] = R.u1.bi;
       scal[5] = x1.ar; scal[6] = x1.ai; scal[7] = x1.br; scal[8] = x1.bi;
