@@ -156,12 +156,14 @@ def test_tridiag_eig_one_block(gpu_ctx, n, kind):
     assert np.abs(Z.T @ Z - np.eye(n)).max() <= tol
 
 
-@pytest.mark.parametrize("kind", ["clement", "constant", "integer"])
+@pytest.mark.parametrize("kind", ["clement", "constant", "integer", "decay", "growth"])
 def test_tridiag_eig_structured(gpu_ctx, kind):
     """Tridiagonals whose secular equations have roots within a rounding of an
     end of their first bracket (the midpoint of two poles, or the bound of the
     last root), where a Newton step that ends the iteration can round out of the
-    bracket.  Bound as for one block, with a merge level more per doubling."""
+    bracket; and entries over the whole range of a double, down to zero, whose
+    products underflow.  Bound as for one block, with a merge level more per
+    doubling."""
     import torch
     rng = np.random.default_rng(5)
     for n in list(range(2, 65)) + [65, 80, 96, 100, 127, 128, 129, 130]:
@@ -171,8 +173,12 @@ def test_tridiag_eig_structured(gpu_ctx, kind):
             d, e = np.zeros(n), np.sqrt((k + 1.0) * (n - 1 - k))
         elif kind == "constant":
             d, e = rng.integers(0, 5, n).astype(float), np.full(n - 1, 0.1 * rng.integers(1, 60))
-        else:
+        elif kind == "integer":
             d, e = rng.integers(0, 3, n).astype(float), rng.integers(0, 3, n - 1).astype(float)
+        else:
+            d, e = rng.uniform(-1, 1, n) * 10.0 ** (-5.0 * np.arange(n)), rng.uniform(0, 1, n - 1) * 10.0 ** (-5.0 * k)
+            if kind == "growth":
+                d, e = d[::-1].copy(), e[::-1]
         dd, de = torch.from_numpy(d).cuda(), torch.from_numpy(np.r_[e, 0.0]).cuda()
         dw = torch.zeros(n, dtype=torch.float64, device="cuda")
         dz = torch.zeros(n * n, dtype=torch.float64, device="cuda")

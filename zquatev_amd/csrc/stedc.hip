@@ -808,9 +808,11 @@ __global__ void __launch_bounds__(BT) k_dc_base(const int* __restrict__ leaves, 
   int bad;
   const double scale = tridiag_scale(ob, n, d, e, bad), inv = 1.0 / scale;
   const bool torn0 = lo0 > ob, torn1 = lo0 + m < ob + n;
-  // entries below 1e-130 of the largest count as zero: the secular equations
-  // multiply two differences of them and a squared weight
-  auto rel = [=](double v) { return bad || fabs(v * inv) < 1e-130 ? 0.0 : v * inv; };
+  // Entries below 1e-100 of the largest count as zero: the secular equations
+  // multiply two differences of them and squared weights down to 1e-31.  Where
+  // such a product underflows, a root can be lost (two equal columns), and from
+  // unordered roots the ranks of the next merge would collide.
+  auto rel = [=](double v) { return bad || fabs(v * inv) < 1e-100 ? 0.0 : v * inv; };
   if (tid < m) {
     const double ei = tid < m - 1 || torn1 ? rel(e[lo0 + tid]) : 0.0;
     double v = rel(d[lo0 + tid]);
