@@ -268,7 +268,9 @@ void slab_layout(Bump& b, int n, int nb, bool vectors, Plan* p) {
   p->rw.Pcol = p->rw.Prow ? p->rw.Prow + (size_t)p->rw.pcs * n : nullptr;
   p->rw.TS = b.take<quat>((size_t)2 * nb);
   p->rw.ldtsp = 8 * nb;
-  p->rw.TSP = b.take<double>((size_t)(cdiv(nmax, 16) + 1) * 8 * nb);
+  // the matvec's finishing blocks read a row of TSP in whole waves: up to 63
+  // doubles beyond the last row where it is narrower
+  p->rw.TSP = b.take<double>((size_t)(cdiv(nmax, 16) + 1) * 8 * nb + 64);
   p->rw.QF = b.take<double>((size_t)zq::matvec_tile_slots(nmax));
   p->rw.part = b.take<double>(cdiv(nmax, 16) + 16);
   p->rw.scal = b.take<double>(16);

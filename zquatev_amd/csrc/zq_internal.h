@@ -352,7 +352,7 @@ struct ReduceWork {
   quat* Pcol;     // matvec column partials: ceil(n/64) x n, right after Prow's
   int pcs;        // Pcol = Prow + pcs n
   quat* TS;       // tall-skinny products [W^* u | V^* u]: 2 x nb
-  double* TSP;    // their per-block partials: ceil(n/16) x ldtsp
+  double* TSP;    // their per-block partials: ceil(n/16) x ldtsp, and 64 beyond
   int ldtsp;      // 8 nb
   double* QF;     // per-tile partials of x^* M x: ceil(n/64) (ceil(n/64) + 1)
   double* part;   // ceil(n/16)
