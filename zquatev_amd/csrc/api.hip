@@ -1010,12 +1010,13 @@ const char* zq_error_string(int code) {
 }
 
 int zq_tuned_panel_width(int n) {
-  // measured on MI355X (eigenvalues only, 16 / 24 / 32): 2n = 2048 9.36 / 9.74 /
-  // 9.71 ms, 4096 27.2 / 27.6 / 27.5, 6000 55.8 / 56.4 / 56.2, 8192 109.3 / 109.6 /
-  // 109.1 (16's column kernel holds half the panel coefficients per thread; 32
-  // halves the passes of the trailing update over the matrix, the larger part
-  // only beyond).  One width for n <= 4096 also keeps a batch of such sizes in
-  // one lockstep group.  zq_autotune refines it per size bucket (floor(log2 n)).
+  // 16's column kernel holds half the panel coefficients per thread; 32 halves the
+  // passes of the trailing update over the matrix.  Measured on MI355X
+  // (eigenvalues only, 16 / 32): 2n = 1024 4.06 / 4.20 ms, 3000 16.0 / 16.3, 4096
+  // 26.9 / 27.2, 8192 107.6 / 108.1, 9000 140.8 / 141.4, 12000 328.8 / 329.6, 16384
+  // 836.5 / 826.4; with eigenvectors 32768 8.86 / 8.72 s.  The two are within 0.5%
+  // from n = 4096 to 6000 and 32 is ahead from n = 8192 on: the line lies at the
+  // low end of that band.  zq_autotune refines it per size bucket (floor(log2 n)).
   return n <= 4096 ? 16 : 32;
 }
 

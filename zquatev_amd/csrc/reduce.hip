@@ -255,9 +255,11 @@ __global__ void __launch_bounds__(SYT) k_symv(
   // divergent ifs, and an inactive tile computes zeros from its clamped loads
   // and stores nothing -- so the body is one scheduling region: the
   // wave-uniform loads of x at the tile's columns issue alongside the tile
-  // loads instead of after their wait, and the kernel needs 64 VGPRs instead
+  // loads instead of after their wait, and the kernel needs 66 VGPRs instead
   // of 84 (three 512-thread blocks per CU instead of two).  2n = 8192 solve
-  // -1.5 ms.  The narrow tiles keep the branches: branch-free they made the
+  // -1.5 ms.  (Four blocks need 64: held to that it spills 20 bytes and the solve
+  // takes 9 ms more, and with multiplies and adds for the quaternion product's
+  // FMAs, which fits, it is slower too.)  The narrow tiles keep the branches: branch-free they made the
   // 512-problem batch 1.3% slower (also when held to five blocks per CU, their
   // residency with branches), for 0.7% on single solves of 2n <= 1024.
   constexpr bool BF = SW == 32;

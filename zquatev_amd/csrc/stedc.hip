@@ -3,10 +3,12 @@
 // the eigenvalues-only path.
 //
 // Replaces the tridiagonal step of the reference, zhbev_("V","L",n,1,...)
-// (zquatev.cc:74-84; MKL: zhbtrd phase scaling + zsteqr QL/QR).  The phase
-// scaling is done on the quaternion subdiagonal (backtr.hip); this file sees
-// the real tridiagonal (d, |e|) and returns the eigenvalues ascending, as
-// zhbev does, with an orthonormal real eigenvector matrix.
+// (zquatev.cc:74-84; MKL: zhbtrd phase scaling + zsteqr QL/QR).  The divide and
+// conquer solves the real tridiagonal (d, |e|) and returns the eigenvalues
+// ascending, as zhbev does, with an orthonormal real eigenvector matrix.  Where
+// the subdiagonal comes as quaternions (a single solve), its magnitudes are taken
+// as they are read; its phases are formed beside the base blocks (phases_block)
+// and applied by backtr.hip.
 //
 // Tree: halve until a block has at most BASE rows; each split point s couples
 // rows s-1 and s with beta = e[s-1] >= 0, and T = diag(T1', T2') + beta v v^T,
