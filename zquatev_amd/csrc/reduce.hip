@@ -689,14 +689,16 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
 // block in LDS and four waves was bound by its re-reads of the block, one wave
 // per SIMD having nothing to hide them behind: 64 columns took 242 us, now
 // 138 us (149 with 16 waves, 140 with 4; 149 with the stages in one rolled
-// loop, although that quarters the code).
+// loop, although that quarters the code).  Two blocks fit a CU at up to 128
+// registers: with one (136) a batch of 2048 of 2n = 32 .. 64 takes 1.54 ms, with
+// two 1.37.
 // ---------------------------------------------------------------------------
 constexpr int TT = 512;            // threads: 8 waves
 constexpr int TWV = TT / 64;
 constexpr int TKC = TAILN / TWV;    // columns per wave
 static_assert(TAILN == 64 && TKC * TWV == TAILN, "k_tail: lane = row, TKC columns per wave");
 
-__global__ void __launch_bounds__(TT) k_tail(quat* __restrict__ M, int ld, int n, int p,
+__global__ void __launch_bounds__(TT, 4) k_tail(quat* __restrict__ M, int ld, int n, int p,
                                   const int* __restrict__ pstart,
                                              double* __restrict__ d, quat* __restrict__ e, ZB zb) {
   if (zb.nvec) {
@@ -724,23 +726,24 @@ __global__ void __launch_bounds__(TT) k_tail(quat* __restrict__ M, int ld, int n
   // may shrink by a roundoff per column (equal entries: what is left of each
   // column is the rounding of equal sums), down to where squares lose digits and
   // u^* u is no longer 2; there the column is scaled up first.
-  auto reflect = [&](int cl, quat x) {
+  auto reflect = [&](int cl, const quat& x) {
     const int r0 = cl + 1;
     const bool row = tx >= r0 && tx < ms;
-    if (tx == cl) d[p + cl] = x.ar;
-    double tail, down = 1.0;
-    quat x1;
-    for (;;) {
-      tail = wave_sum_d(tx > r0 && tx < ms ? qnorm2(x) : 0.0);
-      x1 = quat{lane_d(x.ar, r0), lane_d(x.ai, r0), lane_d(x.br, r0), lane_d(x.bi, r0)};
-      if (!(qnorm2(x1) + tail < TINY_SQ) || down != 1.0) break;   // uniform
-      x = qscale(x, UPSCALE);
-      down = 1.0 / UPSCALE;
+    double tail = wave_sum_d(tx > r0 && tx < ms ? qnorm2(x) : 0.0);
+    quat x1 = quat{lane_d(x.ar, r0), lane_d(x.ai, r0), lane_d(x.br, r0), lane_d(x.bi, r0)};
+    double up = 1.0;
+    if (qnorm2(x1) + tail < TINY_SQ) {   // uniform
+      up = UPSCALE;
+      tail = wave_sum_d(tx > r0 && tx < ms ? qnorm2(qscale(x, up)) : 0.0);
+      x1 = qscale(x1, up);
     }
     quat alpha;
     const Refl R = reflector(x1, tail, &alpha);
-    if (tx == cl) qstore(e + p + cl, qscale(alpha, down));
-    const quat ui = row ? (tx == r0 ? R.u1 : qscale(x, R.g)) : qzero();
+    if (tx == cl) {
+      d[p + cl] = x.ar;
+      qstore(e + p + cl, qscale(alpha, up == 1.0 ? 1.0 : 1.0 / UPSCALE));
+    }
+    const quat ui = row ? (tx == r0 ? R.u1 : qscale(qscale(x, up), R.g)) : qzero();
     us[cl & 1][tx] = ui;
     if (row) qstore(M + (p + tx) + (size_t)(p + cl) * ld, ui);
   };
