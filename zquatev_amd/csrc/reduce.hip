@@ -692,6 +692,9 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(WPE))) 
 // loop, although that quarters the code).  Two blocks fit a CU at up to 128
 // registers: with one (136) a batch of 2048 of 2n = 32 .. 64 takes 1.54 ms, with
 // two 1.37.
+// Waves pass over absent columns: with their zeros multiplied too,
+// eigenvalues only of 2n = 32 took 99 us where the LDS form took 90; now 80 (2n = 64
+// 145 -> 119.5 us, 112 201 -> 190, 128 216.0 -> 216.8).
 // ---------------------------------------------------------------------------
 constexpr int TT = 512;            // threads: 8 waves
 constexpr int TWV = TT / 64;
@@ -754,12 +757,13 @@ __global__ void __launch_bounds__(TT, 4) k_tail(quat* __restrict__ M, int ld, in
       const int cl = TWV * kk + c;
       if (cl + 1 >= ms) break;   // uniform
       const int r0 = cl + 1, par = cl & 1;
+      const unsigned nt = ms - r0;   // trailing rows
       __syncthreads();   // us of column cl is complete
       const quat ui = us[par][tx];
       quat acc = qzero();   // this lane's row of A u over this wave's columns
 #pragma unroll
       for (int k = kk; k < TKC; ++k)
-        if (wv + TWV * k >= r0) qfma(acc, a[k], us[par][wv + TWV * k]);   // uniform
+        if (unsigned(wv + TWV * k - r0) < nt) qfma(acc, a[k], us[par][wv + TWV * k]);   // uniform: r0 .. ms - 1
       part[wv][tx] = acc;
       __syncthreads();
       if (wv == 0) {
@@ -777,7 +781,7 @@ __global__ void __launch_bounds__(TT, 4) k_tail(quat* __restrict__ M, int ld, in
 #pragma unroll
       for (int k = kk; k < TKC; ++k) {
         const int j = wv + TWV * k;
-        if (j < r0) continue;   // uniform
+        if (unsigned(j - r0) >= nt) continue;   // uniform
         const quat uj = us[par][j], wj = ys[par][j];
         const quat nu = quat{-ui.ar, -ui.ai, -ui.br, -ui.bi}, nw = quat{-wi.ar, -wi.ai, -wi.br, -wi.bi};
         qfma_cr(a[k], nu, wj);
