@@ -177,8 +177,8 @@ def cpu_baseline(n2, reps, small_reps):
     f512 = gen.flops_vectors(256)
     return {"value": round(gen.flops_vectors(n) / med / 1e9, 3), "unit": "GFLOP/s", "cores": threads,
             "kind": big["kind"],
-            "sample": (f"median of {reps} {what} calls (eigenvalues+eigenvectors) at 2n={n2} on {threads} MKL "
-                       f"threads, same U(-1,1) generator, wall clock around the call only "
+            "sample": (f"median of {reps} {what} calls (eigenvalues+eigenvectors) at 2n={n2} on {threads} "
+                       f"{'MKL ' if ref.available() else ''}threads, same U(-1,1) generator, wall clock around the call only "
                        f"({', '.join(f'{t:.2f}' for t in big['seconds'])} s); GFLOP/s on (160/3) n^3"),
             "host": host,
             "runs_s": big["seconds"],
