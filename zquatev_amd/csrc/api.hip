@@ -209,14 +209,13 @@ struct CaptureScope {
   ~CaptureScope();
 };
 
-// reflectors per back-transform block (a multiple of the panel width)
 // Reflectors per compact-WY block of the back-transform.  Batches group
 // their problems by this width (as by panel width), so that a member applies
-// the same blocks as its solo solve.
-// Back-transform block width.  Measured: 128 from n = 449 took the batch of
-// 512 problems of 2n <= 1024 from 82.7 to 74.6 ms and single solves of 2n =
-// 1024 .. 8192 0.6-2.7 % faster; switching lower (n = 193, 321, 385) made the
-// batch slower, and 256 made 2n = 4096 and 8192 slower.
+// the same blocks as its solo solve.  128 against 64 throughout: 2n = 8192
+// 144.6 / 146.4 ms, 2048 10.11 / 10.12, 520 to 1024 equal within 0.3 %, a batch of
+// 512 problems of 2n <= 1024 72.0 / 71.8 ms.  Switching lower costs the batch:
+// from n = 385 72.5, 321 75.4, 257 76.3 ms (its smaller members in a second group
+// of few blocks).  256 made 2n = 4096 and 8192 slower.
 inline int backtr_width(int n) { return n > 448 ? 128 : 64; }
 
 struct Plan {
@@ -385,7 +384,10 @@ int panel_width(const zq_context* ctx, int n) {
   return nb;
 }
 
-constexpr int kTsmDefault = 768;   // matvec strip switch (trailing size)
+// Matvec strip switch (trailing size).  512 / 768 / 1024 / 1536: 2n = 2730 16.10 /
+// 16.08 / 16.14 / 16.31 ms, 4096 32.14 / 32.12 / 32.18 / 32.5, 8192 146.0 / 145.9 /
+// 146.0 / 146.8, a batch of 2n <= 1024 equal.
+constexpr int kTsmDefault = 768;
 constexpr int kTile64Default = 16; // 64-row GEMM tiles from this many 64 x 64 tiles per CU
 
 int matvec_switch(const zq_context* ctx, int n) {
